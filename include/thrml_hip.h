@@ -64,7 +64,8 @@ int thrml_ctx_synchronize(thrml_ctx *ctx);
  * enable: 0 off; 1 an event pair around every launch (each pair adds the
  * markers' own few microseconds); 2 one span, from an event before the first
  * launch to one recorded when the time is read, over the launch count (the
- * average launch-to-launch time, gaps and interleaved kernels included).
+ * average launch-to-launch time, gaps and interleaved kernels included).  A
+ * launch that runs several sweeps counts as one per block and sweep.
  * Changing the mode resets the accumulated times. */
 int thrml_ctx_enable_timing(thrml_ctx *ctx, int enable);
 int thrml_ctx_kernel_time(thrml_ctx *ctx, int kernel, double *avg_ms, uint64_t *count);

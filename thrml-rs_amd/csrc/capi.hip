@@ -145,9 +145,9 @@ int thrml_ctx::time_begin(int k, hipEvent_t *start) {
   return 0;
 }
 
-int thrml_ctx::time_end(int k, hipEvent_t start) {
+int thrml_ctx::time_end(int k, hipEvent_t start, uint64_t half_sweeps) {
   if (timing == 2) {
-    slots[k].span_n += 1;
+    slots[k].span_n += half_sweeps;
     return THRML_OK;
   }
   if (!timing || !start) return THRML_OK;
@@ -156,6 +156,7 @@ int thrml_ctx::time_end(int k, hipEvent_t start) {
   THRML_HIP(hipEventRecord(b, stream));
   slots[k].ev.push_back(start);
   slots[k].ev.push_back(b);
+  slots[k].n.push_back(half_sweeps);
   if (slots[k].ev.size() >= 4096) return flush_timing(k);
   return THRML_OK;
 }
@@ -184,10 +185,11 @@ int thrml_ctx::flush_timing(int k) {
     float ms = 0.f;
     THRML_HIP(hipEventElapsedTime(&ms, v[i], v[i + 1]));
     acc_ms[k] += ms;
-    acc_n[k] += 1;
+    acc_n[k] += slots[k].n[i / 2];
   }
   for (auto e : v) (void)hipEventDestroy(e);
   v.clear();
+  slots[k].n.clear();
   return THRML_OK;
 }
 
@@ -592,6 +594,17 @@ bool detect_lattice(thrml_prog *p, uint32_t n_nodes, const std::vector<uint32_t>
   return true;
 }
 
+// Slot records {tail position, weight} as uploaded, with 16 spare ones: the
+// sweep kernel reads them in batches of 16.
+std::vector<uint32_t> pack_slots(const std::vector<uint32_t> &pos, const std::vector<float> &w) {
+  std::vector<uint32_t> r(2 * (pos.size() + 16), 0u);
+  for (size_t s = 0; s < pos.size(); ++s) {
+    r[2 * s] = pos[s];
+    std::memcpy(&r[2 * s + 1], &w[s], 4);
+  }
+  return r;
+}
+
 // An RBM-shaped model for the matrix-core path, taken only when the caller
 // sets THRML_ISING_DENSE: two blocks (free ++ clamped) of at least
 // THRML_DENSE_MIN_SIDE nodes whose edges are exactly the complete bipartite
@@ -786,20 +799,27 @@ extern "C" int thrml_ising_program_create(thrml_ctx *ctx, const thrml_ising_desc
   std::vector<uint32_t> dir;
   if (!intra && one_per_block && detect_lattice(p, d->n_nodes, row_off, slot_pos, dir)) {
     p->kind = K_LATTICE;
-    DevBuf d_dir, d_w, d_b;
+    DevBuf d_dir, d_slots, d_b;
+    const std::vector<uint32_t> slots2 = pack_slots(slot_pos, slot_w);
     if ((rc = upload(p, p->row_off, row_off)) || (rc = upload(p, d_dir, dir)) ||
-        (rc = upload(p, d_w, slot_w)) || (rc = upload(p, d_b, bias_w)) ||
+        (rc = upload(p, d_slots, slots2)) || (rc = upload(p, d_b, bias_w)) ||
         (rc = p->table.alloc(nf * 16 * sizeof(uint32_t)))) {
       delete p;
       return rc;
     }
     p->device_bytes += p->table.bytes;
-    rc = launch_lattice_table(p, d_dir.as<uint32_t>(), d_w.as<float>(), d_b.as<float>());
-    if (!rc) {
-      hipError_t e = hipStreamSynchronize(ctx->stream);
-      if (e != hipSuccess) rc = hip_fail(e, "lattice table");
-    }
-    p->device_bytes -= p->row_off.bytes + d_dir.bytes + d_w.bytes + d_b.bytes;
+    rc = launch_lattice_table(p, d_dir.as<uint32_t>(), d_slots.as<uint2>(), d_b.as<float>());
+    // the threshold table decides up where a sum is NaN and spin_decision
+    // down: only sums that cannot overflow run resident
+    double mag = 0.0;
+    for (float x : slot_w) mag += std::fabs((double)x);
+    for (float x : bias_w) mag += std::fabs((double)x);
+    std::vector<uint8_t> keep;
+    if (!rc && mag < 1e38)
+      rc = resident_tables(p, row_off, p->row_off.as<uint32_t>(), d_slots.as<uint2>(), d_b.as<float>(), keep);
+    const hipError_t e = hipStreamSynchronize(ctx->stream);
+    if (!rc && e != hipSuccess) rc = hip_fail(e, "lattice table");
+    p->device_bytes -= p->row_off.bytes + d_dir.bytes + d_slots.bytes + d_b.bytes;
     p->row_off.release();
     if (rc) {
       delete p;
@@ -808,21 +828,20 @@ extern "C" int thrml_ising_program_create(thrml_ctx *ctx, const thrml_ising_desc
   } else {
     p->kind = K_CSR;
     csr_windows(p, row_off);
-    // 16 spare slots: the sweep kernel reads slot records in batches of 16
-    std::vector<uint32_t> slots2(2 * (ns + 16), 0u);
-    for (uint64_t s = 0; s < ns; ++s) {
-      slots2[2 * s] = slot_pos[s];
-      std::memcpy(&slots2[2 * s + 1], &slot_w[s], 4);
-    }
+    const std::vector<uint32_t> slots2 = pack_slots(slot_pos, slot_w);
     if ((rc = upload(p, p->row_off, row_off)) || (rc = upload(p, p->slots, slots2)) ||
         (rc = upload(p, p->bias_w, bias_w))) {
       delete p;
       return rc;
     }
+    std::vector<uint8_t> keep;
+    rc = resident_tables(p, row_off, p->row_off.as<uint32_t>(), p->slots.as<uint2>(),
+                         p->bias_w.as<float>(), keep);
     hipError_t e = hipStreamSynchronize(ctx->stream);
-    if (e != hipSuccess) {
+    if (!rc && e != hipSuccess) rc = hip_fail(e, "program upload");
+    if (rc) {
       delete p;
-      return hip_fail(e, "program upload");
+      return rc;
     }
   }
   *out = p;
@@ -1272,6 +1291,8 @@ extern "C" int thrml_state_create(thrml_prog *p, uint32_t n_chains, thrml_state 
   // the sweep kernel's half-size gather copy (refreshed at each run's start)
   if (!rc && p->kind == K_CSR && n_chains <= 32u && p->planes == 1u && p->stage_max == 0)
     rc = st->low.alloc((size_t)p->n_total * sizeof(uint32_t));
+  if (!rc && p->res_T)
+    rc = st->bits.alloc((size_t)n_chains * ((p->n_total + 63u) / 64u) * sizeof(uint64_t));
   if (!rc && p->stage_max) {
     // cleared once: the padding chains of a categorical row are copied back
     // with the staged range but never written
@@ -1467,7 +1488,13 @@ int run_plan(thrml_prog *p, thrml_state *st, const Plan &pl, const LatticeMoment
   }
   // the words may have changed since the last run (state writes, hinton_init);
   // the sweeps keep the copy in step from here on
-  if (pl.n_sweeps && st->low.p)
+  // the observations left cut the run into segments
+  const uint64_t n_seg = std::max<uint64_t>(n_obs - oi, 1);
+  bool resident = resident_pays(p, st, pl.n_sweeps, n_seg, can_fuse);
+#ifdef RES_FORCE
+  resident = p->res_T && RES_FORCE;
+#endif
+  if (pl.n_sweeps && st->low.p && !resident)
     if (int rc = launch_pack_low(st)) return rc;
   for (uint64_t s0 = 0; s0 < pl.n_sweeps; s0 += chunk) {
     const uint32_t ns = (uint32_t)std::min<uint64_t>(chunk, pl.n_sweeps - s0);
@@ -1481,6 +1508,18 @@ int run_plan(thrml_prog *p, thrml_state *st, const Plan &pl, const LatticeMoment
     // this launch behind them
     if (int rc = launch_key_schedule(p->ctx, pl.kp, s0, ns, keys)) return rc;
     for (uint32_t k = 0; k < ns; ++k) {
+      if (resident) {
+        // every sweep up to the next observation (or the chunk's end) at once
+        const uint64_t end = oi < n_obs ? std::min<uint64_t>(s0 + ns, (uint64_t)pl.obs_after[oi] + 1) : s0 + ns;
+        const uint32_t nk = (uint32_t)(end - (s0 + k));
+        if (int rc = launch_resident(p, st, keys + (size_t)k * B * st->G * 64u * KEY_WORDS, nk)) return rc;
+        k += nk - 1u;
+        while (oi < n_obs && pl.obs_after[oi] == (int64_t)end - 1) {
+          if (int rc = obs(false)) return rc;
+          ++oi;
+        }
+        continue;
+      }
       const int64_t s = (int64_t)(s0 + k);
       const bool observed = oi < n_obs && pl.obs_after[oi] == s;
       const LatticeMoments *m = (observed && can_fuse) ? fuse : nullptr;

@@ -36,6 +36,21 @@ int hip_fail(hipError_t e, const char *what);
 
 enum ProgKind : uint32_t { K_LATTICE = 0, K_CSR = 1, K_POTTS = 2, K_DENSE = 3, K_DISCRETE = 4 };
 
+// Resident runs (k_resident.hip): a piece is a run of sites of one block, a
+// part the pieces whose keystream blocks one phase computes.
+constexpr uint32_t RES_NONE = 0xffffffffu;
+constexpr uint32_t RES_MAX_NODES = 65535;   // 16-bit positions; one LDS byte each beside the keystream
+constexpr uint32_t RES_MAX_ENT = 10;        // entries per wave of the register kernel
+constexpr int RES_LDS = 160 * 1024;
+struct ResPiece {
+  uint32_t blk, site0, n;  // block, first block-local site, sites
+  uint32_t kb0;            // its first keystream block within the part
+  uint32_t row0, slice0;   // global position of its first site, its first slice
+};
+struct ResPart {
+  uint32_t piece0, piece1, kb;  // pieces [piece0, piece1), keystream blocks
+};
+
 // A device allocation that frees itself.
 struct DevBuf {
   void *p = nullptr;
@@ -69,6 +84,7 @@ struct DevBuf {
 
 struct TimingSlot {
   std::vector<hipEvent_t> ev;  // pairs
+  std::vector<uint64_t> n;     // half-sweeps of each pair's launch
   size_t used = 0;
   hipEvent_t span0 = nullptr;  // span mode: recorded before the first launch
   uint64_t span_n = 0;         // span mode: launches since span0
@@ -93,7 +109,7 @@ struct thrml_ctx {
   std::mutex run_mu;
   int flush_timing(int k);
   int time_begin(int k, hipEvent_t *start);
-  int time_end(int k, hipEvent_t start);
+  int time_end(int k, hipEvent_t start, uint64_t half_sweeps = 1);
 };
 
 struct thrml_prog {
@@ -152,6 +168,14 @@ struct thrml_prog {
   std::vector<uint32_t> csr_win[4];
   std::vector<uint32_t> csr_maxdeg;  // largest slot count of a site, per free block
 
+  // --- resident runs of small Ising programs (res_T = 0: not eligible)
+  uint32_t res_T = 0;              // threads per workgroup (one chain)
+  uint32_t res_parts = 0, res_kb = 0, res_pf = 0;
+  uint32_t res_ent = 0;            // register kernel: entries per wave (0: streaming kernel)
+  double res_work = 0.0, res_deg = 0.0;  // us per sweep besides the blocks', slots per site
+  thrml::DevBuf r_tab;             // its tables and slot data, at r_off
+  uint64_t r_off[5] = {};
+
   // --- dense bipartite path.  Side 0 ("visible") holds the rows of W, side 1
   // ("hidden") its columns; dense_side[b] is the side of block b (blocks are
   // free ++ clamped in any order) and side_off[s] the global offset of side s.
@@ -206,6 +230,8 @@ struct thrml_state {
   // sweep kernel gathers neighbour states here, half the footprint of the
   // words, and writes both; each run refreshes it from the words first.
   thrml::DevBuf low;
+  // resident runs: [C][ceil(n_total / 64)] u64, the chains' spins at a run's end
+  thrml::DevBuf bits;
   // dense path operands: spin-down bits per block, one bit vector per chain
   // (bit k%32 of word k/32 is 1 when the spin at block position k is down)
   uint32_t C_pad = 0;     // chains rounded up to the 256-wide GEMM tile
@@ -325,6 +351,13 @@ int launch_lattice_moments(thrml_state *st, const LatticeMoments *mom);
 int launch_csr_half(thrml_prog *p, thrml_state *st, uint32_t b, const uint32_t *d_keys);
 // refreshes st->low from the state words (CSR programs that keep it)
 int launch_pack_low(thrml_state *st);
+// Resident runs: tables at program creation, and n_sweeps whole sweeps whose
+// expanded keys start at d_keys.
+int resident_tables(thrml_prog *p, const std::vector<uint32_t> &row_off, const uint32_t *d_row_off,
+                    const uint2 *d_slots, const float *d_bias, std::vector<uint8_t> &keep);
+bool resident_pays(const thrml_prog *p, const thrml_state *st, uint64_t n_sweeps, uint64_t n_seg,
+                   bool fused);
+int launch_resident(thrml_prog *p, thrml_state *st, const uint32_t *d_keys, uint32_t n_sweeps);
 void csr_windows(thrml_prog *p, const std::vector<uint32_t> &row_off);
 int launch_potts_half(thrml_prog *p, thrml_state *st, uint32_t b, const uint32_t *d_keys);
 int launch_discrete_half(thrml_prog *p, thrml_state *st, uint32_t b, const uint32_t *d_keys);
@@ -334,7 +367,7 @@ int reduce_energy(thrml_prog *p, uint32_t C, const double *part, uint32_t n, uin
                   double *out);
 // Dense programs: one half-sweep of side `side` (0 rows of W, 1 columns).
 int launch_dense_half(thrml_prog *p, thrml_state *st, uint32_t side, const uint32_t *d_keys);
-int launch_lattice_table(thrml_prog *p, const uint32_t *d_dir, const float *d_w, const float *d_bias);
+int launch_lattice_table(thrml_prog *p, const uint32_t *d_dir, const uint2 *d_slots, const float *d_bias);
 int launch_hinton(thrml_prog *p, thrml_state *st, uint32_t b, const uint32_t *d_key8,
                   const float *d_prob);
 // State import of block b from device memory; values out of range (spins

@@ -205,7 +205,7 @@ __global__ void lattice_moments_kernel(const uint64_t *__restrict__ words, uint6
 // lattice direction (L, R, U, D) of slot s; slots are in reference order.
 __global__ void lattice_table_kernel(const uint32_t *__restrict__ row_off,
                                      const uint32_t *__restrict__ dir,
-                                     const float *__restrict__ w,
+                                     const uint2 *__restrict__ slots,
                                      const float *__restrict__ bias_w, uint32_t n,
                                      int has_bias, int has_edges, uint32_t *__restrict__ table) {
   const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -217,7 +217,7 @@ __global__ void lattice_table_kernel(const uint32_t *__restrict__ row_off,
     float acc = 0.0f;
     const uint32_t a = row_off[p], b = row_off[p + 1];
     for (uint32_t s = a; s < b; ++s) {
-      const float wt = w[s];
+      const float wt = bitsf(slots[s].y);
       const float tv = ((cfg >> dir[s]) & 1u) ? wt : -wt;
       acc = (s == a) ? tv : acc + tv;
     }
@@ -745,12 +745,12 @@ int launch_pack_low(thrml_state *st) {
   return THRML_OK;
 }
 
-int launch_lattice_table(thrml_prog *p, const uint32_t *d_dir, const float *d_w,
+int launch_lattice_table(thrml_prog *p, const uint32_t *d_dir, const uint2 *d_slots,
                          const float *d_bias) {
   const uint32_t n = (uint32_t)p->blk_off[p->n_free];
   const uint32_t total = n * 16u;
   hipLaunchKernelGGL(lattice_table_kernel, dim3(ceil_div(total, 256)), dim3(256), 0,
-                     p->ctx->stream, p->row_off.as<uint32_t>(), d_dir, d_w, d_bias, n,
+                     p->ctx->stream, p->row_off.as<uint32_t>(), d_dir, d_slots, d_bias, n,
                      p->bias_raw.empty() ? 0 : 1, p->eu.empty() ? 0 : 1, p->table.as<uint32_t>());
   THRML_HIP(hipGetLastError());
   return THRML_OK;

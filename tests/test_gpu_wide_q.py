@@ -133,3 +133,37 @@ def test_q_range_checks(device):
                                  [th.CategoricalEBMFactor([np.arange(2)],
                                                           np.zeros((2, 65537, 1), np.float32))],
                                  [np.array([0, 1])], [], device)
+
+
+@pytest.mark.parametrize("q,n,C,m", [(17, 40, 3, 90), (21, 900, 50, 4000), (33, 5, 1, 6),
+                                     (40, 12000, 64, 24000), (48, 2500, 128, 6000), (95, 300, 60, 900), (129, 64, 2, 100),
+                                     (255, 30, 1, 40), (256, 400, 64, 500), (257, 50, 3, 60),
+                                     (272, 3, 1, 2)])
+def test_lanes_per_item_parity(device, q, n, C, m):
+    """Every number of lanes that can split a site's categories (1 to 64, by
+    items, categories and slots per site), on both program kinds: sites whose
+    first keystream word has every offset, one to three and up to twenty
+    blocks per site, several slots per role and none, infinite biases that
+    send an item to the sequential scan, and near ties."""
+    log_case(f"lanes per item: q={q} n={n} C={C} edges={m}")
+    edges, W, bias, blocks = _random_potts(n, m, q, 2, seed=q + n)
+    bias[0, q - 1] = np.inf
+    bias[1] = -np.inf
+    bias[2] = 0.0
+    W[: max(1, m // 50)] = 0.0
+    rng = np.random.default_rng(n)
+    init = rng.integers(0, q, (C, n)).astype(np.uint16 if q > 256 else np.uint8)
+    o = orc.Potts(n, q, edges, W, bias, blocks)
+    want, _ = o.run_blocks(31, init, 2)
+    prog = th.CategoricalProgram(n, q, edges, W, bias, blocks, device)
+    st = prog.new_state(C)
+    st.set_global(init)
+    th.run_blocks(th.RngKey(31), prog, st, (), 2)
+    assert np.array_equal(st.get_global(), want)
+    fs = [th.CategoricalEBMFactor([np.arange(n)], bias.reshape(n, q, 1)),
+          th.CategoricalEBMFactor([edges[:, 0], edges[:, 1]], W)]
+    fp = th.FactorSamplingProgram(np.ones(n, np.uint8), q, fs, blocks, [], device)
+    sf = fp.new_state(C)
+    sf.set_global(init)
+    th.run_blocks(th.RngKey(31), fp, sf, (), 2)
+    assert np.array_equal(sf.get_global(), want)

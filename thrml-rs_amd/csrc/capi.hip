@@ -933,9 +933,10 @@ extern "C" int thrml_potts_program_create(thrml_ctx *ctx, const thrml_potts_desc
   p->eu.assign(d->edge_u, d->edge_u + d->n_edges);  // for the energies
   p->ev.assign(d->edge_v, d->edge_v + d->n_edges);
   // per position (free and clamped: the energies read every position)
-  std::vector<float> bias((size_t)p->n_total * q);
+  std::vector<float> bias((size_t)p->n_total * q + 2 * ROW_PAD);
   for (uint64_t k = 0; k < p->n_total; ++k)
-    for (uint32_t c = 0; c < q; ++c) bias[k * q + c] = 0.0f + d->biases[(size_t)p->pos_node[k] * q + c];
+    for (uint32_t c = 0; c < q; ++c)
+      bias[ROW_PAD + k * q + c] = 0.0f + d->biases[(size_t)p->pos_node[k] * q + c];
   // weights and their transpose (a u-role slot reads column x_v of W[e], row
   // x_v of W[e]^T); with q <= 16 an all-zero edge E is appended, the padding
   // slots' matrix in the role-padded kernel.  Wider kernels read only the
@@ -977,7 +978,8 @@ extern "C" int thrml_potts_program_create(thrml_ctx *ctx, const thrml_potts_desc
   }
   if ((rc = upload(p, p->row_off, row_off)) || (rc = upload(p, p->uend, uend)) ||
       (rc = upload(p, p->slots, slots)) || (rc = upload(p, p->bias_w, bias)) ||
-      (rc = p->wts.alloc(n_w * sizeof(float))) || (rc = p->wts_t.alloc(n_w * sizeof(float))) ||
+      (rc = p->wts.alloc((n_w + 2 * ROW_PAD) * sizeof(float))) ||
+      (rc = p->wts_t.alloc((n_w + 2 * ROW_PAD) * sizeof(float))) ||
       (p->pm && (rc = upload(p, p->pslots, ps)))) {
     (void)hipStreamSynchronize(ctx->stream);
     delete p;
@@ -985,7 +987,7 @@ extern "C" int thrml_potts_program_create(thrml_ctx *ctx, const thrml_potts_desc
   }
   p->device_bytes += p->wts.bytes + p->wts_t.bytes;
   if (d->n_edges) {
-    const hipError_t ew = hipMemcpyAsync(p->wts.p, d->weights, d->n_edges * qq * sizeof(float),
+    const hipError_t ew = hipMemcpyAsync(padded(p->wts), d->weights, d->n_edges * qq * sizeof(float),
                                          hipMemcpyHostToDevice, ctx->stream);
     if (ew != hipSuccess) {
       (void)hipStreamSynchronize(ctx->stream);
@@ -993,7 +995,7 @@ extern "C" int thrml_potts_program_create(thrml_ctx *ctx, const thrml_potts_desc
       return hip_fail(ew, "program upload");
     }
   }
-  if ((rc = launch_potts_weights(ctx, p->wts.as<float>(), p->wts_t.as<float>(), d->n_edges, q, n_w))) {
+  if ((rc = launch_potts_weights(ctx, padded(p->wts), padded(p->wts_t), d->n_edges, q, n_w))) {
     (void)hipStreamSynchronize(ctx->stream);
     delete p;
     return rc;
@@ -1123,15 +1125,16 @@ extern "C" int thrml_discrete_program_create(thrml_ctx *ctx, const thrml_discret
   if (n_w >= 0xffffffffull) return bail(fail(THRML_EUNSUPPORTED, "more than 2^32-1 factor weights"));
   // at least 16 floats: a slot past a site's last one (the sweep reads the
   // spare record below) reads entries 0..15 of the array and adds nothing
-  std::vector<float> w(std::max<uint64_t>(n_w, 16), 0.0f);
+  std::vector<float> w(std::max<uint64_t>(n_w, 16) + 2 * ROW_PAD, 0.0f);
   for (const DiscFactor &df : fs) {
     const thrml_discrete_factor &F = *df.f;
-    std::copy(F.weights, F.weights + (size_t)F.batch * F.d1 * F.d2, w.begin() + (long)df.w_base);
+    std::copy(F.weights, F.weights + (size_t)F.batch * F.d1 * F.d2,
+              w.begin() + (long)(ROW_PAD + df.w_base));
     if (F.n_cat_groups == 2)
       for (uint64_t b = 0; b < F.batch; ++b)
         for (uint32_t c = 0; c < F.d1; ++c)
           for (uint32_t x = 0; x < F.d2; ++x)
-            w[df.wt_base + (b * F.d2 + x) * F.d1 + c] = F.weights[(b * F.d1 + c) * F.d2 + x];
+            w[ROW_PAD + df.wt_base + (b * F.d2 + x) * F.d1 + c] = F.weights[(b * F.d1 + c) * F.d2 + x];
   }
 
   // slots: a counting pass, then a filling pass
@@ -1206,6 +1209,7 @@ extern "C" int thrml_discrete_program_create(thrml_ctx *ctx, const thrml_discret
   if (sp.size() >= DISC_NONE) return bail(fail(THRML_EUNSUPPORTED, "too many spin tails"));
   p->intra_block_edges = intra;
   plan_staging(p);
+  p->mean_slots = nf ? (uint32_t)((row_off[nf] + nf / 2) / nf) : 0u;
 
   // energy terms: factor rows whose nodes all have a position
   std::vector<uint32_t> terms, tsp;

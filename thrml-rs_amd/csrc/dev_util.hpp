@@ -235,43 +235,19 @@ __device__ __forceinline__ void load_row(const float *row, float (&v)[Q]) {
   }
 }
 
-// Load the 16 floats row[q0 .. q0 + 15] of a row of Q floats (entries
-// outside the row are never used, and are loaded from inside it).  AL = 16:
-// q0 is a multiple of 16 with q0 + 16 <= Q and row 16-byte aligned (four
-// 16-byte loads).  AL = 4: Q and q0 multiples of 4 and row 16-byte aligned,
-// so each group of 4 categories lies wholly inside or wholly outside the row;
-// a group's start is clamped into 0..Q-4 (four 16-byte loads).  AL = 2 alike
-// with Q even and groups of 2 (eight 8-byte loads).  AL = 1: each index
-// clamped into 0..Q-1.
-template <int AL>
-__device__ __forceinline__ void load_chunk16(const float *row, int32_t q0, uint32_t Q,
-                                             float (&v)[16]) {
-  if constexpr (AL == 16 || AL == 4) {
+// Load the 16 floats row[q0 .. q0 + 15] of a row of Q floats, -16 < q0 < Q.
+// Entries outside the row are never used: they are the neighbouring rows' or
+// the ROW_PAD floats before and after the array.  16-byte loads from 4-byte
+// boundaries: 4 instead of 16 for rows that no 16-byte boundary need hold.
+typedef float float4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void load_chunk16(const float *row, int32_t q0, float (&v)[16]) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      int32_t q = q0 + 4 * t;
-      if constexpr (AL == 4) q = q < 0 ? 0 : q > (int32_t)Q - 4 ? (int32_t)Q - 4 : q;
-      const float4 f = *reinterpret_cast<const float4 *>(row + q);
-      v[4 * t] = f.x;
-      v[4 * t + 1] = f.y;
-      v[4 * t + 2] = f.z;
-      v[4 * t + 3] = f.w;
-    }
-  } else if constexpr (AL == 2) {
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      int32_t q = q0 + 2 * t;
-      q = q < 0 ? 0 : q > (int32_t)Q - 2 ? (int32_t)Q - 2 : q;
-      const float2 f = *reinterpret_cast<const float2 *>(row + q);
-      v[2 * t] = f.x;
-      v[2 * t + 1] = f.y;
-    }
-  } else {
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      const int32_t q = q0 + t;
-      v[t] = row[q < 0 ? 0 : q >= (int32_t)Q ? (int32_t)Q - 1 : q];
-    }
+  for (int t = 0; t < 4; ++t) {
+    const float4_a4 f = *reinterpret_cast<const float4_a4 *>(row + q0 + 4 * t);
+    v[4 * t] = f.x;
+    v[4 * t + 1] = f.y;
+    v[4 * t + 2] = f.z;
+    v[4 * t + 3] = f.w;
   }
 }
 
@@ -346,28 +322,28 @@ __device__ __forceinline__ void top2_merge(float &best, float &second, uint32_t 
   best = fmaxf(best, ob);
 }
 
-// wide_pick with the site's keystream blocks split over the 64 lanes of a
-// wave (every lane calls it with the same arguments but its lane index): lane
-// l takes blocks l, l + 64, ... (block k holds categories 16k - o ..
-// 16k - o + 15, as in wide_pick), keeps the top two fast scores and the first
-// maximum of its categories, and a butterfly over the wave merges them; if
-// the top two are within gumbel_margin, every lane scores its categories
-// again with gumbel_b and the first maximum is merged the same way.  The
-// result equals wide_pick's sequential scan: with no NaN the maximum, the
-// runner-up and the first index of the maximum do not depend on the order of
-// the merges; a NaN score (a NaN or infinite weight) sends the item to
-// wide_pick itself, which every lane then runs alike.  Returns the category
-// in every lane.
-template <typename F>
-__device__ __forceinline__ uint32_t wave_pick(uint32_t Q, uint64_t w0, const uint32_t (&key)[8],
-                                              uint32_t lane, F &&theta_chunk) {
+// wide_pick with the site's keystream blocks split over a group of P
+// consecutive lanes (a power of two up to 64; the group's lanes call it with
+// the same arguments but their index sub): lane sub takes blocks sub, sub + P,
+// ... (block k holds categories 16k - o .. 16k - o + 15, as in wide_pick), keeps
+// the top two fast scores and the first maximum of its categories, and a
+// butterfly over the group merges them; if the top two are within
+// gumbel_margin, every lane scores its categories again with gumbel_b and the
+// first maximum is merged the same way.  The result equals wide_pick's
+// sequential scan: with no NaN the maximum, the runner-up and the first index
+// of the maximum do not depend on the order of the merges; a NaN score (a NaN
+// or infinite weight) sends the item to wide_pick itself, which the group's
+// lanes then run alike.  Returns the category in every lane.
+template <int P, typename F>
+__device__ __forceinline__ uint32_t group_pick(uint32_t Q, uint64_t w0, const uint32_t (&key)[8],
+                                               uint32_t sub, F &&theta_chunk) {
   const int32_t o = (int32_t)(w0 & 15u);
   const uint64_t b0 = w0 >> 4;
   const uint32_t nb = ((uint32_t)o + Q + 15u) >> 4;
   float best = -INFINITY, second = -INFINITY;
   uint32_t arg = 0xffffffffu;
   bool nan = false;
-  for (uint32_t k = lane; k < nb; k += 64u) {
+  for (uint32_t k = sub; k < nb; k += P) {
     const int32_t q0 = 16 * (int32_t)k - o;
     float th[16];
     theta_chunk(k, q0, th);
@@ -385,14 +361,16 @@ __device__ __forceinline__ uint32_t wave_pick(uint32_t Q, uint64_t w0, const uin
     }
   }
   // the sequential scan itself (NaN compares make the merges order-dependent)
-  if (__builtin_amdgcn_ballot_w64(nan) != 0u) return wide_pick(Q, w0, key, theta_chunk);
+  uint64_t any_nan = __builtin_amdgcn_ballot_w64(nan);
+  if constexpr (P < 64) any_nan = (any_nan >> (__lane_id() & ~(uint32_t)(P - 1))) & ((1ull << P) - 1ull);
+  if (any_nan != 0u) return wide_pick(Q, w0, key, theta_chunk);
 #pragma unroll
-  for (int m = 32; m > 0; m >>= 1)
+  for (int m = P / 2; m > 0; m >>= 1)
     top2_merge(best, second, arg, __shfl_xor(best, m), __shfl_xor(second, m), __shfl_xor(arg, m));
   if (best - second > gumbel_margin(best, second)) return arg;
   best = -INFINITY;
   arg = 0xffffffffu;
-  for (uint32_t k = lane; k < nb; k += 64u) {
+  for (uint32_t k = sub; k < nb; k += P) {
     const int32_t q0 = 16 * (int32_t)k - o;
     float th[16];
     theta_chunk(k, q0, th);
@@ -411,7 +389,7 @@ __device__ __forceinline__ uint32_t wave_pick(uint32_t Q, uint64_t w0, const uin
     }
   }
 #pragma unroll
-  for (int m = 32; m > 0; m >>= 1) {
+  for (int m = P / 2; m > 0; m >>= 1) {
     const float ob = __shfl_xor(best, m);
     const uint32_t oa = __shfl_xor(arg, m);
     const bool take = ob > best || (ob == best && oa < arg);

@@ -147,7 +147,7 @@ struct thrml_prog {
   thrml::DevBuf pslots;           // Potts: [n_free_total][2*pm] uint2, role-padded slots
   uint32_t pm = 0;                // Potts: padded role width (2 or 4), 0 = unpadded kernel
   uint32_t cat_bytes = 1;         // byte-layout programs: bytes per (position, chain), 2 for q > 256
-  uint32_t mean_slots = 0;        // Potts: slots per free position, rounded
+  uint32_t mean_slots = 0;        // Potts, discrete: slots per free position, rounded
   uint64_t n_edges = 0;
   bool intra_block_edges = false;
   // Superblocks (crates/thrml-samplers/src/program.rs:28-64): superblock s
@@ -409,21 +409,47 @@ int fast_math_gate(thrml_ctx *ctx, float *v_out, int *ok_out);
 // categories of a categorical node: one byte of state per (position, chain)
 constexpr uint32_t POTTS_MAX_Q = 256;       // one byte of state per node
 constexpr uint32_t POTTS_WIDE_MAX_Q = 65536;  // Potts programs: two bytes above 256
-// Categorical blocks with more than 256 categories run one wave per (site,
-// chain) item, the lanes splitting the site's nb = q/16 (+1) keystream
-// blocks, when that is the faster of the two kernels by their measured costs
-// on MI355X (bias-only blocks, q = 300 .. 16384, 16K .. 1M items per launch):
-// the wave kernel about 1.1 ns per item for each keystream block a lane
-// takes (ceil(nb / 64)); the lane kernel about 0.021 ns per item and block
-// once the launch fills the chip, and no less than about 80 us below that
-// (each lane walks its nb blocks in sequence).
-constexpr uint32_t POTTS_WAVE_MIN_Q = 257;
-inline bool potts_wave_pays(uint32_t q, uint64_t items) {
-  const double nb = (double)((q + 30u) / 16u);
-  const double t_wave = (double)items * std::ceil(nb / 64.0) * 1.1e-3;  // us
-  const double t_lane = std::max(80.0, (double)items * nb * 0.021e-3);
-  return q >= POTTS_WAVE_MIN_Q && t_wave < t_lane;
+// Lanes per (site, chain) item of the wide kernels (q > 16): P lanes split a
+// site's keystream blocks of 16 categories, nb = (offset of its first word +
+// q + 15) / 16 of them, in ceil(nb / P) steps each.  Fitted to launches on
+// MI355X (tori of side 16 .. 256 and Erdos-Renyi graphs, q = 17 .. 256, 1 ..
+// 128 chains; bias-only blocks of q = 300 .. 16384), in us:
+//   2 + steps (1.2 + 0.8 slots) + 1.1 items P steps (17 + 5 slots) / 10^6;
+// for P = 1 and 2, which read one and two slots at a time, 1.5 and 1.1 instead
+// of 0.8 and 1 instead of 1.1.  The first part is one wave's chain of dependent
+// loads, the second the whole chip's issue, to which idle lanes count as much
+// as busy ones.
+//   us per launch                        P = 1     2     4     8    16
+//   E-R 10007 deg 8, q = 21, 62K items      37    21    19    29    51
+//   E-R 1000 deg 8, q = 100, 7K items      111    49    23    15    15
+//   128^2, q = 32, 1M items                 79    70   121   234   459
+//   16^2, q = 256, 1K items                 62    33    16   9.5   6.0
+inline uint32_t wide_lanes(uint32_t q, uint64_t items, uint32_t slots) {
+  uint32_t step = 16u;  // the offsets a site's first word can have: multiples of gcd(q, 16)
+  while (q % step) step /= 2u;
+  uint32_t best = 1u;
+  double best_t = 0.0;
+  for (uint32_t P = 1; P <= (q > 256u ? 64u : 16u); P *= P == 16u ? 4u : 2u) {
+    if (items * P >= (1ull << 32)) break;  // lanes are indexed in 32 bits
+    double steps = 0.0;
+    for (uint32_t o = 0; o < 16u; o += step) steps += (double)(((o + q + 15u) / 16u + P - 1u) / P);
+    steps /= 16u / step;
+    const double t = 2.0 + steps * (1.2 + (P == 1u ? 1.5 : P == 2u ? 1.1 : 0.8) * slots) +
+                     (P > 2u ? 1.1 : 1.0) * (double)items * P * steps * (17.0 + 5.0 * slots) * 1e-6;
+    if (P == 1u || t < best_t) {
+      best = P;
+      best_t = t;
+    }
+  }
+  return best;
 }
+
+// Weight rows may be loaded up to 15 floats past either end (load_chunk16):
+// their arrays carry ROW_PAD floats before and after (256 bytes, so that rows
+// of 32 floats still lie in one cache line each: 64 bytes cost a 256^2 torus
+// of 32 categories 8 %).
+constexpr uint32_t ROW_PAD = 64;
+inline float *padded(const DevBuf &b) { return b.as<float>() + ROW_PAD; }
 
 constexpr uint32_t BATCH_GATHER_MAX_INDICES = 64;
 struct BatchGatherStrides {

@@ -16,9 +16,7 @@
 // quarter of a keystream block), lcm(q, 16) / q for categories (whole
 // blocks); consecutive lanes are consecutive chains, so a site's slot
 // records are read by all of its chains at once.  Spin sites are summed four
-// at a time with their slots interleaved.  q = 17..256: one categorical site
-// per lane, its categories one keystream block at a time
-// (discrete_wide_kernel).  The generic path: the
+// at a time with their slots interleaved.  q > 16: discrete_wide_kernel.  The generic path: the
 // benchmarked Ising and categorical programs have their own kernels.
 #include "dev_util.hpp"
 #include "internal.hpp"
@@ -288,22 +286,19 @@ void discrete_half_kernel(DiscArgs a) {
   }
 }
 
-// Categorical blocks with 16 < Q <= 256 categories: one lane per (site,
-// chain).  The site's categories go one keystream block at a time
-// (wide_pick); for each, the slots are walked again and summed per category
-// as above (groups from their first slot, added to theta in order), the
-// first four slots' rows and signs kept from one read.  AL (load_chunk16):
-// 16 for Q a multiple of 16, 4 for Q a multiple of 4, 2 for even Q (weight
-// rows start at multiples of 4 floats), else 1.
-// WAVE: one wave per item, its lanes splitting the site's keystream blocks
-// (wave_pick; two-byte programs with few items for their categories,
-// potts_wave_pays), else one lane per item.
-template <int AL, class T = uint8_t, bool WAVE = false>
+// Categorical blocks with 16 < Q <= 65536 categories: P consecutive lanes per
+// (site, chain), splitting the site's keystream blocks of 16 categories
+// (wide_pick, group_pick), as the categorical programs' wide kernel.  For each
+// block the slots are walked again and summed per category as above (groups
+// from their first slot, added to theta in order).  P = 1 keeps the first four
+// slots' rows and signs from one read; P > 1, with one block per lane or few,
+// takes the slots four at a time, so that their chains of dependent loads
+// overlap.
+template <class T, int P>
 __global__ __launch_bounds__(256) void discrete_wide_kernel(DiscArgs a, uint32_t Q) {
   const T *state = reinterpret_cast<const T *>(a.state);
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t item = WAVE ? blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)
-                             : blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t item = P == 64 ? blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)
+                                : (blockIdx.x * 256u + threadIdx.x) / (uint32_t)P;
   if (item >= a.n_items) return;
   const uint32_t i = fdiv(item, a.div_c);
   const uint32_t c = item - i * a.C;
@@ -311,10 +306,9 @@ __global__ __launch_bounds__(256) void discrete_wide_kernel(DiscArgs a, uint32_t
   load_key8(a.keys, c, key);
   const uint32_t pos = a.blk_off + i;
   const uint32_t k0 = a.row_off[pos], deg = a.row_off[pos + 1] - k0;
-  // slot j: its row's offset in W, and its sign (bit 0) and group-start
+  // slot record r: its row's offset in W, and its sign (bit 0) and group-start
   // (bit 1) flags
-  auto slot = [&](uint32_t j, uint32_t &off, uint32_t &fl) {
-    const uint4 r = a.slots[k0 + j];
+  auto slot = [&](const uint4 &r, uint32_t &off, uint32_t &fl) {
     const uint32_t nsp = r.w & 255u;
     uint32_t neg = 0u;
     for (uint32_t t = 0; t < nsp; ++t)
@@ -323,51 +317,77 @@ __global__ __launch_bounds__(256) void discrete_wide_kernel(DiscArgs a, uint32_t
     off = r.x + (((r.w >> 9) & 3u) == 2u ? x * Q : 0u);
     fl = neg | (((r.w >> 8) & 1u) << 1);
   };
-  // the first 4 slots are read once for all blocks
-  uint32_t ro[4], rf[4];
-#pragma unroll
-  for (uint32_t j = 0; j < 4; ++j) {
-    ro[j] = rf[j] = 0u;
-    if (j < deg) slot(j, ro[j], rf[j]);
-  }
-  auto theta_chunk = [&](uint32_t, int32_t q0, float (&th)[16]) {
-    float acc[16];
-#pragma unroll
-    for (int t = 0; t < 16; ++t) th[t] = acc[t] = 0.0f;
-    for (uint32_t j = 0; j < deg; ++j) {
-      uint32_t off, fl;
-      if (j < 4u) {
-        off = j == 0 ? ro[0] : j == 1 ? ro[1] : j == 2 ? ro[2] : ro[3];
-        fl = j == 0 ? rf[0] : j == 1 ? rf[1] : j == 2 ? rf[2] : rf[3];
-      } else {
-        slot(j, off, fl);
-      }
-      const bool neg = fl & 1u;
-      float wv[16];
-      load_chunk16<AL>(a.W + off, q0, Q, wv);
-      const bool first = fl & 2u;
-      if (first && j != 0u) {
-#pragma unroll
-        for (int t = 0; t < 16; ++t) th[t] = th[t] + acc[t];
-      }
-#pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        const float v = neg ? -wv[t] : wv[t];
-        acc[t] = first ? v : acc[t] + v;
-      }
-    }
-    if (deg) {
+  // adds slot j's row to the sums
+  auto add = [&](uint32_t j, uint32_t fl, const float (&wv)[16], float (&th)[16], float (&acc)[16]) {
+    const bool neg = fl & 1u, first = fl & 2u;
+    if (first && j != 0u) {
 #pragma unroll
       for (int t = 0; t < 16; ++t) th[t] = th[t] + acc[t];
     }
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      const float v = neg ? -wv[t] : wv[t];
+      acc[t] = first ? v : acc[t] + v;
+    }
   };
-  if constexpr (WAVE) {
-    const uint32_t arg = wave_pick(Q, (uint64_t)i * Q, key, lane, theta_chunk);
-    if (lane == 0u) reinterpret_cast<T *>(a.out)[(size_t)i * a.Cp + c] = (T)arg;
+  uint32_t arg;
+  if constexpr (P == 1) {
+    uint32_t ro[4], rf[4];
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+      ro[j] = rf[j] = 0u;
+      if (j < deg) slot(a.slots[k0 + j], ro[j], rf[j]);
+    }
+    arg = wide_pick(Q, (uint64_t)i * Q, key, [&](uint32_t, int32_t q0, float(&th)[16]) {
+      float acc[16];
+#pragma unroll
+      for (int t = 0; t < 16; ++t) th[t] = acc[t] = 0.0f;
+      for (uint32_t j = 0; j < deg; ++j) {
+        uint32_t off, fl;
+        if (j < 4u) {
+          off = j == 0 ? ro[0] : j == 1 ? ro[1] : j == 2 ? ro[2] : ro[3];
+          fl = j == 0 ? rf[0] : j == 1 ? rf[1] : j == 2 ? rf[2] : rf[3];
+        } else {
+          slot(a.slots[k0 + j], off, fl);
+        }
+        float wv[16];
+        load_chunk16(a.W + off, q0, wv);
+        add(j, fl, wv, th, acc);
+      }
+      if (deg) {
+#pragma unroll
+        for (int t = 0; t < 16; ++t) th[t] = th[t] + acc[t];
+      }
+    });
   } else {
-    const uint32_t arg = wide_pick(Q, (uint64_t)i * Q, key, theta_chunk);
-    reinterpret_cast<T *>(a.out)[(size_t)i * a.Cp + c] = (T)arg;
+    const uint32_t sub = threadIdx.x & (uint32_t)(P - 1);
+    arg = group_pick<P>(Q, (uint64_t)i * Q, key, sub, [&](uint32_t, int32_t q0, float(&th)[16]) {
+      constexpr int U = P == 2 ? 2 : 4;
+      float acc[16];
+#pragma unroll
+      for (int t = 0; t < 16; ++t) th[t] = acc[t] = 0.0f;
+      for (uint32_t j = 0; j < deg; j += U) {
+        uint4 r[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) r[u] = a.slots[k0 + min(j + (uint32_t)u, deg - 1u)];
+        uint32_t off[U], fl[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) slot(r[u], off[u], fl[u]);
+        float wv[U][16];
+#pragma unroll
+        for (int u = 0; u < U; ++u) load_chunk16(a.W + off[u], q0, wv[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (j + (uint32_t)u < deg) add(j + (uint32_t)u, fl[u], wv[u], th, acc);
+      }
+      if (deg) {
+#pragma unroll
+        for (int t = 0; t < 16; ++t) th[t] = th[t] + acc[t];
+      }
+    });
+    if (sub != 0u) return;
   }
+  reinterpret_cast<T *>(a.out)[(size_t)i * a.Cp + c] = (T)arg;
 }
 
 static inline uint32_t cdiv32(uint64_t x, uint64_t y) { return (uint32_t)((x + y - 1) / y); }
@@ -375,6 +395,24 @@ static inline uint32_t cdiv32(uint64_t x, uint64_t y) { return (uint32_t)((x + y
 template <int Q, class T = uint8_t>
 static void launch_dq(const DiscArgs &a, hipStream_t s) {
   hipLaunchKernelGGL((discrete_half_kernel<Q, T>), dim3(cdiv32(a.n_items, 256)), dim3(256), 0, s, a);
+}
+
+template <class T, int P>
+static void launch_wide_p(const DiscArgs &a, uint32_t Q, hipStream_t s) {
+  hipLaunchKernelGGL((discrete_wide_kernel<T, P>), dim3(cdiv32((uint64_t)a.n_items * P, 256)),
+                     dim3(256), 0, s, a, Q);
+}
+template <class T>
+static void launch_wide(const DiscArgs &a, uint32_t Q, uint32_t P, hipStream_t s) {
+  switch (P) {
+    case 1: launch_wide_p<T, 1>(a, Q, s); break;
+    case 2: launch_wide_p<T, 2>(a, Q, s); break;
+    case 4: launch_wide_p<T, 4>(a, Q, s); break;
+    case 8: launch_wide_p<T, 8>(a, Q, s); break;
+    case 16: launch_wide_p<T, 16>(a, Q, s); break;
+    default:
+      if constexpr (sizeof(T) == 2) launch_wide_p<T, 64>(a, Q, s);
+  }
 }
 
 int launch_discrete_half(thrml_prog *p, thrml_state *st, uint32_t b, const uint32_t *d_keys) {
@@ -396,7 +434,7 @@ int launch_discrete_half(thrml_prog *p, thrml_state *st, uint32_t b, const uint3
   a.row_off = p->row_off.as<uint32_t>();
   a.slots = p->d_slots.as<uint4>();
   a.sp = p->d_sp.as<uint32_t>();
-  a.W = p->d_w.as<float>();
+  a.W = padded(p->d_w);
   a.keys = d_keys;
   a.n_b = n_b;
   a.blk_off = (uint32_t)p->blk_off[b];
@@ -438,23 +476,9 @@ int launch_discrete_half(thrml_prog *p, thrml_state *st, uint32_t b, const uint3
     default: {
       if (Q > (p->cat_bytes == 2 ? POTTS_WIDE_MAX_Q : POTTS_MAX_Q))
         return fail(THRML_EINVAL, "q must lie in 2..65536");
-      const dim3 grid(cdiv32(a.n_items, 256));
-      if (potts_wave_pays(Q, a.n_items)) {
-        // few items for their categories (two-byte states): one wave per item
-        const dim3 wg(cdiv32(a.n_items, 4));
-        if (Q % 16 == 0) hipLaunchKernelGGL((discrete_wide_kernel<16, uint16_t, true>), wg, dim3(256), 0, s, a, Q);
-        else if (Q % 4 == 0) hipLaunchKernelGGL((discrete_wide_kernel<4, uint16_t, true>), wg, dim3(256), 0, s, a, Q);
-        else if (Q % 2 == 0) hipLaunchKernelGGL((discrete_wide_kernel<2, uint16_t, true>), wg, dim3(256), 0, s, a, Q);
-        else hipLaunchKernelGGL((discrete_wide_kernel<1, uint16_t, true>), wg, dim3(256), 0, s, a, Q);
-      } else if (p->cat_bytes == 2) {
-        if (Q % 16 == 0) hipLaunchKernelGGL((discrete_wide_kernel<16, uint16_t>), grid, dim3(256), 0, s, a, Q);
-        else if (Q % 4 == 0) hipLaunchKernelGGL((discrete_wide_kernel<4, uint16_t>), grid, dim3(256), 0, s, a, Q);
-        else if (Q % 2 == 0) hipLaunchKernelGGL((discrete_wide_kernel<2, uint16_t>), grid, dim3(256), 0, s, a, Q);
-        else hipLaunchKernelGGL((discrete_wide_kernel<1, uint16_t>), grid, dim3(256), 0, s, a, Q);
-      } else if (Q % 16 == 0) hipLaunchKernelGGL(discrete_wide_kernel<16>, grid, dim3(256), 0, s, a, Q);
-      else if (Q % 4 == 0) hipLaunchKernelGGL(discrete_wide_kernel<4>, grid, dim3(256), 0, s, a, Q);
-      else if (Q % 2 == 0) hipLaunchKernelGGL(discrete_wide_kernel<2>, grid, dim3(256), 0, s, a, Q);
-      else hipLaunchKernelGGL(discrete_wide_kernel<1>, grid, dim3(256), 0, s, a, Q);
+      const uint32_t P = wide_lanes(Q, a.n_items, p->mean_slots);
+      if (p->cat_bytes == 2) launch_wide<uint16_t>(a, Q, P, s);
+      else launch_wide<uint8_t>(a, Q, P, s);
     }
   }
   THRML_HIP(hipGetLastError());
@@ -514,7 +538,7 @@ int discrete_energy(thrml_prog *p, thrml_state *st, double *out) {
   a.cat16 = p->cat_bytes == 2 ? st->cat.as<uint16_t>() : nullptr;
   a.terms = p->d_terms.as<uint4>();
   a.tsp = p->d_tsp.as<uint32_t>();
-  a.W = p->d_w.as<float>();
+  a.W = padded(p->d_w);
   a.n_terms = p->d_nterms;
   a.n_ch = std::max<uint32_t>(1u, cdiv32(p->d_nterms, DISC_EN_CHUNK));
   a.C = st->C;

@@ -276,8 +276,8 @@ int potts_energy(thrml_prog *p, thrml_state *st, double *out) {
   a.cat = p->cat_bytes == 1 ? st->cat.as<uint8_t>() : nullptr;
   a.cat16 = p->cat_bytes == 2 ? st->cat.as<uint16_t>() : nullptr;
   a.epos = p->en_pos.as<uint2>();
-  a.W = p->wts.as<float>();
-  a.bias = p->bias_w.as<float>();
+  a.W = padded(p->wts);
+  a.bias = padded(p->bias_w);
   a.n_e = p->en_ne;
   a.n_pos = p->n_total;
   a.Cp = st->Cp;

@@ -18,8 +18,7 @@
 // block key's ChaCha8 stream) are exactly lcm(Q, 16) / 16 whole ChaCha8
 // blocks; lanes of one wave are consecutive chains of the same run, so a
 // site's slot lists and bias row are shared by the wave and the chains'
-// neighbour bytes are contiguous.  Q = 17..256 (potts_wide_kernel): a lane
-// takes one site and walks its categories one keystream block at a time.
+// neighbour bytes are contiguous.  Q > 16: potts_wide_kernel.
 #include "dev_util.hpp"
 #include "internal.hpp"
 
@@ -207,14 +206,13 @@ __global__ __launch_bounds__(256) void potts_half_kernel(PottsArgs a) {
 // (entries outside 0..Q-1 are ignored by the caller): ((0 + b) + sum_u) +
 // sum_v, each role summed over its slots in order, as in the generic kernel.
 // s0, s1, s2 delimit the position's u-role and v-role slots; ro holds the row
-// offsets (edge * Q + x_t) * Q of its first four slots.  AL (load_chunk16):
-// 16 for Q a multiple of 16, 4 for Q a multiple of 4, 2 for even Q, else 1.
-template <int AL, class T>
+// offsets (edge * Q + x_t) * Q of its first four slots.
+template <class T>
 __device__ __forceinline__ void wide_theta(const PottsArgs &a, const T *state, uint32_t Q,
                                            uint32_t pos, uint32_t c, uint32_t s0, uint32_t s1,
                                            uint32_t s2, const uint64_t (&ro)[4], int32_t q0,
                                            float (&th)[16]) {
-  load_chunk16<AL>(a.bias + (size_t)pos * Q, q0, Q, th);
+  load_chunk16(a.bias + (size_t)pos * Q, q0, th);
   for (int role = 0; role < 2; ++role) {
     const uint32_t k0 = role ? s1 : s0, k1 = role ? s2 : s1;
     if (k0 == k1) continue;  // an empty role adds nothing: theta is never -0 (bias is 0 + b)
@@ -231,7 +229,7 @@ __device__ __forceinline__ void wide_theta(const PottsArgs &a, const T *state, u
         off = ((uint64_t)sl.y * Q + state[(size_t)sl.x * a.Cp + c]) * Q;
       }
       float we[16];
-      load_chunk16<AL>(w + off, q0, Q, we);
+      load_chunk16(w + off, q0, we);
 #pragma unroll
       for (int t = 0; t < 16; ++t) sr[t] = (k == k0) ? we[t] : sr[t] + we[t];
     }
@@ -263,51 +261,88 @@ __device__ __forceinline__ void wide_slots(const PottsArgs &a, const T *state, u
   }
 }
 
-// Wide kernel (16 < Q <= 65536): one lane per (site, chain).  The site's Q
-// categories go one keystream block at a time (wide_pick), so a lane holds 16
-// of them; slot records and tail bytes past a site's fourth slot are read
-// again for every block (they stay in the caches).
+// wide_theta for a lane that takes one keystream block of its site (or few):
+// U slots at a time, their records, then their tails, then their rows loaded
+// together, so that the chains of dependent loads overlap U-fold.  A slot past
+// the role's last loads that one again and adds nothing.
+template <int U, class T>
+__device__ __forceinline__ void group_theta(const PottsArgs &a, const T *state, uint32_t Q,
+                                            uint32_t pos, uint32_t c, uint32_t s0, uint32_t s1,
+                                            uint32_t s2, int32_t q0, float (&th)[16]) {
+  load_chunk16(a.bias + (size_t)pos * Q, q0, th);
+  float sr[16];
+  for (uint32_t k = s0; k < s2; k += U) {
+    uint2 sl[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) sl[u] = a.slots[min(k + (uint32_t)u, s2 - 1u)];
+    uint32_t xt[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) xt[u] = state[(size_t)sl[u].x * a.Cp + c];
+    float we[U][16];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      // u-role: column x_v of W[e], row x_v of the transposed copy
+      const float *w = min(k + (uint32_t)u, s2 - 1u) < s1 ? a.Wt : a.W;
+      load_chunk16(w + ((uint64_t)sl[u].y * Q + xt[u]) * Q, q0, we[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t j = k + (uint32_t)u;
+      if (j < s2) {
+        const bool first = j == s0 || j == s1;
+        if (j == s1 && s1 > s0) {  // the u-role's sum is whole
+#pragma unroll
+          for (int t = 0; t < 16; ++t) th[t] = th[t] + sr[t];
+        }
+#pragma unroll
+        for (int t = 0; t < 16; ++t) sr[t] = first ? we[u][t] : sr[t] + we[u][t];
+      }
+    }
+  }
+  // an empty role adds nothing: theta is never -0 (bias is 0 + b)
+  if (s2 > s0) {
+#pragma unroll
+    for (int t = 0; t < 16; ++t) th[t] = th[t] + sr[t];
+  }
+}
+
+// Wide kernel (16 < Q <= 65536): P consecutive lanes per (site, chain),
+// splitting the site's keystream blocks of 16 categories (wide_pick, group_pick).
+// P = 1: a lane walks its site's Q categories one block at a time; slot
+// records and tails past a site's fourth slot are read again for every block
+// (they stay in the caches).
 // T: the state's element, uint8_t (q <= 256) or uint16_t (q up to 65536).
-template <int AL, class T = uint8_t>
+template <class T, int P>
 __global__ __launch_bounds__(256) void potts_wide_kernel(PottsArgs a, uint32_t Q) {
   const T *state = reinterpret_cast<const T *>(a.state);
-  const uint32_t item = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t item = P == 64 ? blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)
+                                : (blockIdx.x * 256u + threadIdx.x) / (uint32_t)P;
   if (item >= a.n_items) return;
   const uint32_t i = fdiv(item, a.div_c);
   const uint32_t c = item - i * a.C;
   uint32_t key[8];
   load_key8(a.keys, c, key);
   const uint32_t pos = a.blk_off + i;
-  uint32_t s0, s1, s2;
-  uint64_t ro[4];
-  wide_slots(a, state, Q, pos, c, s0, s1, s2, ro);
-  const uint32_t arg = wide_pick(Q, (uint64_t)i * Q, key, [&](uint32_t, int32_t q0, float(&th)[16]) {
-    wide_theta<AL>(a, state, Q, pos, c, s0, s1, s2, ro, q0, th);
-  });
+  uint32_t arg;
+  if constexpr (P == 1) {
+    uint32_t s0, s1, s2;
+    uint64_t ro[4];
+    wide_slots(a, state, Q, pos, c, s0, s1, s2, ro);
+    arg = wide_pick(Q, (uint64_t)i * Q, key, [&](uint32_t, int32_t q0, float(&th)[16]) {
+      wide_theta(a, state, Q, pos, c, s0, s1, s2, ro, q0, th);
+    });
+  } else {
+    const uint32_t sub = threadIdx.x & (uint32_t)(P - 1);
+    const uint32_t s0 = a.has_edges ? a.row_off[pos] : 0u, s1 = a.has_edges ? a.uend[pos] : 0u;
+    const uint32_t s2 = a.has_edges ? a.row_off[pos + 1] : 0u;
+    // (P = 2 runs the large launches, where occupancy pays more than overlap)
+    constexpr int U = P == 2 ? 2 : 4;
+    arg = group_pick<P>(Q, (uint64_t)i * Q, key, sub, [&](uint32_t, int32_t q0, float(&th)[16]) {
+      group_theta<U>(a, state, Q, pos, c, s0, s1, s2, q0, th);
+    });
+    if (sub != 0u) return;
+  }
   reinterpret_cast<T *>(a.out)[(size_t)i * a.Cp + c] = (T)arg;
-}
-
-// Wave kernel for few (site, chain) items with many categories each
-// (potts_wave_pays; Q > 256): one wave per item, the lanes splitting the
-// site's keystream blocks (wave_pick).
-template <int AL, class T>
-__global__ __launch_bounds__(256) void potts_wave_kernel(PottsArgs a, uint32_t Q) {
-  const T *state = reinterpret_cast<const T *>(a.state);
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t item = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (item >= a.n_items) return;  // wave-uniform
-  const uint32_t i = fdiv(item, a.div_c);
-  const uint32_t c = item - i * a.C;
-  uint32_t key[8];
-  load_key8(a.keys, c, key);
-  const uint32_t pos = a.blk_off + i;
-  uint32_t s0, s1, s2;
-  uint64_t ro[4];
-  wide_slots(a, state, Q, pos, c, s0, s1, s2, ro);
-  const uint32_t out = wave_pick(Q, (uint64_t)i * Q, key, lane, [&](uint32_t, int32_t q0, float(&th)[16]) {
-    wide_theta<AL>(a, state, Q, pos, c, s0, s1, s2, ro, q0, th);
-  });
-  if (lane == 0u) reinterpret_cast<T *>(a.out)[(size_t)i * a.Cp + c] = (T)out;
 }
 
 // Role-padded kernel (Q a multiple of 4, at most M u-role and M v-role slots
@@ -568,6 +603,24 @@ static void launch_q(const PottsArgs &a, uint32_t pm, uint32_t mean_slots, hipSt
   else hipLaunchKernelGGL((potts_half_kernel<Q, Q <= 8 ? 4 : 2>), g, dim3(256), 0, s, b);
 }
 
+template <class T, int P>
+static void launch_wide_p(const PottsArgs &a, uint32_t Q, hipStream_t s) {
+  hipLaunchKernelGGL((potts_wide_kernel<T, P>), dim3(cdiv32((uint64_t)a.n_items * P, 256)), dim3(256),
+                     0, s, a, Q);
+}
+template <class T>
+static void launch_wide(const PottsArgs &a, uint32_t Q, uint32_t P, hipStream_t s) {
+  switch (P) {
+    case 1: launch_wide_p<T, 1>(a, Q, s); break;
+    case 2: launch_wide_p<T, 2>(a, Q, s); break;
+    case 4: launch_wide_p<T, 4>(a, Q, s); break;
+    case 8: launch_wide_p<T, 8>(a, Q, s); break;
+    case 16: launch_wide_p<T, 16>(a, Q, s); break;
+    default:
+      if constexpr (sizeof(T) == 2) launch_wide_p<T, 64>(a, Q, s);
+  }
+}
+
 int launch_potts_half(thrml_prog *p, thrml_state *st, uint32_t b, const uint32_t *d_keys) {
   const uint32_t n_b = (uint32_t)(p->blk_off[b + 1] - p->blk_off[b]);
   const uint32_t Q = p->q;
@@ -584,9 +637,9 @@ int launch_potts_half(thrml_prog *p, thrml_state *st, uint32_t b, const uint32_t
   a.row_off = p->row_off.as<uint32_t>();
   a.uend = p->uend.as<uint32_t>();
   a.slots = p->slots.as<uint2>();
-  a.bias = p->bias_w.as<float>();
-  a.W = p->wts.as<float>();
-  a.Wt = p->wts_t.as<float>();
+  a.bias = padded(p->bias_w);
+  a.W = padded(p->wts);
+  a.Wt = padded(p->wts_t);
   a.pslots = p->pm ? p->pslots.as<uint4>() : nullptr;
   a.keys = d_keys;
   a.n_b = n_b;
@@ -631,24 +684,9 @@ int launch_potts_half(thrml_prog *p, thrml_state *st, uint32_t b, const uint32_t
       if ((uint64_t)n_b * st->C >= (1ull << 31))
         return fail(THRML_EINVAL, "categorical block too large: sites x chains must stay below 2^31");
       a.n_items = n_b * st->C;
-      const dim3 grid(cdiv32(a.n_items, 256));
-      if (potts_wave_pays(Q, a.n_items)) {
-        // few items for their categories (two-byte states): one wave per item
-        static_assert(POTTS_WAVE_MIN_Q > POTTS_MAX_Q, "the wave kernel reads two-byte states");
-        const dim3 wg(cdiv32(a.n_items, 4));
-        if (Q % 16 == 0) hipLaunchKernelGGL((potts_wave_kernel<16, uint16_t>), wg, dim3(256), 0, s, a, Q);
-        else if (Q % 4 == 0) hipLaunchKernelGGL((potts_wave_kernel<4, uint16_t>), wg, dim3(256), 0, s, a, Q);
-        else if (Q % 2 == 0) hipLaunchKernelGGL((potts_wave_kernel<2, uint16_t>), wg, dim3(256), 0, s, a, Q);
-        else hipLaunchKernelGGL((potts_wave_kernel<1, uint16_t>), wg, dim3(256), 0, s, a, Q);
-      } else if (p->cat_bytes == 2) {
-        if (Q % 16 == 0) hipLaunchKernelGGL((potts_wide_kernel<16, uint16_t>), grid, dim3(256), 0, s, a, Q);
-        else if (Q % 4 == 0) hipLaunchKernelGGL((potts_wide_kernel<4, uint16_t>), grid, dim3(256), 0, s, a, Q);
-        else if (Q % 2 == 0) hipLaunchKernelGGL((potts_wide_kernel<2, uint16_t>), grid, dim3(256), 0, s, a, Q);
-        else hipLaunchKernelGGL((potts_wide_kernel<1, uint16_t>), grid, dim3(256), 0, s, a, Q);
-      } else if (Q % 16 == 0) hipLaunchKernelGGL(potts_wide_kernel<16>, grid, dim3(256), 0, s, a, Q);
-      else if (Q % 4 == 0) hipLaunchKernelGGL(potts_wide_kernel<4>, grid, dim3(256), 0, s, a, Q);
-      else if (Q % 2 == 0) hipLaunchKernelGGL(potts_wide_kernel<2>, grid, dim3(256), 0, s, a, Q);
-      else hipLaunchKernelGGL(potts_wide_kernel<1>, grid, dim3(256), 0, s, a, Q);
+      const uint32_t P = wide_lanes(Q, a.n_items, p->mean_slots);
+      if (p->cat_bytes == 2) launch_wide<uint16_t>(a, Q, P, s);
+      else launch_wide<uint8_t>(a, Q, P, s);
     }
   }
   THRML_HIP(hipGetLastError());

@@ -294,6 +294,10 @@ int thrml_state_set_block(thrml_state *st, uint32_t b, const void *src, int dtyp
                           int src_on_device);
 int thrml_state_get_block(thrml_state *st, uint32_t b, void *dst, int dtype,
                           int dst_on_device);
+/* The whole global state as [n_chains][n_total] (free blocks, then clamped
+ * blocks), in one transfer.  A rejected write leaves the state unchanged. */
+int thrml_state_set_global(thrml_state *st, const void *src, int dtype, int src_on_device);
+int thrml_state_get_global(thrml_state *st, void *dst, int dtype, int dst_on_device);
 
 /* ---- execution ----------------------------------------------------------- */
 /* hinton_init (crates/thrml-models/src/ising.rs:602-673) of every free
@@ -389,10 +393,10 @@ int thrml_observer_run(thrml_prog *prog, uint64_t key, thrml_schedule sched, thr
  * with the chains' state in place on the device and the context's stream
  * (hipStream_t), on which the sweeps before it are queued and those after it
  * will be.  The observer keeps its own carry behind `user`.  It may read the
- * state (thrml_state_get_block per block, into host or device memory) and
+ * state (thrml_state_get_block, thrml_state_get_global, into host or device memory) and
  * queue work of its own on that stream (the later sweeps then
  * wait for it), but must not change the state or start a run on the same
- * context: thrml_state_set_block, thrml_hinton_init and every run entry point
+ * context: thrml_state_set_block / _global, thrml_hinton_init and every run entry point
  * called from inside it on that context fail with THRML_EINVAL.  A nonzero
  * return stops the run and is returned. */
 typedef int (*thrml_observe_fn)(void *user, uint64_t iteration, thrml_state *st, void *hip_stream);

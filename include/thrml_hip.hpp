@@ -505,39 +505,30 @@ class State {
   Result<std::vector<uint16_t>> get_global16() const { return get_global_as<uint16_t>(); }
 
  private:
-  // blocks cross the C ABI as u8 for byte values, as f32 otherwise
+  // the state crosses the C ABI as u8 for byte values, as f32 otherwise
   template <class T>
   Result<void> set_global_as(const std::vector<T> &g) {
-    constexpr int dt = sizeof(T) == 1 ? THRML_DTYPE_U8 : THRML_DTYPE_F32;
-    using E = typename std::conditional<sizeof(T) == 1, uint8_t, float>::type;
-    const uint64_t nt = prog_->n_total();
-    if (g.size() != (size_t)C_ * nt) return Result<void>::err(THRML_EINVAL, "state has the wrong size");
-    const uint32_t nb = (uint32_t)(prog_->free_blocks().size() + prog_->clamped_blocks().size());
-    for (uint32_t b = 0; b < nb; ++b) {
-      const auto r = prog_->block_range(b);
-      std::vector<E> blk((size_t)C_ * r.second);
-      for (uint32_t c = 0; c < C_; ++c)
-        for (uint64_t i = 0; i < r.second; ++i) blk[(size_t)c * r.second + i] = (E)g[(size_t)c * nt + r.first + i];
-      const auto rc = detail::check(thrml_state_set_block(h_, b, blk.data(), dt, 0));
-      if (rc.is_err()) return rc;
+    if (g.size() != (size_t)C_ * prog_->n_total())
+      return Result<void>::err(THRML_EINVAL, "state has the wrong size");
+    if constexpr (sizeof(T) == 1) {
+      return detail::check(thrml_state_set_global(h_, g.data(), THRML_DTYPE_U8, 0));
+    } else {
+      const std::vector<float> f(g.begin(), g.end());
+      return detail::check(thrml_state_set_global(h_, f.data(), THRML_DTYPE_F32, 0));
     }
-    return Result<void>::ok();
   }
   template <class T>
   Result<std::vector<T>> get_global_as() const {
-    constexpr int dt = sizeof(T) == 1 ? THRML_DTYPE_U8 : THRML_DTYPE_F32;
-    using E = typename std::conditional<sizeof(T) == 1, uint8_t, float>::type;
-    const uint64_t nt = prog_->n_total();
-    std::vector<T> g((size_t)C_ * nt);
-    const uint32_t nb = (uint32_t)(prog_->free_blocks().size() + prog_->clamped_blocks().size());
-    for (uint32_t b = 0; b < nb; ++b) {
-      const auto r = prog_->block_range(b);
-      std::vector<E> blk((size_t)C_ * r.second);
-      const int rc = thrml_state_get_block(h_, b, blk.data(), dt, 0);
-      if (rc != THRML_OK) return detail::fail<std::vector<T>>(rc);
-      for (uint32_t c = 0; c < C_; ++c)
-        for (uint64_t i = 0; i < r.second; ++i) g[(size_t)c * nt + r.first + i] = (T)blk[(size_t)c * r.second + i];
+    std::vector<T> g((size_t)C_ * prog_->n_total());
+    int rc;
+    if constexpr (sizeof(T) == 1) {
+      rc = thrml_state_get_global(h_, g.data(), THRML_DTYPE_U8, 0);
+    } else {
+      std::vector<float> f(g.size());
+      rc = thrml_state_get_global(h_, f.data(), THRML_DTYPE_F32, 0);
+      for (size_t i = 0; i < g.size(); ++i) g[i] = (T)f[i];
     }
+    if (rc != THRML_OK) return detail::fail<std::vector<T>>(rc);
     return Result<std::vector<T>>::ok(std::move(g));
   }
 

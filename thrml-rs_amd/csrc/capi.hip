@@ -237,6 +237,7 @@ extern "C" int thrml_ctx_set_stream(thrml_ctx *ctx, void *s) {
     THRML_HIP(hipStreamSynchronize(ctx->stream));
     THRML_HIP(hipStreamDestroy(ctx->stream));
   }
+  if (ctx->own_stream || ctx->stream != reinterpret_cast<hipStream_t>(s)) ctx->pool.new_stream();
   ctx->stream = reinterpret_cast<hipStream_t>(s);
   ctx->own_stream = false;
   return THRML_OK;
@@ -594,6 +595,14 @@ bool detect_lattice(thrml_prog *p, uint32_t n_nodes, const std::vector<uint32_t>
   return true;
 }
 
+// The block of every position.
+std::vector<uint32_t> blocks_by_position(const thrml_prog *p) {
+  std::vector<uint32_t> r(p->n_total);
+  for (size_t b = 0; b + 1 < p->blk_off.size(); ++b)
+    std::fill(r.begin() + (long)p->blk_off[b], r.begin() + (long)p->blk_off[b + 1], (uint32_t)b);
+  return r;
+}
+
 // Slot records {tail position, weight} as uploaded, with 16 spare ones: the
 // sweep kernel reads them in batches of 16.
 std::vector<uint32_t> pack_slots(const std::vector<uint32_t> &pos, const std::vector<float> &w) {
@@ -771,9 +780,8 @@ extern "C" int thrml_ising_program_create(thrml_ctx *ctx, const thrml_ising_desc
   std::vector<float> slot_w(ns);
   std::vector<uint32_t> fill(row_off.begin(), row_off.end() - 1);
   bool intra = false;
-  auto blk_of = [&](uint64_t pos) {
-    return (uint32_t)(std::upper_bound(p->blk_off.begin(), p->blk_off.end(), pos) - p->blk_off.begin() - 1);
-  };
+  const std::vector<uint32_t> pos_blk = blocks_by_position(p);
+  auto blk_of = [&](uint64_t pos) { return pos_blk[pos]; };
   for (int pass = 0; pass < 2; ++pass) {
     for (uint64_t e = 0; e < d->n_edges; ++e) {
       const uint32_t head = pass == 0 ? d->edge_u[e] : d->edge_v[e];
@@ -803,7 +811,7 @@ extern "C" int thrml_ising_program_create(thrml_ctx *ctx, const thrml_ising_desc
     const std::vector<uint32_t> slots2 = pack_slots(slot_pos, slot_w);
     if ((rc = upload(p, p->row_off, row_off)) || (rc = upload(p, d_dir, dir)) ||
         (rc = upload(p, d_slots, slots2)) || (rc = upload(p, d_b, bias_w)) ||
-        (rc = p->table.alloc(nf * 16 * sizeof(uint32_t)))) {
+        (rc = p->table.alloc(nf * 16 * sizeof(uint32_t), &ctx->pool))) {
       delete p;
       return rc;
     }
@@ -908,10 +916,8 @@ extern "C" int thrml_potts_program_create(thrml_ctx *ctx, const thrml_potts_desc
     fv[k] = uend[k];
   }
   std::vector<uint32_t> slots(2 * (size_t)row_off[nf]);
-  auto blk_of = [&](uint64_t pos) {
-    return (uint32_t)(std::upper_bound(p->blk_off.begin(), p->blk_off.end(), pos) -
-                      p->blk_off.begin() - 1);
-  };
+  const std::vector<uint32_t> pos_blk = blocks_by_position(p);
+  auto blk_of = [&](uint64_t pos) { return pos_blk[pos]; };
   bool intra = false;
   for (uint64_t e = 0; e < d->n_edges; ++e) {
     const uint32_t pu = (uint32_t)p->node_pos[d->edge_u[e]];
@@ -978,8 +984,8 @@ extern "C" int thrml_potts_program_create(thrml_ctx *ctx, const thrml_potts_desc
   }
   if ((rc = upload(p, p->row_off, row_off)) || (rc = upload(p, p->uend, uend)) ||
       (rc = upload(p, p->slots, slots)) || (rc = upload(p, p->bias_w, bias)) ||
-      (rc = p->wts.alloc((n_w + 2 * ROW_PAD) * sizeof(float))) ||
-      (rc = p->wts_t.alloc((n_w + 2 * ROW_PAD) * sizeof(float))) ||
+      (rc = p->wts.alloc((n_w + 2 * ROW_PAD) * sizeof(float), &ctx->pool)) ||
+      (rc = p->wts_t.alloc((n_w + 2 * ROW_PAD) * sizeof(float), &ctx->pool)) ||
       (p->pm && (rc = upload(p, p->pslots, ps)))) {
     (void)hipStreamSynchronize(ctx->stream);
     delete p;
@@ -1140,9 +1146,8 @@ extern "C" int thrml_discrete_program_create(thrml_ctx *ctx, const thrml_discret
   // slots: a counting pass, then a filling pass
   const uint64_t nf = p->blk_off[p->n_free];
   std::vector<uint32_t> row_off(nf + 1, 0), cursor, slots, sp, last(nf, DISC_NONE);
-  auto blk_of = [&](uint64_t pos) {
-    return (uint32_t)(std::upper_bound(p->blk_off.begin(), p->blk_off.end(), pos) - p->blk_off.begin() - 1);
-  };
+  const std::vector<uint32_t> pos_blk = blocks_by_position(p);
+  auto blk_of = [&](uint64_t pos) { return pos_blk[pos]; };
   bool intra = false;
   for (int pass = 0; pass < 2; ++pass) {
     if (pass == 1) {
@@ -1286,22 +1291,23 @@ extern "C" int thrml_state_create(thrml_prog *p, uint32_t n_chains, thrml_state 
   DevBuf &buf = cat ? st->cat : st->words;
   const size_t bytes = cat ? (size_t)st->Cp * p->n_total * p->cat_bytes
                            : (size_t)st->G * p->planes * p->n_total * sizeof(uint64_t);
-  int rc = buf.alloc(bytes);
+  DevPool *const pool = &p->ctx->pool;
+  int rc = buf.alloc(bytes, pool);
   if (!rc) {
     hipError_t e = hipMemsetAsync(buf.p, 0, bytes, p->ctx->stream);
     if (e != hipSuccess) rc = hip_fail(e, "hipMemsetAsync");
   }
-  if (!rc) rc = st->flag.alloc(sizeof(uint32_t));
+  if (!rc) rc = st->flag.alloc(sizeof(uint32_t), pool);
   // the sweep kernel's half-size gather copy (refreshed at each run's start)
   if (!rc && p->kind == K_CSR && n_chains <= 32u && p->planes == 1u && p->stage_max == 0)
-    rc = st->low.alloc((size_t)p->n_total * sizeof(uint32_t));
+    rc = st->low.alloc((size_t)p->n_total * sizeof(uint32_t), pool);
   if (!rc && p->res_T)
-    rc = st->bits.alloc((size_t)n_chains * ((p->n_total + 63u) / 64u) * sizeof(uint64_t));
+    rc = st->bits.alloc((size_t)n_chains * ((p->n_total + 63u) / 64u) * sizeof(uint64_t), pool);
   if (!rc && p->stage_max) {
     // cleared once: the padding chains of a categorical row are copied back
     // with the staged range but never written
     rc = st->scratch.alloc(cat ? (size_t)st->Cp * p->stage_max * p->cat_bytes
-                               : (size_t)st->G * p->planes * p->stage_max * sizeof(uint64_t));
+                               : (size_t)st->G * p->planes * p->stage_max * sizeof(uint64_t), pool);
     if (!rc) {
       hipError_t e = hipMemsetAsync(st->scratch.p, 0, st->scratch.bytes, p->ctx->stream);
       if (e != hipSuccess) rc = hip_fail(e, "hipMemsetAsync");
@@ -1309,8 +1315,8 @@ extern "C" int thrml_state_create(thrml_prog *p, uint32_t n_chains, thrml_state 
   }
   if (!rc && p->kind == K_DENSE) {
     st->C_pad = (n_chains + 255u) / 256u * 256u;
-    rc = st->dbits_v.alloc((size_t)st->C_pad * (p->Vp / 32) * 4);
-    if (!rc) rc = st->dbits_h.alloc((size_t)st->C_pad * (p->Hp / 32) * 4);
+    rc = st->dbits_v.alloc((size_t)st->C_pad * (p->Vp / 32) * 4, pool);
+    if (!rc) rc = st->dbits_h.alloc((size_t)st->C_pad * (p->Hp / 32) * 4, pool);
     if (!rc) rc = launch_dense_sync_act(st, 0);
     if (!rc) rc = launch_dense_sync_act(st, 1);
   }
@@ -1353,65 +1359,121 @@ struct ObservingScope {
   ObservingScope &operator=(const ObservingScope &) = delete;
 };
 
-static int state_io(thrml_state *st, uint32_t b, void *buf, int dtype, int on_device, bool write) {
-  if (!st || !buf) return fail(THRML_EINVAL, "NULL argument");
+// Device memory for one host transfer: the context's kept staging buffer, or
+// a buffer of its own when that would keep too much.
+struct Staging {
+  std::unique_lock<std::mutex> lk;
+  DevBuf own;
+  void *p = nullptr;
+  int get(thrml_ctx *ctx, size_t bytes) {
+    if (bytes > thrml_ctx::IO_KEEP) {
+      if (int rc = own.alloc(bytes)) return rc;
+      p = own.p;
+      return THRML_OK;
+    }
+    lk = std::unique_lock<std::mutex>(ctx->io_mu);
+    if (ctx->io.bytes < bytes)  // (its last use has ended: every user waits before unlocking)
+      if (int rc = ctx->io.alloc(std::max<size_t>(bytes, 1u << 16))) return rc;
+    p = ctx->io.p;
+    return THRML_OK;
+  }
+};
+
+// Blocks b0 .. b1 - 1 (consecutive positions) from / to rows of their values.
+static int state_io(thrml_state *st, uint32_t b0, uint32_t b1, void *buf, int dtype, int on_device,
+                    bool write) {
   thrml_prog *p = st->prog;
-  if (b >= p->n_free + p->n_clamped) return fail(THRML_EINVAL, "block index out of range");
   if (dtype != THRML_DTYPE_U8 && dtype != THRML_DTYPE_F32) return fail(THRML_EINVAL, "unknown dtype");
   if (!write && dtype == THRML_DTYPE_U8 && p->cat_bytes == 2)
     return fail(THRML_EINVAL, "categories above 255 do not fit the u8 dtype: read this state as f32");
   if (write && tl_observing == p->ctx)
     return fail(THRML_EINVAL, "a state cannot be written inside an observer callback on its context");
   THRML_HIP(hipSetDevice(p->ctx->device));
-  const size_t n = (size_t)st->C * (p->blk_off[b + 1] - p->blk_off[b]);
-  const size_t bytes = n * (dtype == THRML_DTYPE_U8 ? 1 : 4);
+  const uint64_t p0 = p->blk_off[b0];
+  const uint32_t n = (uint32_t)(p->blk_off[b1] - p0);
+  const size_t bytes = (size_t)st->C * n * (dtype == THRML_DTYPE_U8 ? 1 : 4);
+  hipStream_t s = p->ctx->stream;
   void *dev = buf;
-  DevBuf tmp;
+  Staging tmp;
   if (!on_device) {
-    if (int rc = tmp.alloc(bytes)) return rc;
+    if (int rc = tmp.get(p->ctx, bytes)) return rc;
     dev = tmp.p;
-    if (write) THRML_HIP(hipMemcpyAsync(dev, buf, bytes, hipMemcpyHostToDevice, p->ctx->stream));
   }
-  int rc;
-  uint32_t *bad = st->flag.as<uint32_t>();
-  if (write) {
-    // every value is checked before the block is written, so a rejected
-    // import leaves the state as it was
-    const uint32_t q = byte_layout(p) ? block_q(p, b) : 2u;
-    uint32_t bad_h = 0;
-    THRML_HIP(hipMemsetAsync(bad, 0, sizeof(uint32_t), p->ctx->stream));
-    if ((rc = launch_import_check(p->ctx, dev, dtype, n, q, bad))) return rc;
-    THRML_HIP(hipMemcpyAsync(&bad_h, bad, sizeof(uint32_t), hipMemcpyDeviceToHost, p->ctx->stream));
-    THRML_HIP(hipStreamSynchronize(p->ctx->stream));
-    if (bad_h) {
-      if (q > 2 || p->kind == K_POTTS)
-        return fail(THRML_EINVAL, "category value out of range: block " + std::to_string(b) +
-                                      " holds a value outside 0.." + std::to_string(q - 1) +
-                                      " (the state is unchanged)");
-      return fail(THRML_EINVAL, "spin value out of range: block " + std::to_string(b) +
-                                    " holds a value other than 0 and 1 (the state is unchanged)");
+  // nothing of this call is in flight when it returns: the staging buffer and
+  // the caller's memory are free again
+  const int rc = [&]() -> int {
+    if (!write) {
+      if (int r = byte_layout(p) ? launch_potts_unpack(st, p0, n, dev, dtype, n, 0)
+                                 : launch_unpack(st, p0, n, dev, dtype, n, 0))
+        return r;
+      if (!on_device) THRML_HIP(hipMemcpyAsync(buf, dev, bytes, hipMemcpyDeviceToHost, s));
+      return THRML_OK;
     }
+    if (!on_device) THRML_HIP(hipMemcpyAsync(dev, buf, bytes, hipMemcpyHostToDevice, s));
+    // every value is checked before any is written, so a rejected import
+    // leaves the state as it was: the import kernel reads the check's verdict
+    uint32_t *bad = st->flag.as<uint32_t>();
+    if (int r = launch_import_reset(p->ctx, bad)) return r;
+    // blocks with the same values (all of them but in mixed programs) at once
+    for (uint32_t b = b0; b < b1;) {
+      const uint32_t q = byte_layout(p) ? block_q(p, b) : 2u;
+      uint32_t e = b + 1;
+      while (e < b1 && (byte_layout(p) ? block_q(p, e) : 2u) == q) ++e;
+      if (int r = launch_import_check(p->ctx, dev, dtype, st->C, (uint32_t)(p->blk_off[e] - p->blk_off[b]), n,
+                                      p->blk_off[b] - p0, q, bad))
+        return r;
+      b = e;
+    }
+    if (int r = byte_layout(p) ? launch_potts_pack(st, p0, n, dev, dtype, n, 0, bad)
+                               : launch_pack(st, p0, n, dev, dtype, n, 0, bad))
+      return r;
+    if (p->kind == K_DENSE)
+      for (uint32_t b = b0; b < b1; ++b)
+        if (int r = launch_dense_sync_act(st, p->dense_side[b])) return r;
+    uint32_t col = IMPORT_OK;
+    THRML_HIP(hipMemcpyAsync(&col, bad, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    THRML_HIP(hipStreamSynchronize(s));
+    if (col == IMPORT_OK) return THRML_OK;
+    uint32_t b = b0;
+    while (p->blk_off[b + 1] <= p0 + col) ++b;
+    const uint32_t q = byte_layout(p) ? block_q(p, b) : 2u;
+    if (q > 2 || p->kind == K_POTTS)
+      return fail(THRML_EINVAL, "category value out of range: block " + std::to_string(b) +
+                                    " holds a value outside 0.." + std::to_string(q - 1) +
+                                    " (the state is unchanged)");
+    return fail(THRML_EINVAL, "spin value out of range: block " + std::to_string(b) +
+                                  " holds a value other than 0 and 1 (the state is unchanged)");
+  }();
+  if (write || !on_device || rc) {
+    const hipError_t e = hipStreamSynchronize(s);
+    if (!rc && e != hipSuccess) return hip_fail(e, "state transfer");
   }
-  if (byte_layout(p))
-    rc = write ? launch_potts_pack(st, b, dev, dtype, bad) : launch_potts_unpack(st, b, dev, dtype);
-  else
-    rc = write ? launch_pack(st, b, dev, dtype, bad) : launch_unpack(st, b, dev, dtype);
-  if (!rc && write && p->kind == K_DENSE) rc = launch_dense_sync_act(st, p->dense_side[b]);
-  if (rc) return rc;
-  if (!write && !on_device)
-    THRML_HIP(hipMemcpyAsync(buf, dev, bytes, hipMemcpyDeviceToHost, p->ctx->stream));
-  if (write || !on_device) THRML_HIP(hipStreamSynchronize(p->ctx->stream));  // tmp is freed on return
-  return THRML_OK;
+  return rc;
 }
 
 extern "C" int thrml_state_set_block(thrml_state *st, uint32_t b, const void *src, int dtype,
                                      int src_on_device) {
-  return state_io(st, b, const_cast<void *>(src), dtype, src_on_device, true);
+  if (!st || !src) return fail(THRML_EINVAL, "NULL argument");
+  if (b >= st->prog->n_free + st->prog->n_clamped) return fail(THRML_EINVAL, "block index out of range");
+  return state_io(st, b, b + 1, const_cast<void *>(src), dtype, src_on_device, true);
 }
 
 extern "C" int thrml_state_get_block(thrml_state *st, uint32_t b, void *dst, int dtype,
                                      int dst_on_device) {
-  return state_io(st, b, dst, dtype, dst_on_device, false);
+  if (!st || !dst) return fail(THRML_EINVAL, "NULL argument");
+  if (b >= st->prog->n_free + st->prog->n_clamped) return fail(THRML_EINVAL, "block index out of range");
+  return state_io(st, b, b + 1, dst, dtype, dst_on_device, false);
+}
+
+extern "C" int thrml_state_set_global(thrml_state *st, const void *src, int dtype, int src_on_device) {
+  if (!st || !src) return fail(THRML_EINVAL, "NULL argument");
+  return state_io(st, 0, st->prog->n_free + st->prog->n_clamped, const_cast<void *>(src), dtype,
+                  src_on_device, true);
+}
+
+extern "C" int thrml_state_get_global(thrml_state *st, void *dst, int dtype, int dst_on_device) {
+  if (!st || !dst) return fail(THRML_EINVAL, "NULL argument");
+  return state_io(st, 0, st->prog->n_free + st->prog->n_clamped, dst, dtype, dst_on_device, false);
 }
 
 // ---------------------------------------------------------------------------
@@ -1667,22 +1729,30 @@ extern "C" int thrml_moments_create(thrml_prog *p, const uint32_t *nodes, uint64
   m->native = p->kind == K_LATTICE && lattice_pair_slots(p, ppos, pslot);
   m->len1 = m->native ? p->n_total : n1;
   m->len2 = m->native ? (uint64_t)p->L * p->half * 4u : n2;
-  int rc;
-  if (m->native) {
-    if ((rc = upload_to(p->ctx, m->slot1, npos)) || (rc = upload_to(p->ctx, m->slot2, pslot))) {
-      delete m;
-      return rc;
-    }
-  } else if ((rc = upload_to(p->ctx, m->npos, npos)) || (rc = upload_to(p->ctx, m->ppos, ppos))) {
+  // 8-byte parts first: output staging, totals, then counters, then the table
+  const std::vector<uint32_t> &tab2 = m->native ? pslot : ppos;
+  const size_t tab = (npos.size() + tab2.size()) * 4;
+  const size_t wide = (n1 + n2 + m->len1 + m->len2) * 8, cnt = (m->len1 + m->len2) * 4;
+  if (int rc = m->buf.alloc(wide + cnt + tab, &p->ctx->pool)) {
     delete m;
     return rc;
   }
-  if ((rc = m->cnt1.alloc(m->len1 * 4)) || (rc = m->cnt2.alloc(m->len2 * 4)) ||
-      (rc = m->acc1.alloc(m->len1 * 8)) || (rc = m->acc2.alloc(m->len2 * 8))) {
-    delete m;
-    return rc;
-  }
-  hipError_t e = hipStreamSynchronize(p->ctx->stream);  // uploads read host vectors
+  m->out = m->buf.as<int64_t>();
+  m->acc1 = reinterpret_cast<uint64_t *>(m->out + n1 + n2);
+  m->acc2 = m->acc1 + m->len1;
+  m->cnt1 = reinterpret_cast<uint32_t *>(m->acc2 + m->len2);
+  m->cnt2 = m->cnt1 + m->len1;
+  m->clear_bytes = (m->len1 + m->len2) * 12;
+  uint32_t *const t1 = m->cnt2 + m->len2, *const t2 = t1 + npos.size();
+  (m->native ? m->slot1 : m->npos) = t1;
+  (m->native ? m->slot2 : m->ppos) = t2;
+  hipError_t e = hipSuccess;
+  if (!npos.empty())
+    e = hipMemcpyAsync(t1, npos.data(), npos.size() * 4, hipMemcpyHostToDevice, p->ctx->stream);
+  if (e == hipSuccess && !tab2.empty())
+    e = hipMemcpyAsync(t2, tab2.data(), tab2.size() * 4, hipMemcpyHostToDevice, p->ctx->stream);
+  const hipError_t es = hipStreamSynchronize(p->ctx->stream);  // uploads read host vectors
+  if (e == hipSuccess) e = es;
   if (e != hipSuccess) {
     delete m;
     return hip_fail(e, "moment spec upload");
@@ -1709,26 +1779,22 @@ extern "C" int thrml_moments_run(thrml_prog *p, uint64_t key, thrml_schedule sch
   if (int rc = not_observing(p->ctx)) return rc;
   std::lock_guard<std::mutex> lk(p->ctx->run_mu);
   hipStream_t s = p->ctx->stream;
-  THRML_HIP(hipMemsetAsync(m->cnt1.p, 0, m->cnt1.bytes, s));
-  THRML_HIP(hipMemsetAsync(m->cnt2.p, 0, m->cnt2.bytes, s));
-  THRML_HIP(hipMemsetAsync(m->acc1.p, 0, m->acc1.bytes, s));
-  THRML_HIP(hipMemsetAsync(m->acc2.p, 0, m->acc2.bytes, s));
-  uint32_t *c1 = m->cnt1.as<uint32_t>(), *c2 = m->cnt2.as<uint32_t>();
+  if (m->clear_bytes) THRML_HIP(hipMemsetAsync(m->acc1, 0, m->clear_bytes, s));
+  uint32_t *c1 = m->cnt1, *c2 = m->cnt2;
   uint64_t n_obs = 0, since_fold = 0;
   const uint64_t max_before_fold = 0xffffffffull / st->C;  // counters grow <= C per observation
   LatticeMoments lm{c1, c2};
   auto obs = [&](bool fused) -> int {
     if (!fused) {
       const int r = m->native ? launch_lattice_moments(st, &lm)
-                              : launch_moments(st, m->npos.as<uint32_t>(), m->n1,
-                                               m->ppos.as<uint32_t>(), m->n2, c1, c2);
+                              : launch_moments(st, m->npos, m->n1, m->ppos, m->n2, c1, c2);
       if (r) return r;
     }
     ++n_obs;
     if (++since_fold >= max_before_fold) {
       since_fold = 0;
-      if (int r = launch_fold_counts(p->ctx, c1, m->acc1.as<uint64_t>(), m->len1)) return r;
-      return launch_fold_counts(p->ctx, c2, m->acc2.as<uint64_t>(), m->len2);
+      if (int r = launch_fold_counts(p->ctx, c1, m->acc1, m->len1)) return r;
+      return launch_fold_counts(p->ctx, c2, m->acc2, m->len2);
     }
     return THRML_OK;
   };
@@ -1736,17 +1802,9 @@ extern "C" int thrml_moments_run(thrml_prog *p, uint64_t key, thrml_schedule sch
   ks.grow = &p->ctx->keys;
   int rc = run_plan(p, st, schedule_plan(p, st, key, sched), m->native ? &lm : nullptr, obs, ks);
   if (rc) return rc;
-  int64_t *o1 = node_sums, *o2 = pair_sums;
-  if (!out_on_device) {
-    if ((rc = m->out.alloc((m->n1 + m->n2) * 8))) return rc;
-    o1 = m->out.as<int64_t>();
-    o2 = o1 + m->n1;
-  }
+  int64_t *o1 = out_on_device ? node_sums : m->out, *o2 = out_on_device ? pair_sums : m->out + m->n1;
   const int64_t cn = (int64_t)st->C * (int64_t)n_obs;
-  rc = launch_finalize_moments(p->ctx, c1, m->acc1.as<uint64_t>(),
-                               m->native ? m->slot1.as<uint32_t>() : nullptr, m->n1, c2,
-                               m->acc2.as<uint64_t>(), m->native ? m->slot2.as<uint32_t>() : nullptr,
-                               m->n2, cn, o1, o2);
+  rc = launch_finalize_moments(p->ctx, c1, m->acc1, m->slot1, m->n1, c2, m->acc2, m->slot2, m->n2, cn, o1, o2);
   if (rc) return rc;
   if (!out_on_device) {
     if (m->n1) THRML_HIP(hipMemcpyAsync(node_sums, o1, m->n1 * 8, hipMemcpyDeviceToHost, s));
@@ -1801,7 +1859,7 @@ extern "C" int thrml_observer_create(thrml_prog *p, const uint64_t *row_offsets,
   if (off.empty()) off.push_back(0);
   int rc = upload_to(p->ctx, o->row_off, off);
   if (!rc) rc = upload_to(p->ctx, o->pos, pos);
-  if (!rc) rc = o->acc.alloc(std::max<uint64_t>(n_rows, 1) * sizeof(int64_t));
+  if (!rc) rc = o->acc.alloc(std::max<uint64_t>(n_rows, 1) * sizeof(int64_t), &p->ctx->pool);
   if (!rc) {
     hipError_t e = hipStreamSynchronize(p->ctx->stream);
     if (e != hipSuccess) rc = hip_fail(e, "observer upload");
@@ -1896,36 +1954,38 @@ extern "C" int thrml_sample_states_as(thrml_prog *p, uint64_t key, thrml_schedul
     return fail(THRML_EINVAL, "categories above 255 do not fit the u8 dtype: sample this program's "
                               "states as f32");
   THRML_HIP(hipSetDevice(p->ctx->device));
-  const uint32_t nb = p->n_free + p->n_clamped;
-  const size_t esz = dtype == THRML_DTYPE_U8 ? 1 : 4;
-  const size_t per = (size_t)st->C * p->n_total * esz;  // bytes of one observation
-  DevBuf tmp;
-  if (int rc = tmp.alloc(per)) return rc;
-  std::vector<uint8_t> blk;
-  uint64_t k_obs = 0;
-  auto obs = [&](bool) -> int {
-    uint8_t *dst = static_cast<uint8_t *>(out) + k_obs * per;
-    for (uint32_t b = 0; b < nb; ++b) {
-      const size_t n_b = p->blk_off[b + 1] - p->blk_off[b];
-      uint8_t *dblk = tmp.as<uint8_t>() + (size_t)st->C * p->blk_off[b] * esz;
-      const int rc = byte_layout(p) ? launch_potts_unpack(st, b, dblk, dtype)
-                                        : launch_unpack(st, b, dblk, dtype);
-      if (rc) return rc;
-      blk.resize((size_t)st->C * n_b * esz);
-      THRML_HIP(hipMemcpyAsync(blk.data(), dblk, blk.size(), hipMemcpyDeviceToHost, p->ctx->stream));
-      THRML_HIP(hipStreamSynchronize(p->ctx->stream));
-      for (uint32_t c = 0; c < st->C; ++c)
-        std::memcpy(dst + ((size_t)c * p->n_total + p->blk_off[b]) * esz,
-                    blk.data() + (size_t)c * n_b * esz, n_b * esz);
-    }
-    ++k_obs;
-    return THRML_OK;
-  };
   if (int rc = not_observing(p->ctx)) return rc;
   std::lock_guard<std::mutex> lk(p->ctx->run_mu);
+  const size_t per = (size_t)st->C * p->n_total * (dtype == THRML_DTYPE_U8 ? 1 : 4);  // one observation
+  const Plan plan = schedule_plan(p, st, key, sched);
+  // observations are gathered on the device and copied out several at a time,
+  // so that the sweeps are not stopped for each of them
+  const uint64_t batch = std::max<uint64_t>(1, std::min<uint64_t>(plan.obs_after.size(), thrml_ctx::IO_KEEP / per));
+  Staging tmp;
+  if (int rc = tmp.get(p->ctx, batch * per)) return rc;
+  uint8_t *dst = static_cast<uint8_t *>(out);
+  uint64_t held = 0;
+  auto flush = [&]() -> int {
+    if (held) THRML_HIP(hipMemcpyAsync(dst, tmp.p, held * per, hipMemcpyDeviceToHost, p->ctx->stream));
+    dst += held * per;
+    held = 0;
+    return THRML_OK;
+  };
+  auto obs = [&](bool) -> int {
+    void *d = static_cast<uint8_t *>(tmp.p) + held * per;
+    const uint32_t n = (uint32_t)p->n_total;
+    if (int rc = byte_layout(p) ? launch_potts_unpack(st, 0, n, d, dtype, n, 0)
+                                : launch_unpack(st, 0, n, d, dtype, n, 0))
+      return rc;
+    return ++held == batch ? flush() : THRML_OK;
+  };
   KeyStore ks;
   ks.grow = &p->ctx->keys;
-  return run_plan(p, st, schedule_plan(p, st, key, sched), nullptr, obs, ks);
+  int rc = run_plan(p, st, plan, nullptr, obs, ks);
+  if (!rc) rc = flush();
+  const hipError_t e = hipStreamSynchronize(p->ctx->stream);  // before the staging buffer is let go
+  if (!rc && e != hipSuccess) return hip_fail(e, "observation transfer");
+  return rc;
 }
 
 extern "C" int thrml_sample_states(thrml_prog *p, uint64_t key, thrml_schedule sched,
@@ -1951,7 +2011,7 @@ extern "C" int thrml_hinton_init(thrml_prog *p, uint64_t key, thrml_state *st) {
   }
   DevBuf dk, dp;
   int rc;
-  if ((rc = dk.alloc(k8.size() * 4)) || (rc = dp.alloc(prob.size() * 4))) return rc;
+  if ((rc = dk.alloc(k8.size() * 4, &p->ctx->pool)) || (rc = dp.alloc(prob.size() * 4, &p->ctx->pool))) return rc;
   THRML_HIP(hipMemcpyAsync(dk.p, k8.data(), k8.size() * 4, hipMemcpyHostToDevice, p->ctx->stream));
   THRML_HIP(hipMemcpyAsync(dp.p, prob.data(), prob.size() * 4, hipMemcpyHostToDevice, p->ctx->stream));
   for (uint32_t b = 0; b < p->n_free; ++b) {

@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <map>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -51,7 +52,59 @@ struct ResPart {
   uint32_t piece0, piece1, kb;  // pieces [piece0, piece1), keystream blocks
 };
 
-// A device allocation that frees itself.
+// Device memory that the objects of one context have let go of, for its next
+// objects of about the same size: a training step that builds programs,
+// states and moments anew then allocates nothing (a hipMalloc and hipFree pair
+// of more than 2 MiB takes 100-200 us).  All work of a context is ordered on
+// its stream, so a block may be taken again while the last kernels that use it
+// still run.  Bounded by KEEP bytes; emptied with the context and when its
+// stream changes (blocks taken before that are then freed, not kept: their
+// last use may lie on the old stream).
+class DevPool {
+ public:
+  static constexpr size_t KEEP = 256u << 20, LARGEST = 64u << 20;
+  ~DevPool() { clear(); }
+  // a block of at least n bytes and at most twice as many (capacity in *cap), or
+  // null; *era goes back with the block
+  void *take(size_t n, size_t *cap, uint64_t *era) {
+    std::lock_guard<std::mutex> lk(mu_);
+    *era = era_;
+    const auto it = free_.lower_bound(n);
+    if (it == free_.end() || it->first > 2 * n + 4096) return nullptr;
+    void *p = it->second;
+    *cap = it->first;
+    held_ -= it->first;
+    free_.erase(it);
+    return p;
+  }
+  bool give(void *p, size_t cap, uint64_t era) {
+    std::lock_guard<std::mutex> lk(mu_);
+    if (era != era_ || cap > LARGEST || held_ + cap > KEEP) return false;
+    free_.emplace(cap, p);
+    held_ += cap;
+    return true;
+  }
+  void new_stream() {
+    clear();
+    std::lock_guard<std::mutex> lk(mu_);
+    ++era_;
+  }
+  void clear() {
+    std::lock_guard<std::mutex> lk(mu_);
+    for (auto &b : free_) (void)hipFree(b.second);
+    free_.clear();
+    held_ = 0;
+  }
+
+ private:
+  std::mutex mu_;
+  std::multimap<size_t, void *> free_;
+  size_t held_ = 0;
+  uint64_t era_ = 0;
+};
+
+// A device allocation that frees itself, from and back to a context's pool
+// when it is allocated with one.
 struct DevBuf {
   void *p = nullptr;
   size_t bytes = 0;
@@ -60,19 +113,29 @@ struct DevBuf {
   DevBuf &operator=(const DevBuf &) = delete;
   ~DevBuf() { release(); }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p && !(pool_ && pool_->give(p, cap_, era_))) (void)hipFree(p);
     p = nullptr;
-    bytes = 0;
+    pool_ = nullptr;
+    bytes = cap_ = 0;
   }
-  int alloc(size_t n) {
+  int alloc(size_t n, DevPool *pool = nullptr) {
     release();
     if (n == 0) n = 16;
-    hipError_t e = hipMalloc(&p, n);
-    if (e != hipSuccess) {
-      p = nullptr;
-      return fail(THRML_ENOMEM, "device allocation of " + std::to_string(n) + " bytes failed: " +
-                                    hipGetErrorString(e));
+    if (pool) p = pool->take(n, &cap_, &era_);
+    if (!p) {
+      hipError_t e = hipMalloc(&p, n);
+      if (e != hipSuccess && pool) {  // what the pool holds may be what is missing
+        pool->clear();
+        e = hipMalloc(&p, n);
+      }
+      if (e != hipSuccess) {
+        p = nullptr;
+        return fail(THRML_ENOMEM, "device allocation of " + std::to_string(n) + " bytes failed: " +
+                                      hipGetErrorString(e));
+      }
+      cap_ = n;
     }
+    pool_ = pool;
     bytes = n;
     return THRML_OK;
   }
@@ -80,6 +143,11 @@ struct DevBuf {
   T *as() const {
     return reinterpret_cast<T *>(p);
   }
+
+ private:
+  DevPool *pool_ = nullptr;
+  size_t cap_ = 0;
+  uint64_t era_ = 0;
 };
 
 struct TimingSlot {
@@ -107,6 +175,13 @@ struct thrml_ctx {
   // serialises the runs of host threads that share the context.
   thrml::DevBuf keys;
   std::mutex run_mu;
+  thrml::DevPool pool;  // what this context's objects have let go of
+  // Staging of host transfers (state import and export, moment sums), grown as
+  // needed up to IO_KEEP bytes (larger transfers allocate their own).  io_mu is
+  // held from the transfer's first use of it until its stream work has ended.
+  static constexpr size_t IO_KEEP = 64u << 20;
+  thrml::DevBuf io;
+  std::mutex io_mu;
   int flush_timing(int k);
   int time_begin(int k, hipEvent_t *start);
   int time_end(int k, hipEvent_t start, uint64_t half_sweeps = 1);
@@ -224,7 +299,7 @@ struct thrml_state {
   thrml::DevBuf cat;    // categorical programs: [n_total][Cp] u8, chains fastest
   uint32_t Cp = 0;      // C rounded up to 4
   thrml::DevBuf scratch;// per-block staging for programs with intra-block edges / dense operands
-  thrml::DevBuf flag;   // u32: set by the import kernels when a value is out of range
+  thrml::DevBuf flag;   // u32: the first column an import check refuses, or IMPORT_OK
   // CSR spin programs with at most 32 chains and no staged block: [n_total]
   // u32, the low halves of the state words (the high halves are zero).  The
   // sweep kernel gathers neighbour states here, half the footprint of the
@@ -252,11 +327,15 @@ struct thrml_moments {
   bool native = false;
   uint64_t n1 = 0, n2 = 0;      // requested nodes, pairs
   uint64_t len1 = 0, len2 = 0;  // counters
-  thrml::DevBuf slot1, slot2;   // native: counter index per requested entry
-  thrml::DevBuf npos, ppos;     // generic: positions of nodes / pair endpoints
-  thrml::DevBuf cnt1, cnt2;     // u32 counters of the current fold period
-  thrml::DevBuf acc1, acc2;     // u64 totals
-  thrml::DevBuf out;            // int64 staging for host outputs
+  // one allocation: native, the counter index per requested entry (slot1,
+  // slot2), else the positions of nodes and of pair endpoints (npos, ppos);
+  // u32 counters of the current fold period, u64 totals, host-output staging
+  thrml::DevBuf buf;
+  uint32_t *slot1 = nullptr, *slot2 = nullptr, *npos = nullptr, *ppos = nullptr;
+  uint32_t *cnt1 = nullptr, *cnt2 = nullptr;
+  uint64_t *acc1 = nullptr, *acc2 = nullptr;
+  int64_t *out = nullptr;
+  size_t clear_bytes = 0;       // totals and counters, from acc1 on
 };
 
 // A general moment observer (MomentAccumulatorObserver with any spec): row r
@@ -276,7 +355,7 @@ namespace thrml {
 // Allocates buf for v and queues the upload on the context's stream.
 template <class T>
 int upload_to(thrml_ctx *ctx, DevBuf &buf, const std::vector<T> &v) {
-  if (int rc = buf.alloc(v.size() * sizeof(T))) return rc;
+  if (int rc = buf.alloc(v.size() * sizeof(T), &ctx->pool)) return rc;
   if (!v.empty())
     THRML_HIP(hipMemcpyAsync(buf.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice,
                              ctx->stream));
@@ -370,14 +449,19 @@ int launch_dense_half(thrml_prog *p, thrml_state *st, uint32_t side, const uint3
 int launch_lattice_table(thrml_prog *p, const uint32_t *d_dir, const uint2 *d_slots, const float *d_bias);
 int launch_hinton(thrml_prog *p, thrml_state *st, uint32_t b, const uint32_t *d_key8,
                   const float *d_prob);
-// State import of block b from device memory; values out of range (spins
-// other than 0/1, categories outside 0..q-1) are stored as 0 and set *d_bad.
-int launch_potts_pack(thrml_state *st, uint32_t b, const void *d_src, int dtype, uint32_t *d_bad);
-int launch_potts_unpack(thrml_state *st, uint32_t b, void *d_dst, int dtype);
+// State import and export of positions p0 .. p0 + n - 1 from / to device memory
+// that holds one row of `stride` values per chain, at columns col0 .. col0 + n - 1.
+// An import writes nothing unless *d_bad is IMPORT_OK (launch_import_check).
+int launch_potts_pack(thrml_state *st, uint64_t p0, uint32_t n, const void *d_src, int dtype,
+                      uint64_t stride, uint64_t col0, const uint32_t *d_bad);
+int launch_potts_unpack(thrml_state *st, uint64_t p0, uint32_t n, void *d_dst, int dtype, uint64_t stride,
+                        uint64_t col0);
+int launch_pack(thrml_state *st, uint64_t p0, uint32_t n, const void *d_src, int dtype,
+                uint64_t stride, uint64_t col0, const uint32_t *d_bad);
+int launch_unpack(thrml_state *st, uint64_t p0, uint32_t n, void *d_dst, int dtype, uint64_t stride,
+                  uint64_t col0);
 int launch_potts_weights(thrml_ctx *ctx, float *w, float *wt, uint64_t n_edges, uint32_t q,
                          uint64_t n_w);
-int launch_pack(thrml_state *st, uint32_t b, const void *d_src, int dtype, uint32_t *d_bad);
-int launch_unpack(thrml_state *st, uint32_t b, void *d_dst, int dtype);
 int launch_moments(thrml_state *st, const uint32_t *d_npos, uint64_t n1, const uint32_t *d_ppos,
                    uint64_t n2, uint32_t *d_ones, uint32_t *d_diff);
 // Dense programs: recompute side `side`'s spin-down operand bits from the
@@ -399,9 +483,12 @@ int potts_energy(thrml_prog *p, thrml_state *st, double *out);
 int launch_dense_energy(thrml_prog *p, thrml_state *st, double *part);
 int launch_sigmoid_bernoulli(thrml_ctx *ctx, const float *g, const float *u, float *o, uint64_t n);
 int launch_fast_math_check(thrml_ctx *ctx, float out[3]);
-// Raises *d_bad if one of the n values at d_src is not a state value 0..q-1.
-int launch_import_check(thrml_ctx *ctx, const void *d_src, int dtype, uint64_t n, uint32_t q,
-                        uint32_t *d_bad);
+// *d_bad = IMPORT_OK, and lowered to the first column among col0 .. col0 + n - 1
+// that holds something else than a state value 0..q-1 in one of C rows.
+constexpr uint32_t IMPORT_OK = 0xffffffffu;
+int launch_import_reset(thrml_ctx *ctx, uint32_t *d_bad);
+int launch_import_check(thrml_ctx *ctx, const void *d_src, int dtype, uint32_t C, uint32_t n,
+                        uint64_t stride, uint64_t col0, uint32_t q, uint32_t *d_bad);
 // The per-device cached self-check (run at the first call on a device).  With
 // ok_out NULL it fails with THRML_EUNSUPPORTED when the bounds do not hold;
 // otherwise it reports the values and the verdict.

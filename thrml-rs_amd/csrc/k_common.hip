@@ -63,117 +63,187 @@ int launch_key_schedule(thrml_ctx *ctx, const KeyPlan &kp, uint64_t s0, uint32_t
 }
 
 // ---------------------------------------------------------------------------
-// State import: src[c][i] (u8 or f32) of block b -> bit planes.  One wave per
-// (group, 64-site chunk); lane = chain.  A spin must be 0 or 1 (u8), or 0.0 or
-// 1.0 (f32); any other value is stored as 0 and raises *bad.
-__global__ void pack_kernel(const void *__restrict__ src, int dtype, uint32_t C, uint32_t n_b,
-                            uint32_t planes, uint64_t *__restrict__ words, uint64_t plane_stride,
-                            uint64_t blk_off, uint32_t n_chunks, uint32_t G,
-                            uint32_t *__restrict__ bad) {
-  const uint32_t wave = blockIdx.x * 4u + (threadIdx.x >> 6);
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t g = wave / n_chunks, chunk = wave % n_chunks;
-  if (g >= G || (uint64_t)chunk * 64u >= n_b) return;
-  const uint32_t c = g * 64u + lane;
-  const uint32_t i_end = min(n_b, (chunk + 1u) * 64u);
-  for (uint32_t i = chunk * 64u; i < i_end; ++i) {
-    uint32_t v = 0;
-    if (c < C) {
-      const size_t off = (size_t)c * n_b + i;
-      bool ok;
-      if (dtype == THRML_DTYPE_U8) {
-        v = reinterpret_cast<const uint8_t *>(src)[off];
-        ok = v <= 1u;
-      } else {
-        const float x = reinterpret_cast<const float *>(src)[off];
-        ok = x == 0.0f || x == 1.0f;
-        v = x == 1.0f ? 1u : 0u;
-      }
-      if (!ok) {
-        v = 0u;
-        *bad = 1u;
-      }
-    }
-    for (uint32_t pl = 0; pl < planes; ++pl) {
-      const uint64_t m = __builtin_amdgcn_ballot_w64((v >> pl) & 1u);
-      if (lane == 0) words[(size_t)(g * planes + pl) * plane_stride + blk_off + i] = m;
-    }
-  }
-}
+// State import / export: positions p0 .. p0 + n - 1 of every chain, the caller's
+// side one row of `stride` values per chain (u8 or f32) starting at column
+// col0.  Lane = position (IO_PER consecutive ones for u8), so that a row's
+// values and the state words both move in whole cache lines; a lane's 64
+// chain bits of a word are its own, and no bits cross lanes.
+struct StateIo {
+  uint64_t *words;        // first word of position p0, group 0
+  uint64_t plane_stride;
+  uint32_t C, n, n_chunks;
+  uint64_t stride, col0;
+};
+constexpr uint32_t IO_PER = 4;     // positions per lane, u8 rows
+constexpr uint32_t IO_CHAINS = 16; // chains per wave, export
+typedef uint32_t u32_a1 __attribute__((aligned(1)));
 
-__global__ void unpack_kernel(void *__restrict__ dst, int dtype, uint32_t C, uint32_t n_b,
-                              uint32_t planes, const uint64_t *__restrict__ words,
-                              uint64_t plane_stride, uint64_t blk_off, uint32_t n_chunks,
-                              uint32_t G) {
-  const uint32_t wave = blockIdx.x * 4u + (threadIdx.x >> 6);
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t g = wave / n_chunks, chunk = wave % n_chunks;
-  if (g >= G || (uint64_t)chunk * 64u >= n_b) return;
-  const uint32_t c = g * 64u + lane;
-  const uint32_t i_end = min(n_b, (chunk + 1u) * 64u);
-  for (uint32_t i = chunk * 64u; i < i_end; ++i) {
-    uint32_t v = 0;
-    for (uint32_t pl = 0; pl < planes; ++pl) {
-      const uint64_t w = words[(size_t)(g * planes + pl) * plane_stride + blk_off + i];
-      v |= (uint32_t)((w >> lane) & 1u) << pl;
-    }
-    if (c < C) {
-      const size_t off = (size_t)c * n_b + i;
-      if (dtype == THRML_DTYPE_U8)
-        reinterpret_cast<uint8_t *>(dst)[off] = (uint8_t)v;
+// The import is checked before (import_check_kernel): *bad is IMPORT_OK or
+// nothing is written.  A wave takes one chain group.
+template <class V>
+__global__ __launch_bounds__(256) void pack_kernel(const V *__restrict__ src, StateIo a, uint32_t n_tasks,
+                                                   const uint32_t *__restrict__ bad) {
+  constexpr uint32_t PER = sizeof(V) == 1 ? IO_PER : 1u;
+  const uint32_t task = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (task >= n_tasks || *bad != IMPORT_OK) return;
+  const uint32_t g = task / a.n_chunks, chunk = task - g * a.n_chunks;
+  const uint32_t i = (chunk * 64u + (threadIdx.x & 63u)) * PER;
+  if (i >= a.n) return;
+  const uint32_t live = min(a.C - g * 64u, 64u);
+  const V *row = src + (size_t)g * 64u * a.stride + a.col0 + i;
+  uint32_t lo[PER] = {}, hi[PER] = {};
+  const bool whole = i + PER <= a.n;
+#pragma unroll 16
+  for (uint32_t c = 0; c < live; ++c, row += a.stride) {
+    uint32_t v[PER];
+    if constexpr (sizeof(V) == 1) {
+      uint32_t x = 0;
+      if (whole) x = *reinterpret_cast<const u32_a1 *>(row);
       else
-        reinterpret_cast<float *>(dst)[off] = (float)v;
+        for (uint32_t k = 0; i + k < a.n; ++k) x |= (uint32_t)row[k] << (8u * k);
+#pragma unroll
+      for (uint32_t k = 0; k < PER; ++k) v[k] = (x >> (8u * k)) & 1u;
+    } else {
+      v[0] = *row == 1.0f ? 1u : 0u;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < PER; ++k) {
+      if (c < 32u) lo[k] |= v[k] << c;
+      else hi[k] |= v[k] << (c - 32u);
+    }
+  }
+  uint64_t *w = a.words + (size_t)g * a.plane_stride + i;
+#pragma unroll
+  for (uint32_t k = 0; k < PER; ++k)
+    if (i + k < a.n) w[k] = ((uint64_t)hi[k] << 32) | lo[k];
+}
+
+// A wave takes IO_CHAINS chains of one group.
+template <class V>
+__global__ __launch_bounds__(256) void unpack_kernel(V *__restrict__ dst, StateIo a, uint32_t n_tasks) {
+  constexpr uint32_t PER = sizeof(V) == 1 ? IO_PER : 1u;
+  const uint32_t task = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (task >= n_tasks) return;
+  const uint32_t q = task / a.n_chunks, chunk = task - q * a.n_chunks;
+  const uint32_t c0 = q * IO_CHAINS, g = c0 >> 6;
+  const uint32_t i = (chunk * 64u + (threadIdx.x & 63u)) * PER;
+  if (i >= a.n || c0 >= a.C) return;
+  const uint64_t *w = a.words + (size_t)g * a.plane_stride + i;
+  uint32_t b[PER];  // this wave's chains' bits of the lane's positions
+#pragma unroll
+  for (uint32_t k = 0; k < PER; ++k) b[k] = i + k < a.n ? (uint32_t)(w[k] >> (c0 & 63u)) : 0u;
+  V *row = dst + (size_t)c0 * a.stride + a.col0 + i;
+  const bool whole = i + PER <= a.n;
+#pragma unroll
+  for (uint32_t c = 0; c < IO_CHAINS; ++c, row += a.stride) {
+    if (c0 + c >= a.C) break;
+    if constexpr (sizeof(V) == 1) {
+      uint32_t x = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < PER; ++k) x |= ((b[k] >> c) & 1u) << (8u * k);
+      if (whole) *reinterpret_cast<u32_a1 *>(row) = x;
+      else
+        for (uint32_t k = 0; i + k < a.n; ++k) row[k] = (uint8_t)(x >> (8u * k));
+    } else {
+      *row = (b[0] >> c) & 1u ? 1.0f : 0.0f;
     }
   }
 }
 
-// Import check before any write: raises *bad if some value of the caller's
-// block is not a state value (0..q-1 as u8, or the floats 0.0..q-1.0).
-__global__ void import_check_kernel(const void *__restrict__ src, int dtype, uint64_t n,
-                                    uint32_t q, uint32_t *__restrict__ bad) {
+// Import check before any write: *bad becomes the smallest column that holds
+// something else than a state value (0..q-1 as u8, or the floats 0.0..q-1.0),
+// among columns col0 .. col0 + n - 1 of the rows of `stride` values.
+__global__ __launch_bounds__(256) void import_check_kernel(const void *__restrict__ src, int dtype,
+                                                           uint32_t C, uint32_t n, uint64_t stride,
+                                                           uint64_t col0, uint32_t q, uint32_t n_chunks,
+                                                           uint32_t *__restrict__ bad) {
   const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  bool ok;
+  const uint32_t c = (uint32_t)(t / n_chunks), k = (uint32_t)(t - (uint64_t)c * n_chunks);
+  if (c >= C) return;
+  const uint32_t i0 = k * 16u, i1 = min(i0 + 16u, n);
+  const size_t at = (size_t)c * stride + col0;
   if (dtype == THRML_DTYPE_U8) {
-    ok = reinterpret_cast<const uint8_t *>(src)[t] < q;
+    const uint8_t *p = reinterpret_cast<const uint8_t *>(src) + at;
+    if (i0 + 16u <= n && q <= 128u) {
+      // a byte is 128 or more, or its low seven bits plus 128 - q carry into bit 7
+      uint32_t any = 0u;
+#pragma unroll
+      for (uint32_t j = 0; j < 4u; ++j) {
+        const uint32_t x = *reinterpret_cast<const u32_a1 *>(p + i0 + 4u * j);
+        any |= (x | ((x & 0x7f7f7f7fu) + (128u - q) * 0x01010101u)) & 0x80808080u;
+      }
+      if (any == 0u) return;
+    }
+    for (uint32_t i = i0; i < i1; ++i)
+      if (p[i] >= q) {
+        atomicMin(bad, (uint32_t)(col0 + i));
+        return;
+      }
   } else {
-    const float x = reinterpret_cast<const float *>(src)[t];
-    ok = x >= 0.0f && x < (float)q && x == __builtin_floorf(x);
+    const float *p = reinterpret_cast<const float *>(src) + at;
+    for (uint32_t i = i0; i < i1; ++i) {
+      const float x = p[i];
+      if (!(x >= 0.0f && x < (float)q && x == __builtin_floorf(x))) {
+        atomicMin(bad, (uint32_t)(col0 + i));
+        return;
+      }
+    }
   }
-  if (!ok) *bad = 1u;
 }
 
-int launch_import_check(thrml_ctx *ctx, const void *d_src, int dtype, uint64_t n, uint32_t q,
-                        uint32_t *d_bad) {
-  if (n == 0) return THRML_OK;
-  const uint64_t nb = (n + 255) / 256;
+__global__ void import_reset_kernel(uint32_t *bad) { *bad = IMPORT_OK; }
+
+int launch_import_reset(thrml_ctx *ctx, uint32_t *d_bad) {
+  hipLaunchKernelGGL(import_reset_kernel, dim3(1), dim3(1), 0, ctx->stream, d_bad);
+  THRML_HIP(hipGetLastError());
+  return THRML_OK;
+}
+
+int launch_import_check(thrml_ctx *ctx, const void *d_src, int dtype, uint32_t C, uint32_t n,
+                        uint64_t stride, uint64_t col0, uint32_t q, uint32_t *d_bad) {
+  const uint32_t n_chunks = cdiv(n, 16);
+  const uint64_t nb = ((uint64_t)C * n_chunks + 255) / 256;
   if (nb > 0x7fffffffull) return fail(THRML_EUNSUPPORTED, "block too large to import");
   hipLaunchKernelGGL(import_check_kernel, dim3((uint32_t)nb), dim3(256), 0, ctx->stream, d_src,
-                     dtype, n, q, d_bad);
+                     dtype, C, n, stride, col0, q, n_chunks, d_bad);
   THRML_HIP(hipGetLastError());
   return THRML_OK;
 }
 
-int launch_pack(thrml_state *st, uint32_t b, const void *d_src, int dtype, uint32_t *d_bad) {
-  thrml_prog *p = st->prog;
-  const uint32_t n_b = (uint32_t)(p->blk_off[b + 1] - p->blk_off[b]);
-  const uint32_t n_chunks = cdiv(n_b, 64);
-  const uint32_t waves = n_chunks * st->G;
-  hipLaunchKernelGGL(pack_kernel, dim3(cdiv(waves, 4)), dim3(256), 0, p->ctx->stream, d_src, dtype,
-                     st->C, n_b, p->planes, st->words.as<uint64_t>(), (uint64_t)p->n_total,
-                     (uint64_t)p->blk_off[b], n_chunks, st->G, d_bad);
+static StateIo state_io_args(thrml_state *st, uint64_t p0, uint32_t n, uint64_t stride, uint64_t col0,
+                             int dtype) {
+  const uint32_t per = 64u * (dtype == THRML_DTYPE_U8 ? IO_PER : 1u);
+  return StateIo{st->words.as<uint64_t>() + p0, st->prog->n_total, st->C, n, cdiv(n, per), stride, col0};
+}
+
+int launch_pack(thrml_state *st, uint64_t p0, uint32_t n, const void *d_src, int dtype,
+                uint64_t stride, uint64_t col0, const uint32_t *d_bad) {
+  hipStream_t s = st->prog->ctx->stream;
+  const StateIo a = state_io_args(st, p0, n, stride, col0, dtype);
+  const uint64_t tasks = (uint64_t)a.n_chunks * st->G;
+  if (tasks > 0x7fffffffull) return fail(THRML_EUNSUPPORTED, "block too large to import");
+  if (dtype == THRML_DTYPE_U8)
+    hipLaunchKernelGGL(pack_kernel<uint8_t>, dim3(cdiv(tasks, 4)), dim3(256), 0, s,
+                       static_cast<const uint8_t *>(d_src), a, (uint32_t)tasks, d_bad);
+  else
+    hipLaunchKernelGGL(pack_kernel<float>, dim3(cdiv(tasks, 4)), dim3(256), 0, s,
+                       static_cast<const float *>(d_src), a, (uint32_t)tasks, d_bad);
   THRML_HIP(hipGetLastError());
   return THRML_OK;
 }
 
-int launch_unpack(thrml_state *st, uint32_t b, void *d_dst, int dtype) {
-  thrml_prog *p = st->prog;
-  const uint32_t n_b = (uint32_t)(p->blk_off[b + 1] - p->blk_off[b]);
-  const uint32_t n_chunks = cdiv(n_b, 64);
-  const uint32_t waves = n_chunks * st->G;
-  hipLaunchKernelGGL(unpack_kernel, dim3(cdiv(waves, 4)), dim3(256), 0, p->ctx->stream, d_dst,
-                     dtype, st->C, n_b, p->planes, st->words.as<uint64_t>(), (uint64_t)p->n_total,
-                     (uint64_t)p->blk_off[b], n_chunks, st->G);
+int launch_unpack(thrml_state *st, uint64_t p0, uint32_t n, void *d_dst, int dtype, uint64_t stride,
+                  uint64_t col0) {
+  hipStream_t s = st->prog->ctx->stream;
+  const StateIo a = state_io_args(st, p0, n, stride, col0, dtype);
+  const uint64_t tasks = (uint64_t)a.n_chunks * cdiv(st->C, IO_CHAINS);
+  if (tasks > 0x7fffffffull) return fail(THRML_EUNSUPPORTED, "block too large to export");
+  if (dtype == THRML_DTYPE_U8)
+    hipLaunchKernelGGL(unpack_kernel<uint8_t>, dim3(cdiv(tasks, 4)), dim3(256), 0, s,
+                       static_cast<uint8_t *>(d_dst), a, (uint32_t)tasks);
+  else
+    hipLaunchKernelGGL(unpack_kernel<float>, dim3(cdiv(tasks, 4)), dim3(256), 0, s,
+                       static_cast<float *>(d_dst), a, (uint32_t)tasks);
   THRML_HIP(hipGetLastError());
   return THRML_OK;
 }

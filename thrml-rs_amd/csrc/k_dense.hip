@@ -631,7 +631,7 @@ int dense_program_create(thrml_ctx *ctx, const DenseSpec &d, thrml_prog **out) {
   // the fewest bf16 pieces that hold every weight exactly, found on the device
   DevBuf wraw, cnt;
   if (int rc = upload_to(ctx, wraw, d.w)) return rc;
-  if (int rc = cnt.alloc(2 * sizeof(uint32_t))) return rc;
+  if (int rc = cnt.alloc(2 * sizeof(uint32_t), &ctx->pool)) return rc;
   const uint32_t cnt_init[2] = {1u, 0u};
   THRML_HIP(hipMemcpyAsync(cnt.p, cnt_init, sizeof cnt_init, hipMemcpyHostToDevice, ctx->stream));
   const uint64_t n_w = (uint64_t)V * H;
@@ -695,8 +695,8 @@ int dense_program_create(thrml_ctx *ctx, const DenseSpec &d, thrml_prog **out) {
   // piece j of row r at r * (P * Kp) + j * Kp
   const size_t n_lay = (size_t)Vp * Hp * P;
   int rc;
-  if ((rc = p->w_vh.alloc(n_lay * 2)) || (rc = p->w_hv.alloc(n_lay * 2)) ||
-      (rc = p->dense_bias.alloc(bias.size() * 4))) {
+  if ((rc = p->w_vh.alloc(n_lay * 2, &ctx->pool)) || (rc = p->w_hv.alloc(n_lay * 2, &ctx->pool)) ||
+      (rc = p->dense_bias.alloc(bias.size() * 4, &ctx->pool))) {
     delete p;
     return rc;
   }

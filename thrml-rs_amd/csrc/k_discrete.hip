@@ -545,7 +545,7 @@ int discrete_energy(thrml_prog *p, thrml_state *st, double *out) {
   a.Cp = st->Cp;
   a.CG = (st->C + 63u) / 64u;
   DevBuf part;
-  if (int rc = part.alloc((size_t)a.n_ch * a.CG * 64u * sizeof(double))) return rc;
+  if (int rc = part.alloc((size_t)a.n_ch * a.CG * 64u * sizeof(double), &p->ctx->pool)) return rc;
   a.part = part.as<double>();
   const uint64_t waves = (uint64_t)a.n_ch * a.CG;
   hipLaunchKernelGGL(discrete_energy_kernel, dim3(cdiv32(waves, 4)), dim3(256), 0, p->ctx->stream, a);

@@ -212,7 +212,7 @@ static int energy_tables(thrml_prog *p) {
 static int finish_energy(thrml_prog *p, uint32_t C, const double *pe, uint32_t ne, uint32_t se,
                          const double *pb, uint32_t nb, uint32_t sb, double beta, double *out) {
   DevBuf dout;
-  if (int rc = dout.alloc((size_t)C * sizeof(double))) return rc;
+  if (int rc = dout.alloc((size_t)C * sizeof(double), &p->ctx->pool)) return rc;
   hipLaunchKernelGGL(energy_reduce_kernel, dim3(C), dim3(256), 0, p->ctx->stream, pe, ne, se, pb,
                      nb, sb, beta, dout.as<double>());
   THRML_HIP(hipGetLastError());
@@ -249,7 +249,7 @@ int spin_energy(thrml_prog *p, thrml_state *st, double *out) {
   a.n_bch = cdiv32(p->n_total, a.chunk);
   const uint32_t S = st->G * 64u;
   DevBuf part, dpart;
-  if (int rc = part.alloc((size_t)(a.n_ech + a.n_bch) * S * sizeof(double))) return rc;
+  if (int rc = part.alloc((size_t)(a.n_ech + a.n_bch) * S * sizeof(double), &p->ctx->pool)) return rc;
   a.part = part.as<double>();
   const uint64_t waves = (uint64_t)(a.n_ech + a.n_bch) * st->G;
   hipLaunchKernelGGL(spin_energy_kernel, dim3(cdiv32(waves, 4)), dim3(256), 0, p->ctx->stream, a);
@@ -260,7 +260,7 @@ int spin_energy(thrml_prog *p, thrml_state *st, double *out) {
     // keep the visible operand bits in step with the state words, then the
     // coupling term per (32 hidden sites, chain)
     if (int rc = launch_dense_sync_act(st, 0)) return rc;
-    if (int rc = dpart.alloc((size_t)(p->Hp / 32u) * st->C_pad * sizeof(double))) return rc;
+    if (int rc = dpart.alloc((size_t)(p->Hp / 32u) * st->C_pad * sizeof(double), &p->ctx->pool)) return rc;
     if (int rc = launch_dense_energy(p, st, dpart.as<double>())) return rc;
     pe = dpart.as<double>();
     ne = p->Hp / 32u;
@@ -288,7 +288,7 @@ int potts_energy(thrml_prog *p, thrml_state *st, double *out) {
   a.CG = (st->C + 63u) / 64u;
   const uint32_t S = a.CG * 64u;
   DevBuf part;
-  if (int rc = part.alloc((size_t)(a.n_ech + a.n_bch) * S * sizeof(double))) return rc;
+  if (int rc = part.alloc((size_t)(a.n_ech + a.n_bch) * S * sizeof(double), &p->ctx->pool)) return rc;
   a.part = part.as<double>();
   const uint64_t waves = (uint64_t)(a.n_ech + a.n_bch) * a.CG;
   hipLaunchKernelGGL(cat_energy_kernel, dim3(cdiv32(waves, 4)), dim3(256), 0, p->ctx->stream, a);

@@ -557,7 +557,7 @@ int resident_tables(thrml_prog *p, const std::vector<uint32_t> &row_off, const u
   }
   keep.resize(end);
   for (int k = 0; k < 6; ++k) std::memcpy(keep.data() + off[k], tab[k].p, tab[k].n);
-  if (int rc = p->r_tab.alloc(end + at)) return rc;
+  if (int rc = p->r_tab.alloc(end + at, &p->ctx->pool)) return rc;
   uint8_t *const d = p->r_tab.as<uint8_t>();
   THRML_HIP(hipMemcpyAsync(d, keep.data(), end, hipMemcpyHostToDevice, p->ctx->stream));
   const uint32_t n = n_slices * 64u;

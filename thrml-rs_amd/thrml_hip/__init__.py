@@ -531,20 +531,21 @@ class DeviceState:
             check(load().thrml_state_set_block(self._h, int(b), ctypes.c_void_p(t.data_ptr()), dt,
                                                1 if t.is_cuda else 0))
             return
-        a = np.asarray(values)
-        if (a.dtype.kind in "biu" and not self._wide and a.size
+        a, dt = self._host_values(np.asarray(values), n)
+        check(load().thrml_state_set_block(self._h, int(b), a.ctypes.data, dt, 0))
+
+    def _host_values(self, a, n):
+        """(contiguous [n_chains, n] array, dtype code) as the C ABI takes them."""
+        if (a.dtype.kind in "biu" and not self._wide and a.size and a.dtype != np.uint8
                 and (a.min() < 0 or a.max() > 255)) or a.dtype.kind in "fc" or self._wide:
             # floats, values that a byte cannot hold (which the library then
             # rejects instead of a wrapped byte slipping through) and more
             # than 256 categories cross the C ABI as float32 (exact for every
             # integer below 2^24)
-            a = a.astype(np.float32)
-            dt = _lib.DTYPE_F32
+            a, dt = a.astype(np.float32, copy=False), _lib.DTYPE_F32
         else:
-            a = a.astype(np.uint8)
-            dt = _lib.DTYPE_U8
-        a = np.ascontiguousarray(a.reshape(self.n_chains, n))
-        check(load().thrml_state_set_block(self._h, int(b), a.ctypes.data, dt, 0))
+            a, dt = a.astype(np.uint8, copy=False), _lib.DTYPE_U8
+        return np.ascontiguousarray(a.reshape(self.n_chains, n)), dt
 
     @property
     def _wide(self):
@@ -563,18 +564,16 @@ class DeviceState:
 
     def set_global(self, full):
         """full: [n_chains, n_total] in global order (free ++ clamped blocks)."""
-        full = np.asarray(full)
-        for b in range(len(self.program.free_blocks) + len(self.program.clamped_blocks)):
-            off, n = self.program.block_range(b)
-            self.set_block(b, np.ascontiguousarray(full[:, off:off + n]))
+        n = self.program.n_total
+        a, dt = self._host_values(np.asarray(full)[:, :n], n)
+        check(load().thrml_state_set_global(self._h, a.ctypes.data, dt, 0))
 
     def get_global(self):
-        out = np.zeros((self.n_chains, self.program.n_total),
-                       dtype=np.uint16 if self._wide else np.uint8)
-        for b in range(len(self.program.free_blocks) + len(self.program.clamped_blocks)):
-            off, n = self.program.block_range(b)
-            out[:, off:off + n] = self.get_block(b)
-        return out
+        shape = (self.n_chains, self.program.n_total)
+        out = np.empty(shape, dtype=np.float32 if self._wide else np.uint8)
+        check(load().thrml_state_get_global(self._h, out.ctypes.data,
+                                            _lib.DTYPE_F32 if self._wide else _lib.DTYPE_U8, 0))
+        return out.astype(np.uint16) if self._wide else out
 
     def close(self):
         if getattr(self, "_h", None) is not None and self._h.value:
@@ -674,7 +673,7 @@ def sample_states(key, program, schedule, init_state, state_clamp=(), nodes_to_s
                                             f.ctypes.data_as(ctypes.c_void_p), _lib.DTYPE_F32))
         out = f.astype(np.uint16)
     else:
-        out = np.zeros((n_obs, st.n_chains, program.n_total), dtype=np.uint8)
+        out = np.empty((n_obs, st.n_chains, program.n_total), dtype=np.uint8)
         check(load().thrml_sample_states(program._h, key.seed, schedule._c(), st._h,
                                          ptr(out, ctypes.c_uint8)))
     c = st.n_chains

@@ -144,3 +144,30 @@ def test_weight_pieces_found_on_the_device(device):
         w[1, 2] = bad
         with pytest.raises(th.ThrmlError, match="not a sum of three normal bf16 values"):
             th.RbmProgram(w, bv, bh, 1.0, device)
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("V,H,C", [(1, 15, 1), (16, 33, 63), (31, 257, 64), (200, 64, 65), (300, 1100, 130)])
+def test_small_tiles_equal_large_tiles(device, V, H, C, f32):
+    """The kernel for products of few tiles against the one for many: the
+    first C chains of a state large enough for the latter, from the same keys
+    and states, through several half-sweeps (each reads the spin bits that the
+    one before wrote); sites around 16 and 32, chains around 64, K of one and
+    of several ring turns."""
+    log_case(f"dense small tiles V={V} H={H} C={C} f32={f32}")
+    rng = np.random.default_rng(V + H + C)
+    W = rng.normal(0, 0.2, (V, H)).astype(np.float32)
+    W = W if f32 else th.bf16_round(W)[0]
+    bv, bh = rng.normal(0, 0.3, V), rng.normal(0, 0.3, H)
+    prog = th.RbmProgram(W, bv, bh, 0.9, device)
+    big_c = 97 * 256  # more tiles than the small kernel takes, whatever V and H
+    small, big = prog.new_state(C), prog.new_state(big_c)
+    x = rng.integers(0, 2, (big_c, V + H)).astype(np.uint8)
+    small.set_global(x[:C])
+    big.set_global(x)
+    for blk in (1, 0, 1, 0):
+        key8 = rng.integers(0, 2**32, (big_c, 8), dtype=np.uint64).astype(np.uint32)
+        prog.half_sweep(small, blk, key8[:C])
+        prog.half_sweep(big, blk, key8)
+        assert np.array_equal(small.get_global(), big.get_global()[:C]), blk
+    prog.close()

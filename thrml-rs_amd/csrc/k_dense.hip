@@ -461,6 +461,179 @@ __global__ __launch_bounds__(512) void dense_half_kernel(DenseArgs a) {
       (dh[0] << 24) | (dh[1] << 16) | (dl[0] << 8) | dl[1];
 }
 
+// The half-sweep of a product too small to fill the chip with 64 x 256 tiles:
+// 32 sites x 64 chains per workgroup of two waves, so eight times the
+// workgroups.  The large tile's time is then its serial walk over K, about
+// 800 clocks per 64-wide slice with two waves per SIMD in step; here a wave has
+// its SIMD to itself and half the rows, and the ring holds eight slices (seven
+// ahead: 3 loads per wave and slice, and an L2 round trip outlasts several of
+// the short steps).  Each output's two partial sums (k steps 0-1 and 2-3 of
+// every slice) are accumulated in the order of the large tile and added, so
+// the results are the same bits.  Wave gi keeps sites 16 gi .. 16 gi + 15 of the
+// tile: one ChaCha8 block per chain, and bytes 3 - gi and 1 - gi of the chain's word of
+// spin-down bits (dbit_pos: odd sites of a segment above, even ones below).
+// Taken up to DENSE_SMALL_TILES large tiles.  us per half-sweep, averaged over
+// the two sides (large tiles each), large kernel -> this one:
+//   512 x 1024, 256 chains, f32 weights (8, 16)        19.9 -> 11.1
+//   1024 x 4096, 512 chains, bf16 weights (32, 128)    21.5 -> 15.1
+//   1024 x 2048, 1024 chains, bf16 weights (64, 128)   17.0 -> 14.4
+//   1024 x 2048, 2048 chains, bf16 weights (128, 256)  18.2 -> 24.0
+constexpr uint32_t DENSE_SMALL_TILES = 96;
+constexpr int SM = 32, SN = 64, SNS = 8;
+constexpr uint32_t SA_BYTES = SM * TK * 2, SSTAGE = SA_BYTES + SN * 8;
+constexpr uint32_t SMALL_LDS = SNS * SSTAGE;
+constexpr uint32_t SDMA = 3;  // loads per wave and slice: 2 x 16 B + 1 x 4 B per lane
+static_assert(SMALL_LDS >= 2 * 4096, "the partial-sum exchange: 4 KiB per wave");
+static_assert(KPAD == TK * SNS / 2, "the slices come in halves of the ring");
+
+__global__ __launch_bounds__(128) void dense_small_kernel(DenseArgs a) {
+  extern __shared__ __align__(16) uint8_t dlds[];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t gi = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t tile = xcd_remap(blockIdx.x, gridDim.x);
+  const uint32_t tr = fdiv(tile, a.div_nt);
+  const uint32_t m0 = tr * SM, g = tile - tr * a.n_nt;  // first site, chain group
+  f32x16 acc[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[j][r] = 0.0f;
+
+  // DMA sources: weight chunks tid and tid + 128 (row id / 8, column as in the
+  // large tile), spin-bit word tid
+  const uint32_t kw = a.Kp / 32u;
+  const uint32_t r0 = tid >> 3, r1 = r0 + 16u;
+  const uint32_t oA0 = (r0 * a.Ka + ((tid & 7u) ^ swz(r0)) * 8u) * 2u;
+  const uint32_t oA1 = (r1 * a.Ka + ((tid & 7u) ^ swz(r1)) * 8u) * 2u;
+  const uint32_t oD = ((tid >> 1) * kw + (tid & 1u)) * 4u;
+  const uint16_t *bA = a.A + (size_t)m0 * a.Ka;
+  const uint32_t *bD = a.D + (size_t)g * SN * kw;
+  const uint32_t lbase = lds_addr(dlds);
+  const uint32_t n_k = a.Ka / TK;  // a multiple of SNS / 2
+  auto issue = [&](uint32_t slot, uint32_t slice) {
+    const uint32_t sb = lbase + slot * SSTAGE;
+    const uint16_t *sA = bA + (size_t)slice * TK;
+    dma16s(sA, oA0, sb + gi * 1024u);
+    dma16s(sA, oA1, sb + 2048u + gi * 1024u);
+    uint32_t ds = slice >= a.kd ? slice - a.kd : slice;
+    ds = ds >= a.kd ? ds - a.kd : ds;
+    dma4s(bD + (size_t)ds * 2u, oD, sb + SA_BYTES + gi * 256u);
+  };
+  const uint32_t fr = lane & 31u, hf = lane >> 5;
+  const uint32_t cx0 = fr * 128u + ((4u * gi + hf) ^ swz(fr)) * 16u;
+  const uint32_t cx1 = fr * 128u + ((4u * gi + 2u + hf) ^ swz(fr)) * 16u;
+  const uint32_t dA = SA_BYTES + fr * 8u + gi * 4u;
+  const uint32_t hs = hf * 4u;
+  uint32_t sign;
+  asm("v_mov_b32 %0, 0x80008000" : "=v"(sign));
+  const uint32_t one = opaque(0x3F803F80u);
+  struct Frag {
+    uint32_t e, f;
+    bf16x8 a, n;
+  };
+  auto load = [&](Frag &F, auto slot_c) {
+    constexpr uint32_t SLOT = decltype(slot_c)::value;
+    const uint8_t *st = dlds + SLOT * SSTAGE;
+    F.e = *reinterpret_cast<const uint32_t *>(st + dA);
+    F.f = *reinterpret_cast<const uint32_t *>(st + dA + 256u);
+    F.a = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(st + cx0));
+    F.n = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(st + cx1));
+  };
+  // Step s: this wave's reads of slice s have returned and its part of slice
+  // s + 1 has landed (slices s + 2 .. s + 6 in flight); the barrier makes all
+  // of slice s + 1 visible and frees slice s - 1's stage; issue slice s + 7
+  // into it, read slice s + 1, compute slice s.  Slices past the end are
+  // clamped to the last one, so that every step issues the same loads.
+#pragma unroll
+  for (uint32_t k = 0; k < SNS - 1u; ++k) issue(k, min(k, n_k - 1u));
+  wait_vmcnt<(SNS - 2) * SDMA>();
+  __builtin_amdgcn_s_barrier();
+  Frag F0, F1;
+  load(F0, std::integral_constant<uint32_t, 0>{});
+  auto half = [&](uint32_t it, auto first_c) {
+    constexpr uint32_t FIRST = decltype(first_c)::value;
+    static_for<SNS / 2>([&](auto j_c) {
+      constexpr uint32_t j = FIRST + decltype(j_c)::value;
+      Frag &cur = (j & 1u) ? F1 : F0;
+      Frag &nxt = (j & 1u) ? F0 : F1;
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+      wait_vmcnt<(SNS - 3) * SDMA>();
+      __builtin_amdgcn_s_barrier();
+      issue((j + SNS - 1u) % SNS, min(it + decltype(j_c)::value + SNS - 1u, n_k - 1u));
+      load(nxt, std::integral_constant<uint32_t, (j + 1u) % SNS>{});
+      __builtin_amdgcn_sched_barrier(0);
+      cur.e <<= hs;
+      cur.f <<= hs;
+      const bf16x8 e0 = spins_bf16<0>(cur.e, sign, one), f0 = spins_bf16<0>(cur.f, sign, one);
+      acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.a, e0, acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.a, f0, acc[1], 0, 0, 0);
+      const bf16x8 e1 = spins_bf16<8>(cur.e, sign, one), f1 = spins_bf16<8>(cur.f, sign, one);
+      acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.n, e1, acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.n, f1, acc[1], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  for (uint32_t it = 0; it < n_k; it += SNS) {
+    half(it, std::integral_constant<uint32_t, 0>{});
+    if (it + SNS / 2 < n_k) half(it + SNS / 2, std::integral_constant<uint32_t, SNS / 2>{});
+  }
+  wait_vmcnt<0>();
+  __syncthreads();
+  // partial sums of the other wave's 16 sites: accumulator rows 8 (1 - gi) + 0..7
+  {
+    float *mine = reinterpret_cast<float *>(dlds) + gi * 1024u + lane;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 8; ++r) mine[(j * 8 + r) * 64] = gi ? acc[j][r] : acc[j][8 + r];
+  }
+  __syncthreads();
+  float lo[8], hi[8];
+  {
+    const float *other = reinterpret_cast<const float *>(dlds) + (gi ^ 1u) * 1024u + lane;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const float t0 = (gi ? acc[0][8 + r] : acc[0][r]) + other[r * 64];
+      const float t1 = (gi ? acc[1][8 + r] : acc[1][r]) + other[(8 + r) * 64];
+      // lane l: chain l of the group, as in the large tile's epilogue
+      const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, t0),
+                                                       __builtin_bit_cast(uint32_t, t1), false, false);
+      lo[r] = __builtin_bit_cast(float, (uint32_t)sw[0]);
+      hi[r] = __builtin_bit_cast(float, (uint32_t)sw[1]);
+    }
+  }
+  const uint32_t s0 = m0 + gi * 16u;  // this wave's sites
+  if (s0 >= a.M) return;              // (their bits stay up)
+  const uint32_t c = g * 64u + lane;
+  const uint32_t live = a.C - g * 64u;
+  const uint64_t valid = live >= 64u ? ~0ull : ((1ull << live) - 1ull);
+  uint32_t key[KEY_WORDS], x[16];
+  load_keyx(a.keys, c, key);
+  float bias[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) bias[k] = a.bias[s0 + k];
+  chacha_block_pre<8>(key, s0 >> 4, x);
+  uint32_t dh = 0u, dl = 0u, wlo = 0u, whi = 0u;
+  static_for<16>([&](auto k_c) {
+    constexpr int k = decltype(k_c)::value;
+    constexpr int q = k / 8, h = (k / 4) & 1, t = k % 4;
+    const float v = h ? hi[4 * q + t] : lo[4 * q + t];
+    uint64_t up = ~0ull;
+    if (s0 + k < a.M) up = spin_decision_mask(__builtin_fmaf(a.beta, v, bias[k]), x[k]);
+    const uint64_t mk = up & valid;
+    wlo = writelane<k>(wlo, (uint32_t)mk);
+    whi = writelane<k>(whi, (uint32_t)(mk >> 32));
+    if constexpr (k & 1) dh = shift_in(dh, ~up);
+    else dl = shift_in(dl, ~up);
+  });
+  if (lane < 16u && s0 + lane < a.M)
+    a.words[(size_t)g * a.plane_stride + s0 + lane] = ((uint64_t)whi << 32) | wlo;
+  uint8_t *d = reinterpret_cast<uint8_t *>(a.dout + (size_t)c * (a.Mp / 32u) + m0 / 32u);
+  d[3u - gi] = (uint8_t)dh;
+  d[1u - gi] = (uint8_t)dl;
+}
+
 // Spin-down bits of block b for every chain from the state words (bit order
 // dbit_pos); padded positions and chains read as up.
 __global__ void dense_sync_bits_kernel(const uint64_t *__restrict__ words, uint64_t plane_stride,
@@ -526,7 +699,13 @@ int launch_dense_half(thrml_prog *p, thrml_state *st, uint32_t side, const uint3
   const uint32_t n_wg = (a.Mp / TM) * (st->C_pad / TN);
   hipEvent_t t0 = nullptr;
   if (p->ctx->time_begin(0, &t0)) return THRML_EHIP;
-  hipLaunchKernelGGL(dense_half_kernel<false>, dim3(n_wg), dim3(512), DENSE_LDS, p->ctx->stream, a);
+  if (n_wg <= DENSE_SMALL_TILES) {
+    a.n_nt = a.G;
+    a.div_nt = make_fastdiv(a.G);
+    hipLaunchKernelGGL(dense_small_kernel, dim3(cdiv_u(a.M, SM) * a.G), dim3(128), SMALL_LDS, p->ctx->stream, a);
+  } else {
+    hipLaunchKernelGGL(dense_half_kernel<false>, dim3(n_wg), dim3(512), DENSE_LDS, p->ctx->stream, a);
+  }
   THRML_HIP(hipGetLastError());
   return p->ctx->time_end(0, t0);
 }
@@ -577,25 +756,28 @@ __host__ __device__ int bf16_pieces(float w, uint16_t p[3]) {
 }
 
 // The most bf16 pieces any weight needs (out[0], at least 1) and whether a
-// weight has no exact three-piece form (out[1] != 0): one atomic per wave.
-__global__ void dense_pieces_count_kernel(const float *__restrict__ w, uint64_t n,
-                                          uint32_t *__restrict__ out) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// weight has no exact three-piece form (out[1] != 0): one atomic per workgroup
+// of a fixed grid (one per wave made 4M weights take 747 us, all of them on one
+// address).
+__global__ __launch_bounds__(256) void dense_pieces_count_kernel(const float *__restrict__ w, uint64_t n,
+                                                                 uint32_t *__restrict__ out) {
+  __shared__ uint32_t wg[2];
+  if (threadIdx.x == 0u) wg[0] = wg[1] = 0u;
+  __syncthreads();
   uint32_t k = 1u, bad = 0u;
-  if (i < n) {
+  const uint64_t stride = (uint64_t)gridDim.x * 256u;
+  for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < n; i += stride) {
     uint16_t pc[3];
     const int r = bf16_pieces(w[i], pc);
     if (r < 0) bad = 1u;
-    else k = r > 1 ? (uint32_t)r : 1u;
+    else k = max(k, (uint32_t)r);
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    k = max(k, (uint32_t)__shfl_xor((int)k, off));
-    bad |= (uint32_t)__shfl_xor((int)bad, off);
-  }
-  if ((threadIdx.x & 63u) == 0u) {
-    atomicMax(out, k);
-    if (bad) atomicOr(out + 1, 1u);
+  atomicMax(&wg[0], k);
+  if (bad) wg[1] = 1u;
+  __syncthreads();
+  if (threadIdx.x == 0u) {
+    atomicMax(out, wg[0]);
+    if (wg[1]) atomicOr(out + 1, 1u);
   }
 }
 
@@ -636,8 +818,8 @@ int dense_program_create(thrml_ctx *ctx, const DenseSpec &d, thrml_prog **out) {
   THRML_HIP(hipMemcpyAsync(cnt.p, cnt_init, sizeof cnt_init, hipMemcpyHostToDevice, ctx->stream));
   const uint64_t n_w = (uint64_t)V * H;
   if ((n_w + 255) / 256 > 0x7fffffffull) return fail(THRML_EUNSUPPORTED, "too many dense weights");
-  hipLaunchKernelGGL(dense_pieces_count_kernel, dim3((uint32_t)((n_w + 255) / 256)), dim3(256), 0,
-                     ctx->stream, wraw.as<float>(), n_w, cnt.as<uint32_t>());
+  hipLaunchKernelGGL(dense_pieces_count_kernel, dim3((uint32_t)std::min<uint64_t>((n_w + 255) / 256, 512)),
+                     dim3(256), 0, ctx->stream, wraw.as<float>(), n_w, cnt.as<uint32_t>());
   THRML_HIP(hipGetLastError());
   uint32_t cnt_h[2] = {0u, 0u};
   THRML_HIP(hipMemcpyAsync(cnt_h, cnt.p, sizeof cnt_h, hipMemcpyDeviceToHost, ctx->stream));

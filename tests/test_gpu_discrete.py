@@ -332,3 +332,34 @@ def test_constructor_checks_and_state_values(device):
     st.set_block(1, np.array([[0, 2], [1, 1]], np.uint8))
     assert np.array_equal(st.get_block(1), [[0, 2], [1, 1]])
     st.close()
+
+
+@pytest.mark.parametrize("n_spin,C,q", [(1, 1, 3), (3, 70, 3), (15, 4, 2), (16, 64, 3), (17, 65, 4),
+                                        (33, 21, 5), (250, 3, 4), (21, 6, 300)])
+def test_spin_groups_and_tails(device, n_spin, C, q):
+    """Spin blocks around the kernel's 16-site groups and its workgroups of 64
+    (group, chain) pairs: remainders of both, sites without any slot (the last
+    one among them), and slots with no, one, two and three spin tails, alone
+    and beside a categorical tail, bit for bit against the oracle."""
+    rng = np.random.default_rng(n_spin + C)
+    n_far, n_cat = 8, 6
+    n = n_spin + n_far + n_cat
+    S = np.arange(n_spin)
+    F, X = np.arange(n_spin, n_spin + n_far), np.arange(n_spin + n_far, n)
+    kinds = np.r_[np.zeros(n_spin + n_far), np.ones(n_cat)].astype(np.uint8)
+    heads = S[:max(1, n_spin - 1)]  # the last site, and a third of the others, have no slots
+    m = 2 * n_spin
+
+    def rows(k_far, k_cat):
+        far = [rng.choice(F, k_far, replace=False) for _ in range(m)]
+        h = rng.choice(heads[heads % 3 != 1], m)
+        sg = [h] + [np.array([r[i] for r in far]) for i in range(k_far)]
+        cg = [rng.choice(X, m)] * k_cat
+        w = rng.normal(0, 0.6, (m, q if k_cat else 1, 1))
+        return ([g.astype(np.uint32) for g in sg], [g.astype(np.uint32) for g in cg], w.astype(np.float32))
+
+    factors = [rows(k, c) for c in (0, 1) for k in (0, 1, 2, 3)]
+    free = [S, F, X]
+    log_case(f"discrete spin groups n={n_spin} C={C} q={q}")
+    prog, o = _programs(device, n, kinds, q, factors, free)
+    _parity(prog, o, _init(rng, kinds, q, C, free), 43, 3)

@@ -1178,7 +1178,7 @@ extern "C" int thrml_discrete_program_create(thrml_ctx *ctx, const thrml_discret
           // tails: spin groups (minus the head's own for a spin head), then
           // categorical groups (minus the head's for a categorical head);
           // the first categorical tail is the one the conditionals read
-          uint32_t n_sp = 0, cat = DISC_NONE;
+          uint32_t n_sp = 0, cat = DISC_NONE, sp_last = 0;
           const uint32_t sp_beg = (uint32_t)sp.size();
           for (uint32_t k = 0; k < ns + nc; ++k) {
             if (spin_head ? k == hi : k == ns + h) continue;
@@ -1188,6 +1188,7 @@ extern "C" int thrml_discrete_program_create(thrml_ctx *ctx, const thrml_discret
             if (read && blk_of((uint64_t)tp) == blk_of((uint64_t)hp)) intra = true;
             if (k < ns) {
               ++n_sp;
+              sp_last = (uint32_t)tp;
               if (pass == 1) sp.push_back((uint32_t)tp);
             } else if (cat == DISC_NONE) {
               cat = (uint32_t)tp;
@@ -1205,7 +1206,7 @@ extern "C" int thrml_discrete_program_create(thrml_ctx *ctx, const thrml_discret
           uint32_t *r = &slots[4 * (size_t)cursor[hp]++];
           r[0] = (uint32_t)((tr ? df.wt_base : df.w_base) + (uint64_t)b * F.d1 * F.d2);
           r[1] = cat;
-          r[2] = sp_beg;
+          r[2] = n_sp == 1 ? sp_last : sp_beg;  // a single tail's position is in the record
           r[3] = n_sp | first << 8 | axis << 9;
         }
       }

@@ -269,7 +269,8 @@ struct thrml_prog {
   // spin nodes, 1 for categorical nodes.  Per free position (row_off), slots
   // in the reference's order (groups in order, head positions ascending),
   // each a uint4 {weight offset, first categorical tail's position or
-  // DISC_NONE, first spin tail in d_sp, n_sp | group start << 8 | axis << 9};
+  // DISC_NONE, the spin tail's position (n_sp = 1) or the first spin tail in
+  // d_sp, n_sp | group start << 8 | axis << 9};
   // axis 0: entry c of the row, 2: x * q + c (a head-U slot points at the
   // transposed copy of its factor's weights, so every categorical head reads
   // q contiguous floats; axis 1, c * q + x, is not produced).  Energy terms:

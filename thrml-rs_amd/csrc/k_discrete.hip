@@ -12,12 +12,13 @@
 //   theta[c] accumulated alike with +-W'[c] or +-W'[c][x];
 //   x' = first argmax_c(theta[c] + Gumbel), keystream word i * q + c.
 // State: one byte per (position, chain), chains fastest ([n_total][Cp]).
-// Work split: a lane takes one chain and a run of S sites: 4 for spins (a
-// quarter of a keystream block), lcm(q, 16) / q for categories (whole
-// blocks); consecutive lanes are consecutive chains, so a site's slot
-// records are read by all of its chains at once.  Spin sites are summed four
-// at a time with their slots interleaved.  q > 16: discrete_wide_kernel.  The generic path: the
-// benchmarked Ising and categorical programs have their own kernels.
+// Work split: spin blocks, 4 sites of one chain per lane, four waves sharing
+// the keystream blocks of 16 sites (discrete_spin_kernel); categorical blocks,
+// one chain and lcm(q, 16) / q sites per lane (whole keystream blocks), or
+// parts of them (discrete_half_kernel); consecutive lanes are consecutive
+// chains, so a site's slot records are read by all of its chains at once.
+// q > 16: discrete_wide_kernel.  The generic path: the benchmarked Ising and
+// categorical programs have their own kernels.
 #include "dev_util.hpp"
 #include "internal.hpp"
 
@@ -27,7 +28,7 @@ struct DiscArgs {
   const uint8_t *state;     // [n_total][Cp]
   uint8_t *out;             // new values of this block: [n_b][Cp] (in place or staged)
   const uint32_t *row_off;  // [nf + 1]
-  const uint4 *slots;       // {weight offset, categorical tail | DISC_NONE, first spin tail, flags}
+  const uint4 *slots;       // {weight offset, categorical tail | DISC_NONE, spin tail or first index in sp, flags}
   const uint32_t *sp;       // spin tail positions
   const float *W;           // all factors' weights, flat
   const uint32_t *keys;     // [G*64][KEY_WORDS] stream keys of this (sweep, block)
@@ -35,6 +36,21 @@ struct DiscArgs {
   uint32_t items_per_part;  // items of one part of every run (a multiple of 64 with parts)
   FastDiv div_c;            // by C
 };
+
+// Whether the product of slot record r's spin tails is -1 for chain c: an odd
+// number of them is down.  A single tail's position is in the record itself
+// (one dependent load fewer: 23.4 -> 22.3 us per launch of q = 4 categorical
+// sites beside the spins below), several lie in sp from r.z on.
+template <class T>
+__device__ __forceinline__ uint32_t slot_neg(const DiscArgs &a, const T *state, const uint4 &r, uint32_t c) {
+  const uint32_t nsp = r.w & 255u;
+  uint32_t neg = 0u;
+  if (nsp == 1u) neg = state[(size_t)r.z * a.Cp + c] == 0u ? 1u : 0u;
+  else
+    for (uint32_t t = 0; t < nsp; ++t)
+      neg ^= state[(size_t)a.sp[r.z + t] * a.Cp + c] == 0u ? 1u : 0u;
+  return neg;
+}
 
 constexpr int disc_gcd(int a, int b) { return b == 0 ? a : disc_gcd(b, a % b); }
 
@@ -73,12 +89,7 @@ __device__ __forceinline__ void categorical_sites(const DiscArgs &a, uint32_t i_
         float wv[U][Q];
 #pragma unroll
         for (int v = 0; v < U; ++v) {
-          const uint32_t nsp = r[v].w & 255u;
-          uint32_t ng = 0u;
-          if (nsp >= 1u) ng ^= a.state[(size_t)a.sp[r[v].z] * a.Cp + c] == 0u ? 1u : 0u;
-          for (uint32_t t = 1u; t < nsp; ++t)
-            ng ^= a.state[(size_t)a.sp[r[v].z + t] * a.Cp + c] == 0u ? 1u : 0u;
-          neg[v] = ng;
+          neg[v] = slot_neg(a, a.state, r[v], c);
           const uint32_t x = r[v].y != DISC_NONE ? a.state[(size_t)r[v].y * a.Cp + c] : 0u;
           load_row<Q>(a.W + r[v].x + (((r[v].w >> 9) & 3u) == 2u ? x * Q : 0u), wv[v]);
         }
@@ -128,13 +139,7 @@ __device__ __forceinline__ void categorical_sites(const DiscArgs &a, uint32_t i_
       float wv[G][Q];
 #pragma unroll
       for (int u = 0; u < G; ++u) {
-        const uint32_t nsp = r[u].w & 255u;
-        uint32_t ng = 0u;
-        if (nsp >= 1u) ng ^= a.state[(size_t)a.sp[r[u].z] * a.Cp + c] == 0u ? 1u : 0u;
-        if (nsp >= 2u) ng ^= a.state[(size_t)a.sp[r[u].z + 1u] * a.Cp + c] == 0u ? 1u : 0u;
-        for (uint32_t t = 2u; t < nsp; ++t)
-          ng ^= a.state[(size_t)a.sp[r[u].z + t] * a.Cp + c] == 0u ? 1u : 0u;
-        neg[u] = ng;
+        neg[u] = slot_neg(a, a.state, r[u], c);
         const uint32_t x = r[u].y != DISC_NONE ? a.state[(size_t)r[u].y * a.Cp + c] : 0u;
         // the slot's row of q contiguous floats at entry 0 (axis 0) or x * q
         // (axis 2), 16-byte aligned
@@ -183,24 +188,141 @@ __device__ __forceinline__ void categorical_sites(const DiscArgs &a, uint32_t i_
   }
 }
 
-// q = 4 is held to 64 VGPRs, 8 waves per SIMD: it fits them without spilling,
-// and the compiler's own choice, 67, costs a wave and 7 % per launch
-// T: the state's element, uint8_t, or uint16_t in spin blocks of a program
-// whose categorical nodes have more than 256 categories (those blocks run the
-// wide kernel)
-template <int Q, class T = uint8_t>  // Q: 0 spin block, else the categories of a categorical block
+// ChaCha8 block ctr (below 2^32) of a key by four consecutive lanes: lane col
+// holds column col, words col, col + 4, col + 8 and col + 12 (out[0..3]); the
+// diagonal rounds rotate the rows within the four lanes.  A quarter of the
+// instructions and registers of a whole block per lane.
+__device__ __forceinline__ uint32_t quad_rot(uint32_t v, std::integral_constant<int, 1>) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x39, 0xf, 0xf, true);
+}
+__device__ __forceinline__ uint32_t quad_rot(uint32_t v, std::integral_constant<int, 2>) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4e, 0xf, 0xf, true);
+}
+__device__ __forceinline__ uint32_t quad_rot(uint32_t v, std::integral_constant<int, 3>) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x93, 0xf, 0xf, true);
+}
+__device__ __forceinline__ void chacha_quad(uint32_t k0, uint32_t k1, uint32_t ctr, uint32_t col,
+                                            uint32_t (&out)[4]) {
+  using R1 = std::integral_constant<int, 1>;
+  using R2 = std::integral_constant<int, 2>;
+  using R3 = std::integral_constant<int, 3>;
+  const uint32_t a0 = col == 0u ? 0x61707865u : col == 1u ? 0x3320646eu : col == 2u ? 0x79622d32u : 0x6b206574u;
+  const uint32_t d0 = col == 0u ? ctr : 0u;
+  uint32_t a = a0, b = k0, c = k1, d = d0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    THRML_QR(a, b, c, d);
+    b = quad_rot(b, R1{});
+    c = quad_rot(c, R2{});
+    d = quad_rot(d, R3{});
+    THRML_QR(a, b, c, d);
+    b = quad_rot(b, R3{});
+    c = quad_rot(c, R2{});
+    d = quad_rot(d, R1{});
+  }
+  out[0] = a + a0;
+  out[1] = b + k0;
+  out[2] = c + k1;
+  out[3] = d + d0;
+}
+
+// Spin blocks.  A workgroup takes 64 consecutive (16-site group, chain) pairs,
+// lane = pair, wave w sites 4w .. 4w + 3 of the groups: the four waves share
+// the pairs' keystream blocks, each computed by four lanes (chacha_quad),
+// instead of computing every block four times over.  A lane's four sites are
+// summed with their slots interleaved and the next slots' records loaded
+// ahead, so that four chains of dependent loads are in flight; each site sums
+// its own slots in order.  Bound by the latency of the dependent loads (slot
+// record, tail byte, weight).  A layer of 256 x 256 spins coupled to a layer of
+// 4-category nodes, 32 chains, per launch of half the layer: 19.3 us with one
+// lane computing a whole block for its 4 sites, 14.1 us so.
+// T: the state's element, uint8_t, or uint16_t in a program whose categorical
+// nodes have more than 256 categories.
+template <class T>
+__global__ __launch_bounds__(256) void discrete_spin_kernel(DiscArgs a) {
+  __shared__ __align__(16) uint32_t ks[64 * 16];
+  const T *state = reinterpret_cast<const T *>(a.state);
+  const uint32_t tid = threadIdx.x;
+  const uint32_t base = blockIdx.x * 64u;
+  {
+    // (pairs past the end compute the last pair's block, which no one reads)
+    const uint32_t kp = min(base + (tid >> 2), a.n_items - 1u), col = tid & 3u;
+    const uint32_t kg = fdiv(kp, a.div_c), kc = kp - kg * a.C;
+    const uint32_t *k = a.keys + (size_t)kc * KEY_WORDS;
+    uint32_t w[4];
+    chacha_quad(k[col], k[4u + col], kg, col, w);
+#pragma unroll
+    for (uint32_t q = 0; q < 4u; ++q) ks[(tid >> 2) * 16u + 4u * q + col] = w[q];
+  }
+  const uint32_t pair = base + (tid & 63u), wave = tid >> 6;
+  const bool live = pair < a.n_items;
+  const uint32_t pc = live ? pair : 0u;
+  const uint32_t g = fdiv(pc, a.div_c), c = pc - g * a.C;
+  const uint32_t i_begin = g * 16u + wave * 4u;
+  uint32_t k0[4], deg[4], mx = 0u;
+  float tot[4], acc[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const uint32_t i = i_begin + (uint32_t)u;
+    const uint32_t pos = a.blk_off + min(i, a.n_b - 1u);
+    k0[u] = a.row_off[pos];
+    deg[u] = live && i < a.n_b ? a.row_off[pos + 1] - k0[u] : 0u;
+    mx = max(mx, deg[u]);
+    tot[u] = acc[u] = 0.0f;
+  }
+  uint4 r[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) r[u] = a.slots[k0[u]];
+  for (uint32_t j = 0; j < mx; ++j) {
+    float v[4];
+    uint4 nr[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) nr[u] = a.slots[k0[u] + min(j + 1u, deg[u] ? deg[u] - 1u : 0u)];
+    uint32_t neg[4], x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      neg[u] = slot_neg(a, state, r[u], c);
+      x[u] = r[u].y != DISC_NONE ? state[(size_t)r[u].y * a.Cp + c] : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float w = a.W[r[u].x + x[u]];
+      v[u] = neg[u] ? -w : w;  // w * (+-1) is exactly +-w
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (j < deg[u]) {
+        const bool first = (r[u].w >> 8) & 1u;
+        if (first && j != 0u) tot[u] = tot[u] + acc[u];
+        acc[u] = first ? v[u] : acc[u] + v[u];
+      }
+      r[u] = nr[u];
+    }
+  }
+  __syncthreads();
+  const uint4 wd = *reinterpret_cast<const uint4 *>(ks + (tid & 63u) * 16u + wave * 4u);
+  const uint32_t word[4] = {wd.x, wd.y, wd.z, wd.w};
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const uint32_t i = i_begin + (uint32_t)u;
+    if (deg[u]) tot[u] = tot[u] + acc[u];
+    if (live && i < a.n_b)
+      reinterpret_cast<T *>(a.out)[(size_t)i * a.Cp + c] = spin_decision(tot[u], word[u]) ? 1u : 0u;
+  }
+}
+
+// Categorical blocks of Q <= 16 categories.  q = 4 is held to 64 VGPRs, 8
+// waves per SIMD: it fits them without spilling, and the compiler's own
+// choice, 67, costs a wave and 7 % per launch
+template <int Q>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Q == 4 ? 8 : 1)))
 void discrete_half_kernel(DiscArgs a) {
-  static_assert(Q == 0 || sizeof(T) == 1, "categorical blocks of Q <= 16 hold one byte per node");
-  const T *state = reinterpret_cast<const T *>(a.state);
-  // sites per run: spin blocks 4, a quarter of a keystream block (more waves:
-  // the sums are latency-bound, and 4-site runs measured 25 % faster than
-  // 16-site ones on a 512^2 lattice); categorical blocks lcm(Q, 16) / Q,
-  // whole blocks, split into NP parts of 4 sites when that is 8 or 16 (each
-  // part a lane, its keystream offset fixed at compile time, one part per
-  // wave: items [p * items_per_part, (p + 1) * items_per_part) are part p)
-  constexpr int SG = Q == 0 ? 4 : 16 / disc_gcd(Q, 16);
-  constexpr int NP = Q != 0 && SG > 4 ? SG / 4 : 1;
+  // sites per run: lcm(Q, 16) / Q, whole keystream blocks, split into NP parts
+  // of 4 sites when that is 8 or 16 (each part a lane, its keystream offset
+  // fixed at compile time, one part per wave: items [p * items_per_part,
+  // (p + 1) * items_per_part) are part p)
+  constexpr int SG = 16 / disc_gcd(Q, 16);
+  constexpr int NP = SG > 4 ? SG / 4 : 1;
   constexpr int S = SG / NP;
   const uint32_t item = blockIdx.x * blockDim.x + threadIdx.x;
   if (item >= a.n_items) return;
@@ -214,62 +336,7 @@ void discrete_half_kernel(DiscArgs a) {
   load_key8(a.keys, c, key);
   uint32_t blk[16];
   int have = -1;
-  if constexpr (Q == 0) {
-    const uint32_t i_begin = run * S;
-    const uint64_t ctr0 = i_begin / 16u;
-    chacha_block<8>(key, ctr0, blk);  // the block holding the run's 4 words
-    // spin sites four at a time: slot j of the four sites is read together,
-    // so that four chains of dependent loads (record, tail position, tail
-    // byte, weight) are in flight; each site still sums its slots in order
-    static_assert(S == 4, "a spin run is one quarter of a keystream block");
-#pragma unroll
-    for (int g = 0; g < S; g += 4) {
-      uint32_t k0[4], deg[4], mx = 0u;
-      float tot[4], acc[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const uint32_t i = i_begin + (uint32_t)(g + u);
-        const uint32_t pos = a.blk_off + min(i, a.n_b - 1u);
-        k0[u] = a.row_off[pos];
-        deg[u] = i < a.n_b ? a.row_off[pos + 1] - k0[u] : 0u;
-        mx = max(mx, deg[u]);
-        tot[u] = acc[u] = 0.0f;
-      }
-      for (uint32_t j = 0; j < mx; ++j) {
-        uint4 r[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) r[u] = a.slots[k0[u] + min(j, deg[u] ? deg[u] - 1u : 0u)];
-        float v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const uint32_t nsp = r[u].w & 255u;
-          uint32_t neg = 0u;
-          if (nsp >= 1u) neg ^= state[(size_t)a.sp[r[u].z] * a.Cp + c] == 0u ? 1u : 0u;
-          if (nsp >= 2u) neg ^= state[(size_t)a.sp[r[u].z + 1u] * a.Cp + c] == 0u ? 1u : 0u;
-          for (uint32_t t = 2u; t < nsp; ++t)
-            neg ^= state[(size_t)a.sp[r[u].z + t] * a.Cp + c] == 0u ? 1u : 0u;
-          const uint32_t x = r[u].y != DISC_NONE ? state[(size_t)r[u].y * a.Cp + c] : 0u;
-          const float w = a.W[r[u].x + x];
-          v[u] = neg ? -w : w;  // w * (+-1) is exactly +-w
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          if (j < deg[u]) {
-            const bool first = (r[u].w >> 8) & 1u;
-            if (first && j != 0u) tot[u] = tot[u] + acc[u];
-            acc[u] = first ? v[u] : acc[u] + v[u];
-          }
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const uint32_t i = i_begin + (uint32_t)(g + u);
-        if (deg[u]) tot[u] = tot[u] + acc[u];
-        if (i < a.n_b)
-          reinterpret_cast<T *>(a.out)[(size_t)i * a.Cp + c] = spin_decision(tot[u], blk[i & 15u]) ? 1u : 0u;
-      }
-    }
-  } else {
+  {
     const uint64_t ctr_run = (uint64_t)run * SG * Q / 16u;
     if constexpr (NP == 1) {
       categorical_sites<Q, S, 0>(a, run * SG, c, key, ctr_run, blk, have);
@@ -309,10 +376,7 @@ __global__ __launch_bounds__(256) void discrete_wide_kernel(DiscArgs a, uint32_t
   // slot record r: its row's offset in W, and its sign (bit 0) and group-start
   // (bit 1) flags
   auto slot = [&](const uint4 &r, uint32_t &off, uint32_t &fl) {
-    const uint32_t nsp = r.w & 255u;
-    uint32_t neg = 0u;
-    for (uint32_t t = 0; t < nsp; ++t)
-      neg ^= state[(size_t)a.sp[r.z + t] * a.Cp + c] == 0u ? 1u : 0u;
+    const uint32_t neg = slot_neg(a, state, r, c);
     const uint32_t x = r.y != DISC_NONE ? state[(size_t)r.y * a.Cp + c] : 0u;
     off = r.x + (((r.w >> 9) & 3u) == 2u ? x * Q : 0u);
     fl = neg | (((r.w >> 8) & 1u) << 1);
@@ -392,9 +456,9 @@ __global__ __launch_bounds__(256) void discrete_wide_kernel(DiscArgs a, uint32_t
 
 static inline uint32_t cdiv32(uint64_t x, uint64_t y) { return (uint32_t)((x + y - 1) / y); }
 
-template <int Q, class T = uint8_t>
+template <int Q>
 static void launch_dq(const DiscArgs &a, hipStream_t s) {
-  hipLaunchKernelGGL((discrete_half_kernel<Q, T>), dim3(cdiv32(a.n_items, 256)), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(discrete_half_kernel<Q>, dim3(cdiv32(a.n_items, 256)), dim3(256), 0, s, a);
 }
 
 template <class T, int P>
@@ -421,7 +485,7 @@ int launch_discrete_half(thrml_prog *p, thrml_state *st, uint32_t b, const uint3
   const uint32_t Q = spin ? 0u : p->q;
   const bool wide = Q > 16u;  // one site per lane
   // sites per run and parts per run, as in the kernel
-  const uint32_t SG = wide ? 1u : spin ? 4u : 16u / (uint32_t)disc_gcd((int)Q, 16);
+  const uint32_t SG = wide ? 1u : spin ? 16u : 16u / (uint32_t)disc_gcd((int)Q, 16);
   const uint32_t NP = !spin && SG > 4u ? SG / 4u : 1u;
   DiscArgs a;
   a.state = st->cat.as<uint8_t>();
@@ -446,7 +510,8 @@ int launch_discrete_half(thrml_prog *p, thrml_state *st, uint32_t b, const uint3
   // (parts start on a wave boundary, so that a wave holds one part)
   const uint64_t runs = (uint64_t)cdiv32(n_b, SG) * st->C;
   const uint64_t per = NP > 1 ? (runs + 63u) & ~63ull : runs;
-  if (per * NP >= (1ull << 31))
+  // (a spin run takes four lanes: the launch itself stays below 2^32 threads)
+  if (per * (spin ? 4u : NP) >= (1ull << 31))
     return fail(THRML_EINVAL, "block too large: (sites / runs) x chains must stay below 2^31");
   a.items_per_part = (uint32_t)per;
   a.n_items = (uint32_t)(per * NP);
@@ -454,10 +519,12 @@ int launch_discrete_half(thrml_prog *p, thrml_state *st, uint32_t b, const uint3
   if (p->ctx->time_begin(0, &t0)) return THRML_EHIP;
   hipStream_t s = p->ctx->stream;
   switch (Q) {
-    case 0:
-      if (p->cat_bytes == 2) launch_dq<0, uint16_t>(a, s);
-      else launch_dq<0>(a, s);
+    case 0: {
+      const dim3 grid(cdiv32(a.n_items, 64));  // (16-site group, chain) pairs
+      if (p->cat_bytes == 2) hipLaunchKernelGGL(discrete_spin_kernel<uint16_t>, grid, dim3(256), 0, s, a);
+      else hipLaunchKernelGGL(discrete_spin_kernel<uint8_t>, grid, dim3(256), 0, s, a);
       break;
+    }
     case 2: launch_dq<2>(a, s); break;
     case 3: launch_dq<3>(a, s); break;
     case 4: launch_dq<4>(a, s); break;

@@ -369,3 +369,74 @@ def test_sample_states_u8_refuses_more_than_256_categories(device):
     rc, _ = _sample_states_as(prog, st, 1, sched, 7)
     assert rc == _lib.THRML_EINVAL
     st.close()
+
+
+@pytest.mark.parametrize("C,n_pairs", [(1, 7), (64, 70), (129, 70), (700, 70), (2100, 3),
+                                       (2, (1 << 20) + 5), (70, (1 << 20) - 3)])
+def test_moment_sums_over_splits(device, C, n_pairs):
+    """Moment sums with one to 32 threads per item (1 to 33 chain groups) and,
+    from 2^20 items on, four items per thread: odd chain counts and remainders
+    of items, the nodes' end inside a turn of the pairs."""
+    ebm, blocks = wl.lattice_ising(20, 0.2, 0.3, 0.1)
+    prog = th.IsingSamplingProgram(ebm, blocks, [], device)
+    o = orc.Ising(ebm.n_nodes, ebm.edges, ebm.biases, ebm.weights, ebm.beta,
+                  [np.asarray(b.nodes if hasattr(b, "nodes") else b) for b in blocks])
+    rng = np.random.default_rng(C)
+    nodes = rng.permutation(ebm.n_nodes)[:133].astype(np.uint32)
+    pairs = rng.integers(0, ebm.n_nodes, (n_pairs, 2)).astype(np.uint32)
+    init = rng.integers(0, 2, (C, ebm.n_nodes)).astype(np.uint8)
+    log_case(f"moment sums C={C} pairs={n_pairs}")
+    st = prog.new_state(C)
+    st.set_global(init)
+    ns, es = th.estimate_moments(th.RngKey(9), nodes, pairs, prog, th.SamplingSchedule(1, 2, 1), st,
+                                 return_sums=True)
+    st.close()
+    t = 2 * o.sample_states(9, (1, 2, 1), init).astype(np.int64) - 1
+    t = t[:, :, [o.pos(i) for i in range(ebm.n_nodes)]]
+    corr = np.einsum("scn,scm->nm", t, t)
+    assert np.array_equal(ns, t.sum(axis=(0, 1))[nodes])
+    assert np.array_equal(es, corr[pairs[:, 0], pairs[:, 1]])
+
+
+@pytest.mark.parametrize("transform", [True, False])
+@pytest.mark.parametrize("q,C", [(2, 1), (3, 4), (5, 17), (4, 64), (7, 259), (300, 6), (300, 130)])
+def test_observer_lanes_per_row(device, q, C, transform):
+    """Rows of 0 to 5 nodes with 1 to 64 lanes per row, one and two bytes of
+    state, chain counts that leave a part of the last four chains unused."""
+    n, edges, W, bias, blocks = wl.potts_lattice(6, q, 0.3, 0.2)
+    prog = th.CategoricalProgram(n, q, edges, W, bias, blocks, device)
+    o = orc.Potts(n, q, edges, W, bias, [np.asarray(b.nodes if hasattr(b, "nodes") else b)
+                                         for b in blocks])
+    rng = np.random.default_rng(q + C)
+    spec = _rows(rng, np.arange(n), 4) + [[[int(x) for x in rng.choice(n, 5)] for _ in range(67)]]
+    init = rng.integers(0, q, (C, n)).astype(np.uint8 if q <= 256 else np.uint16)
+    log_case(f"observer lanes per row q={q} C={C} transform={transform}")
+    got = _check(prog, spec, transform, 5, (1, 2, 1), init)
+    want = _expected(o.sample_states(5, (1, 2, 1), init), _positions(o, spec), transform)
+    for g, w in zip(got, want):
+        assert np.array_equal(g, w)
+
+
+@pytest.mark.parametrize("C", [1, 20, 32])
+def test_moment_sums_from_the_low_halves(device, C):
+    """At most 32 chains on a graph above the size of whole runs in one launch:
+    the sums are read from the copy of the words' low halves, after a first
+    observation before any sweep from the words themselves."""
+    ebm, blocks = wl.er_ising(70_001, 3.0, 0.2, 0.0, 0.3)
+    prog = th.IsingSamplingProgram(ebm, blocks, [], device)
+    assert prog.kind == "csr"
+    o = orc.Ising(ebm.n_nodes, ebm.edges, ebm.biases, ebm.weights, ebm.beta,
+                  [np.asarray(b.nodes if hasattr(b, "nodes") else b) for b in blocks])
+    init = np.random.default_rng(C).integers(0, 2, (C, ebm.n_nodes)).astype(np.uint8)
+    st = prog.new_state(C)
+    pos = np.array([o.pos(i) for i in range(ebm.n_nodes)])
+    for sched in ((0, 2, 1), (2, 1, 1)):
+        log_case(f"moment sums from low halves C={C} {sched}")
+        st.set_global(init)
+        ns, es = th.estimate_moments(th.RngKey(3), np.arange(ebm.n_nodes), ebm.edges, prog,
+                                     th.SamplingSchedule(*sched), st, return_sums=True)
+        t = 2 * o.sample_states(3, sched, init).astype(np.int64)[:, :, pos] - 1
+        e = ebm.edges
+        assert np.array_equal(ns, t.sum(axis=(0, 1)))
+        assert np.array_equal(es, (t[:, :, e[:, 0]] * t[:, :, e[:, 1]]).sum(axis=(0, 1)))
+    st.close()

@@ -1549,20 +1549,20 @@ int run_plan(thrml_prog *p, thrml_state *st, const Plan &pl, const LatticeMoment
   const bool can_fuse = fuse && p->kind == K_LATTICE;
   size_t oi = 0;
   const size_t n_obs = pl.obs_after.size();
+  st->low_live = false;
   while (oi < n_obs && pl.obs_after[oi] < 0) {
     if (int rc = obs(false)) return rc;
     ++oi;
   }
-  // the words may have changed since the last run (state writes, hinton_init);
-  // the sweeps keep the copy in step from here on
   // the observations left cut the run into segments
   const uint64_t n_seg = std::max<uint64_t>(n_obs - oi, 1);
-  bool resident = resident_pays(p, st, pl.n_sweeps, n_seg, can_fuse);
-#ifdef RES_FORCE
-  resident = p->res_T && RES_FORCE;
-#endif
-  if (pl.n_sweeps && st->low.p && !resident)
+  const bool resident = resident_pays(p, st, pl.n_sweeps, n_seg, can_fuse);
+  // the words may have changed since the last run (state writes, hinton_init);
+  // the sweeps keep the low halves' copy in step from here on
+  if (pl.n_sweeps && st->low.p && !resident) {
     if (int rc = launch_pack_low(st)) return rc;
+    st->low_live = true;
+  }
   for (uint64_t s0 = 0; s0 < pl.n_sweeps; s0 += chunk) {
     const uint32_t ns = (uint32_t)std::min<uint64_t>(chunk, pl.n_sweeps - s0);
     const uint64_t need = ns * per_sweep;

@@ -305,7 +305,9 @@ struct thrml_state {
   // u32, the low halves of the state words (the high halves are zero).  The
   // sweep kernel gathers neighbour states here, half the footprint of the
   // words, and writes both; each run refreshes it from the words first.
+  // low_live: it holds the current spins (set within a run that keeps it).
   thrml::DevBuf low;
+  bool low_live = false;
   // resident runs: [C][ceil(n_total / 64)] u64, the chains' spins at a run's end
   thrml::DevBuf bits;
   // dense path operands: spin-down bits per block, one bit vector per chain

@@ -254,33 +254,51 @@ int launch_unpack(thrml_state *st, uint64_t p0, uint32_t n, void *d_dst, int dty
 //   ones[k] += #chains with s = 1 at node k,
 //   diff[k] += #chains with s_a != s_b for pair k,
 // so that sum_c t = 2*ones - C*n_obs and sum_c t_a t_b = C*n_obs - 2*diff.
-__global__ void moments_kernel(const uint64_t *__restrict__ words, uint64_t plane_stride,
-                               uint32_t G, uint32_t C, const uint32_t *__restrict__ npos,
-                               uint64_t n1, const uint32_t *__restrict__ ppos, uint64_t n2,
-                               uint32_t *__restrict__ ones, uint32_t *__restrict__ diff) {
-  const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (tid < n1) {
-    const uint32_t pos = npos[tid];
-    uint32_t s = 0;
-    for (uint32_t g = 0; g < G; ++g) {
-      uint64_t w = words[(size_t)g * plane_stride + pos];
-      const uint32_t rem = C - g * 64u;
-      if (rem < 64u) w &= (1ull << rem) - 1ull;
-      s += (uint32_t)__builtin_popcountll(w);
-    }
-    ones[tid] += s;
-  } else if (tid < n1 + n2) {
-    const uint64_t k = tid - n1;
-    const uint32_t pa = ppos[2 * k], pb = ppos[2 * k + 1];
-    uint32_t s = 0;
-    for (uint32_t g = 0; g < G; ++g) {
-      uint64_t w = words[(size_t)g * plane_stride + pa] ^ words[(size_t)g * plane_stride + pb];
-      const uint32_t rem = C - g * 64u;
-      if (rem < 64u) w &= (1ull << rem) - 1ull;
-      s += (uint32_t)__builtin_popcountll(w);
-    }
-    diff[k] += s;
+// Bound by the random reads of a pair's words.  A workgroup takes 256 >> lg
+// items (nodes, then pairs), 1 << lg threads per item, thread `slice` of an item
+// the chain groups slice, slice + (1 << lg), ..., summed through LDS: with few
+// items a thread alone has too few of its loads in flight (5,120 nodes and
+// their pairs, 4,096 chains: 19.1 us per observation with one thread per item,
+// 5.0 us with 32), and above MOMENTS_FILL threads, 16 waves per compute unit,
+// the items fill the chip by themselves.
+constexpr uint32_t MOMENTS_MAX_LG = 5;
+constexpr uint64_t MOMENTS_FILL = 1u << 18;
+
+// W: uint64_t, or uint32_t where one chain group has at most 32 chains and the
+// state keeps a copy of its words' low halves (half the bytes to gather: a
+// million nodes and their 6 million pairs 57.9 -> 41.3 us).
+template <class W>
+__global__ __launch_bounds__(256) void moments_kernel(
+    const W *__restrict__ words, uint64_t plane_stride, uint32_t G, uint32_t C,
+    const uint32_t *__restrict__ npos, uint64_t n1, const uint32_t *__restrict__ ppos, uint64_t n2,
+    uint32_t *__restrict__ ones, uint32_t *__restrict__ diff, uint32_t lg) {
+  __shared__ uint32_t part[256];
+  const uint32_t per = 256u >> lg;
+  const uint32_t slice = threadIdx.x >> (8u - lg);
+  const uint64_t i = (uint64_t)blockIdx.x * per + (threadIdx.x & (per - 1u));
+  // (threads past the last item take the last and store nothing)
+  const uint64_t k = i < n1 + n2 ? i : n1 + n2 - 1u;
+  const bool node = k < n1;
+  const uint32_t *at = node ? npos + k : ppos + 2u * (k - n1);
+  const uint32_t pa = at[0], pb = at[node ? 0 : 1];
+  const W two = node ? (W)0 : (W)~(W)0;  // a node's second word counts as 0
+  uint32_t *cnt = node ? ones + k : diff + (k - n1);
+  const uint32_t old = *cnt;
+  uint32_t sum = 0u;
+#pragma unroll 4
+  for (uint32_t g = slice; g < G; g += 1u << lg) {
+    const W *w = words + (size_t)g * plane_stride;
+    const uint32_t rem = C - g * 64u;
+    const uint64_t valid = rem < 64u ? (1ull << rem) - 1ull : ~0ull;
+    sum += (uint32_t)__builtin_popcountll((uint64_t)(w[pa] ^ (w[pb] & two)) & valid);
   }
+  if (lg != 0u) {
+    part[threadIdx.x] = sum;
+    __syncthreads();
+    if (slice != 0u) return;
+    for (uint32_t t = 1; t < 1u << lg; ++t) sum += part[t * per + threadIdx.x];
+  }
+  if (i < n1 + n2) *cnt = old + sum;
 }
 
 int launch_moments(thrml_state *st, const uint32_t *d_npos, uint64_t n1, const uint32_t *d_ppos,
@@ -290,9 +308,17 @@ int launch_moments(thrml_state *st, const uint32_t *d_npos, uint64_t n1, const u
   if (total == 0) return THRML_OK;
   hipEvent_t t0 = nullptr;
   if (p->ctx->time_begin(1, &t0)) return THRML_EHIP;
-  hipLaunchKernelGGL(moments_kernel, dim3(cdiv(total, 256)), dim3(256), 0, p->ctx->stream,
-                     st->words.as<uint64_t>(), (uint64_t)p->n_total, st->G, st->C, d_npos, n1,
-                     d_ppos, n2, d_ones, d_diff);
+  uint32_t lg = 0;
+  while (lg < MOMENTS_MAX_LG && (2u << lg) <= st->G && (total << lg) < MOMENTS_FILL) ++lg;
+  const dim3 grid(cdiv(total, 256u >> lg));
+  if (st->low_live)
+    hipLaunchKernelGGL(moments_kernel<uint32_t>, grid, dim3(256), 0, p->ctx->stream,
+                       st->low.as<uint32_t>(), (uint64_t)p->n_total, st->G, st->C, d_npos, n1, d_ppos,
+                       n2, d_ones, d_diff, lg);
+  else
+    hipLaunchKernelGGL(moments_kernel<uint64_t>, grid, dim3(256), 0, p->ctx->stream,
+                       st->words.as<uint64_t>(), (uint64_t)p->n_total, st->G, st->C, d_npos, n1,
+                       d_ppos, n2, d_ones, d_diff, lg);
   THRML_HIP(hipGetLastError());
   return p->ctx->time_end(1, t0);
 }
@@ -303,27 +329,38 @@ int launch_moments(thrml_state *st, const uint32_t *d_npos, uint64_t n1, const u
 // number of the row's spins are down, so the row's sum over a word is
 // (chains) - 2 popcount(xor of the inverted words); with f = s it is the
 // popcount of the words' AND.  Byte states: the product per chain in int64.
-// One wave per moment row: lanes over the chain groups (bit-packed spin
-// states) or over the chains (byte states, so a wave reads 64 consecutive
-// bytes of a position), then a wave sum that lane 0 adds to the row's total.
+// 1 << lg lanes take a row: lane l of it the chain groups (spin words), or the
+// runs of 4 consecutive chains (byte states, one load per position), l,
+// l + (1 << lg), ...; then a sum over the row's lanes that the first adds to
+// the row's total.  Bound by the dependent loads (row, positions, states): as
+// many lanes as a row has units of work, so that a wave holds as many rows as
+// it can, and two positions at a time.  131,072 rows of one byte-state
+// node, 32 chains: 34.2 us with a wave per row, 7.1 us so.
+// T: the byte states' element, or uint64_t for spin words.
+template <class T>
 __global__ __launch_bounds__(256) void observe_kernel(
-    const uint64_t *__restrict__ words, const uint8_t *__restrict__ cat,
-    const uint16_t *__restrict__ cat16, uint64_t plane_stride,
+    const T *__restrict__ state, uint64_t plane_stride,
     uint32_t G, uint32_t C, uint32_t Cp, const uint64_t *__restrict__ row_off,
-    const uint32_t *__restrict__ pos, uint64_t n_rows, int transform, int64_t *__restrict__ acc) {
-  const uint64_t r = (uint64_t)blockIdx.x * 4u + (threadIdx.x >> 6);  // wave-uniform
-  const uint32_t lane = threadIdx.x & 63u;
-  if (r >= n_rows) return;
+    const uint32_t *__restrict__ pos, uint64_t n_rows, int transform, int64_t *__restrict__ acc,
+    uint32_t lg) {
+  const uint64_t row = ((uint64_t)blockIdx.x * 256u + threadIdx.x) >> lg;
+  const uint32_t l = threadIdx.x & ((1u << lg) - 1u);
+  const uint64_t r = row < n_rows ? row : n_rows - 1u;
   const uint64_t a = row_off[r], b = row_off[r + 1];
   int64_t sum = 0;
-  if (words) {
-    for (uint32_t g = lane; g < G; g += 64u) {
+  if constexpr (sizeof(T) == 8) {
+    for (uint32_t g = l; g < G; g += 1u << lg) {
       const uint32_t rem = C - g * 64u;
       const uint64_t valid = rem < 64u ? (1ull << rem) - 1ull : ~0ull;
       uint64_t m = transform ? 0ull : ~0ull;
-      for (uint64_t k = a; k < b; ++k) {
-        const uint64_t w = words[(size_t)g * plane_stride + pos[k]];
-        m = transform ? (m ^ ~w) : (m & w);
+      for (uint64_t k = a; k < b; k += 2) {
+        // (a last position without a partner is read twice and counts once)
+        const bool pair = k + 1 < b;
+        const uint32_t p0 = pos[k], p1 = pos[pair ? k + 1 : k];
+        const uint64_t w0 = state[(size_t)g * plane_stride + p0];
+        const uint64_t w1 = state[(size_t)g * plane_stride + p1];
+        if (transform) m ^= ~w0 ^ (pair ? ~w1 : 0ull);
+        else m &= w0 & w1;
       }
       const int64_t n = __builtin_popcountll(valid);
       sum += transform ? n - 2 * (int64_t)__builtin_popcountll(m & valid)
@@ -332,32 +369,51 @@ __global__ __launch_bounds__(256) void observe_kernel(
   } else {
     // the observer's creation bounds every row's product (and the run its
     // sum over chains and observations) below 2^63
-    for (uint32_t c = lane; c < C; c += 64u) {
-      int64_t prod = 1;
-      for (uint64_t k = a; k < b; ++k) {
-        const size_t at = (size_t)pos[k] * Cp + c;
-        const int64_t x = cat16 ? (int64_t)cat16[at] : (int64_t)cat[at];
-        prod *= transform ? 2 * x - 1 : x;
+    struct alignas(4 * sizeof(T)) Four {
+      T v[4];
+    };
+    for (uint32_t c = 4u * l; c < C; c += 4u << lg) {
+      uint64_t prod[4] = {1, 1, 1, 1};  // (chains past C may hold anything)
+      for (uint64_t k = a; k < b; k += 2) {
+        const bool pair = k + 1 < b;
+        const uint32_t p0 = pos[k], p1 = pos[pair ? k + 1 : k];
+        // (Cp is a multiple of 4)
+        const Four x0 = *reinterpret_cast<const Four *>(state + (size_t)p0 * Cp + c);
+        const Four x1 = *reinterpret_cast<const Four *>(state + (size_t)p1 * Cp + c);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int32_t f0 = transform ? 2 * (int32_t)x0.v[u] - 1 : (int32_t)x0.v[u];
+          const int32_t f1 = !pair ? 1 : transform ? 2 * (int32_t)x1.v[u] - 1 : (int32_t)x1.v[u];
+          // (below 2^34: the factors are 16 bits and a sign)
+          prod[u] *= (uint64_t)((int64_t)f0 * f1);
+        }
       }
-      sum += prod;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) sum += c + (uint32_t)u < C ? (int64_t)prod[u] : 0;
     }
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-  if (lane == 0u) acc[r] += sum;
+  for (uint32_t off = (1u << lg) >> 1; off > 0u; off >>= 1) sum += __shfl_xor(sum, (int)off);
+  if (l == 0u && row < n_rows) acc[r] += sum;
+}
+
+template <class T>
+static void launch_observe_t(thrml_state *st, thrml_observer *obs, const T *state) {
+  // lanes per row: one per chain group or run of 4 chains, up to a wave
+  const uint32_t units = sizeof(T) == 8 ? st->G : cdiv(st->C, 4);
+  uint32_t lg = 0;
+  while (lg < 6u && (1u << lg) < units) ++lg;
+  hipLaunchKernelGGL(observe_kernel<T>, dim3(cdiv(obs->n_rows << lg, 256)), dim3(256), 0,
+                     st->prog->ctx->stream, state, (uint64_t)st->prog->n_total, st->G, st->C, st->Cp,
+                     obs->row_off.as<uint64_t>(), obs->pos.as<uint32_t>(), obs->n_rows,
+                     obs->transform ? 1 : 0, obs->acc.as<int64_t>(), lg);
 }
 
 int launch_observe(thrml_state *st, thrml_observer *obs) {
   thrml_prog *p = st->prog;
   if (obs->n_rows == 0) return THRML_OK;
-  const bool bytes = byte_layout(p);
-  hipLaunchKernelGGL(observe_kernel, dim3(cdiv(obs->n_rows, 4)), dim3(256), 0, p->ctx->stream,
-                     bytes ? nullptr : st->words.as<uint64_t>(),
-                     bytes && p->cat_bytes == 1 ? st->cat.as<uint8_t>() : nullptr,
-                     bytes && p->cat_bytes == 2 ? st->cat.as<uint16_t>() : nullptr,
-                     (uint64_t)p->n_total, st->G, st->C,
-                     st->Cp, obs->row_off.as<uint64_t>(), obs->pos.as<uint32_t>(), obs->n_rows,
-                     obs->transform ? 1 : 0, obs->acc.as<int64_t>());
+  if (!byte_layout(p)) launch_observe_t(st, obs, st->words.as<uint64_t>());
+  else if (p->cat_bytes == 2) launch_observe_t(st, obs, st->cat.as<uint16_t>());
+  else launch_observe_t(st, obs, st->cat.as<uint8_t>());
   THRML_HIP(hipGetLastError());
   return THRML_OK;
 }
@@ -414,6 +470,11 @@ int launch_finalize_moments(thrml_ctx *ctx, const uint32_t *cnt1, const uint64_t
 // hinton_init (crates/thrml-models/src/ising.rs:602-673) of free block b:
 // entry (c, i) of the [C, n_b] uniform tensor is keystream word c*n_b + i of
 // the block key; s = (word <= threshold(sigmoid(b_i * beta))).
+// A wave takes 16 sites of a chain group.  Bound by instructions: the two
+// blocks that hold a chain's 16 words, whose alignment differs by lane, are
+// picked from through LDS (a select over 32 registers per word took most of
+// the time: blocks of 100,000 sites on average, 32 chains 28.9 -> 15 us, of
+// 800 sites, one chain 15.2 -> 5.4 us).
 __global__ void hinton_kernel(const uint32_t *__restrict__ key8, const float *__restrict__ prob,
                               uint32_t C, uint32_t n_b, uint64_t *__restrict__ words,
                               uint64_t group_stride, uint64_t blk_off, uint32_t n_seg,
@@ -429,25 +490,31 @@ __global__ void hinton_kernel(const uint32_t *__restrict__ key8, const float *__
   for (int i = 0; i < 8; ++i) key.k[i] = key8[i];
   const uint32_t i0 = seg * 16u;
   const uint64_t w0 = (uint64_t)c * n_b + i0;
-  uint32_t a[16], bb[16];
-  chacha_block<8>(key.k, w0 >> 4, a);
-  chacha_block<8>(key.k, (w0 >> 4) + 1, bb);
+  // the 16 words start anywhere in their first block: both blocks go through
+  // LDS, lane-major (lane 0's words are at ks[0], ks[64], ...)
+  __shared__ uint32_t ks_all[4 * 32 * 64];
+  uint32_t *ks = ks_all + (threadIdx.x >> 6) * (32u * 64u) + lane;
   const uint32_t sh = (uint32_t)(w0 & 15u);
-#pragma unroll 1
-  for (uint32_t k = 0; k < 16u; ++k) {
-    const uint32_t i = i0 + k;
-    if (i >= n_b) break;
-    const uint32_t pos = sh + k;  // 0..30
-    uint32_t wd = 0;
+  {
+    uint32_t a[16];
+    chacha_block<8>(key.k, w0 >> 4, a);
 #pragma unroll
-    for (uint32_t t = 0; t < 16u; ++t) {
-      wd = (pos == t) ? a[t] : wd;
-      wd = (pos == t + 16u) ? bb[t] : wd;
-    }
-    const bool up = (c < C) && (wd <= word_threshold(prob[i]));
-    const uint64_t m = __builtin_amdgcn_ballot_w64(up);
-    if (lane == 0) out[i] = m;
+    for (uint32_t t = 0; t < 16u; ++t) ks[t * 64u] = a[t];
+    chacha_block<8>(key.k, (w0 >> 4) + 1, a);
+#pragma unroll
+    for (uint32_t t = 0; t < 16u; ++t) ks[(t + 16u) * 64u] = a[t];
   }
+  // lane k keeps site i0 + k's word and probability
+  const float pr = prob[min(i0 + (lane & 15u), n_b - 1u)];
+  const uint32_t thr = word_threshold(pr);
+  uint64_t mine = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < 16u; ++k) {
+    const uint32_t th = (uint32_t)__builtin_amdgcn_readlane((int)thr, (int)k);
+    const uint64_t m = __builtin_amdgcn_ballot_w64(c < C && ks[(sh + k) * 64u] <= th);
+    mine = lane == k ? m : mine;
+  }
+  if (lane < 16u && i0 + lane < n_b) out[i0 + lane] = mine;
 }
 
 int launch_hinton(thrml_prog *p, thrml_state *st, uint32_t b, const uint32_t *d_key8,

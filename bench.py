@@ -414,9 +414,10 @@ def workload_c1(args, th, wl, torch):
     step = _run_blocks_workload(th, dev, prog, st, sweeps, keys)
     res = {"config": {"workload": "ising_lattice_64_c256_1000sweeps", "L": 64, "chains": C,
                       "sweeps_per_step": sweeps, "blocks": 2}, "dtype": "f32"}
+    # one launch runs every sweep of a step: the figures are per half-sweep
     return dev, step, C * N * sweeps, res, dict(
-        kernel="lattice_half_kernel", bytes_per_launch=(2 * C * N + 4 * N + 4 * E) / 2.0,
-        traffic="lattice_half_kernel_c1_traffic.txt", valu="lattice_half_kernel_c1_valu.txt",
+        kernel="resident_reg_kernel", bytes_per_launch=(2 * C * N + 4 * N + 4 * E) / 2.0,
+        traffic="resident_reg_kernel_c1_traffic.txt", valu="resident_reg_kernel_c1_valu.txt",
         timing_step=lambda i: step(-1 - i), extra=lambda: {},
         energy=lambda: th.ising_energy(prog, st),
         cpu=lambda: cpu_ising(ebm, blocks, args.cpu_seconds, False),

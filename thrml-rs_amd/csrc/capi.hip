@@ -1302,7 +1302,7 @@ extern "C" int thrml_state_create(thrml_prog *p, uint32_t n_chains, thrml_state 
   // the sweep kernel's half-size gather copy (refreshed at each run's start)
   if (!rc && p->kind == K_CSR && n_chains <= 32u && p->planes == 1u && p->stage_max == 0)
     rc = st->low.alloc((size_t)p->n_total * sizeof(uint32_t), pool);
-  if (!rc && p->res_T)
+  if (!rc && p->res_T && n_chains > 1u)
     rc = st->bits.alloc((size_t)n_chains * ((p->n_total + 63u) / 64u) * sizeof(uint64_t), pool);
   if (!rc && p->stage_max) {
     // cleared once: the padding chains of a categorical row are copied back

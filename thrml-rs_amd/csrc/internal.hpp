@@ -308,7 +308,8 @@ struct thrml_state {
   // low_live: it holds the current spins (set within a run that keeps it).
   thrml::DevBuf low;
   bool low_live = false;
-  // resident runs: [C][ceil(n_total / 64)] u64, the chains' spins at a run's end
+  // resident runs of several chains: [C][ceil(n_total / 64)] u64, the chains'
+  // spins at a run's end
   thrml::DevBuf bits;
   // dense path operands: spin-down bits per block, one bit vector per chain
   // (bit k%32 of word k/32 is 1 when the spin at block position k is down)

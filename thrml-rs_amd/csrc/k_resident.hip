@@ -42,7 +42,7 @@
 namespace thrml {
 
 struct ResArgs {
-  const uint64_t *words;    // state words, group 0
+  uint64_t *words;          // state words, group 0; written here for one chain
   uint64_t *bits;           // [C][n_words] new spins of each chain, 64 positions per word
   const uint32_t *keys;     // [n_sweeps][n_blocks][C_pad][KEY_WORDS]
   const ResPiece *pieces;
@@ -128,10 +128,18 @@ __device__ __forceinline__ void res_load_state(const ResArgs &a, uint32_t chain,
     f(p, (w32[2u * p] >> (chain & 31u)) & 1u);
 }
 
-// The chain's spins, 64 positions per word; up(position) tells a spin.
+// The chain's spins, 64 positions per word; up(position) tells a spin.  A single
+// chain's state words hold nothing else, and no other workgroup writes them:
+// they are written at once, which saves resident_commit_kernel's launch (one
+// chain of a 10^2 torus, 20 observed states: 238 -> 190 us; of two 40^2 layers,
+// a training step of 20 observations: 1750 -> 1668 us).
 template <class F>
 __device__ __forceinline__ void res_store_bits(const ResArgs &a, uint32_t chain, F &&up) {
   const uint32_t lane = threadIdx.x & 63u;
+  if (gridDim.x == 1u) {
+    for (uint32_t p = threadIdx.x; p < a.n_total; p += blockDim.x) a.words[p] = up(p) ? 1ull : 0ull;
+    return;
+  }
   for (uint32_t p0 = threadIdx.x & ~63u; p0 < a.n_total; p0 += blockDim.x) {
     const uint32_t p = p0 + lane;
     const uint64_t m = __builtin_amdgcn_ballot_w64(p < a.n_total && up(p));
@@ -647,10 +655,12 @@ int launch_resident(thrml_prog *p, thrml_state *st, const uint32_t *d_keys, uint
   void *args[] = {&a};
   THRML_HIP(hipLaunchKernel(p->res_ent ? reg_kernel(p->res_ent) : stream_kernel(p->res_pf), dim3(st->C),
                             dim3(p->res_T), args, lds, s));
-  const uint32_t n_tasks = a.n_words * st->G;
-  hipLaunchKernelGGL(resident_commit_kernel, dim3((n_tasks + 3u) / 4u), dim3(256), 0, s, a.bits,
-                     a.n_words, st->C, a.n_total, n_tasks, st->words.as<uint64_t>());
-  THRML_HIP(hipGetLastError());
+  if (st->C > 1u) {
+    const uint32_t n_tasks = a.n_words * st->G;
+    hipLaunchKernelGGL(resident_commit_kernel, dim3((n_tasks + 3u) / 4u), dim3(256), 0, s, a.bits,
+                       a.n_words, st->C, a.n_total, n_tasks, st->words.as<uint64_t>());
+    THRML_HIP(hipGetLastError());
+  }
   return p->ctx->time_end(0, t0, (uint64_t)n_sweeps * p->n_free);
 }
 

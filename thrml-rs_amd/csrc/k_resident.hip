@@ -496,9 +496,6 @@ int resident_tables(thrml_prog *p, const std::vector<uint32_t> &row_off, const u
       pf = c;
     }
   }
-#ifdef RES_PF_FORCE
-  pf = RES_PF_FORCE;
-#endif
   uint64_t at = RES_SITES;  // (an entry's data start 512 bytes before its pairs)
   for (ResSlice &sl : slices) {
     sl.pf = pf;

@@ -1368,13 +1368,13 @@ struct Staging {
   void *p = nullptr;
   int get(thrml_ctx *ctx, size_t bytes) {
     if (bytes > thrml_ctx::IO_KEEP) {
-      if (int rc = own.alloc(bytes)) return rc;
+      if (int rc = own.alloc_own(bytes, &ctx->pool)) return rc;
       p = own.p;
       return THRML_OK;
     }
     lk = std::unique_lock<std::mutex>(ctx->io_mu);
     if (ctx->io.bytes < bytes)  // (its last use has ended: every user waits before unlocking)
-      if (int rc = ctx->io.alloc(std::max<size_t>(bytes, 1u << 16))) return rc;
+      if (int rc = ctx->io.alloc_own(std::max<size_t>(bytes, 1u << 16), &ctx->pool)) return rc;
     p = ctx->io.p;
     return THRML_OK;
   }
@@ -1568,7 +1568,7 @@ int run_plan(thrml_prog *p, thrml_state *st, const Plan &pl, const LatticeMoment
     const uint64_t need = ns * per_sweep;
     if (ks.grow && ks.grow->bytes < need) {
       THRML_HIP(hipStreamSynchronize(p->ctx->stream));
-      if (int rc = ks.grow->alloc(need)) return rc;
+      if (int rc = ks.grow->alloc_own(need, &p->ctx->pool)) return rc;
     }
     uint32_t *keys = ks.grow ? ks.grow->as<uint32_t>() : ks.fixed;
     // the previous chunk's sweeps read the same buffer; stream order keeps

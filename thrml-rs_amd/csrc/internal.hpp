@@ -118,24 +118,22 @@ struct DevBuf {
     pool_ = nullptr;
     bytes = cap_ = 0;
   }
-  int alloc(size_t n, DevPool *pool = nullptr) {
+  // n bytes, from the pool and back to it
+  int alloc(size_t n, DevPool *pool) {
     release();
     if (n == 0) n = 16;
-    if (pool) p = pool->take(n, &cap_, &era_);
-    if (!p) {
-      hipError_t e = hipMalloc(&p, n);
-      if (e != hipSuccess && pool) {  // what the pool holds may be what is missing
-        pool->clear();
-        e = hipMalloc(&p, n);
-      }
-      if (e != hipSuccess) {
-        p = nullptr;
-        return fail(THRML_ENOMEM, "device allocation of " + std::to_string(n) + " bytes failed: " +
-                                      hipGetErrorString(e));
-      }
-      cap_ = n;
-    }
+    p = pool->take(n, &cap_, &era_);
+    if (!p)
+      if (int rc = allocate(n, pool)) return rc;
     pool_ = pool;
+    bytes = n;
+    return THRML_OK;
+  }
+  // n bytes that go back to the device: for buffers that a context keeps itself
+  int alloc_own(size_t n, DevPool *pool) {
+    release();
+    if (n == 0) n = 16;
+    if (int rc = allocate(n, pool)) return rc;
     bytes = n;
     return THRML_OK;
   }
@@ -145,6 +143,23 @@ struct DevBuf {
   }
 
  private:
+  int allocate(size_t n, DevPool *pool) {
+    hipError_t e = hipMalloc(&p, n);
+    if (e != hipSuccess) {  // what the pool holds may be what is missing
+      pool->clear();
+      e = hipMalloc(&p, n);
+      // taken back, or the next launch's check would find the failure
+      (void)hipGetLastError();
+    }
+    if (e != hipSuccess) {
+      p = nullptr;
+      return fail(THRML_ENOMEM, "device allocation of " + std::to_string(n) + " bytes failed: " +
+                                    hipGetErrorString(e));
+    }
+    cap_ = n;
+    return THRML_OK;
+  }
+
   DevPool *pool_ = nullptr;
   size_t cap_ = 0;
   uint64_t era_ = 0;

@@ -956,7 +956,7 @@ extern "C" int thrml_rbm_half_sweep(thrml_prog *p, thrml_state *st, int blk, con
   std::vector<uint32_t> k((size_t)st->G * 64u * KEY_WORDS, 0u);
   for (uint32_t c = 0; c < st->C; ++c) key_expand(key8 + (size_t)c * 8u, &k[(size_t)c * KEY_WORDS]);
   DevBuf dk;
-  if (int rc = dk.alloc(k.size() * 4)) return rc;
+  if (int rc = dk.alloc_own(k.size() * 4, &p->ctx->pool)) return rc;
   THRML_HIP(hipMemcpyAsync(dk.p, k.data(), k.size() * 4, hipMemcpyHostToDevice, p->ctx->stream));
   if (int rc = launch_dense_half(p, st, (uint32_t)blk, dk.as<uint32_t>())) return rc;
   THRML_HIP(hipStreamSynchronize(p->ctx->stream));

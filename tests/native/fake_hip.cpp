@@ -35,7 +35,7 @@ std::mutex mu;
 std::vector<Op> queue;
 std::map<uintptr_t, size_t> blocks;
 size_t capacity = ~(size_t)0, live = 0;
-uint64_t n_malloc = 0, fail_at = 0;  // fail_at: allocations left until one fails
+uint64_t n_malloc = 0, fail_at = 0;  // fail_at: the allocations from which on all fail
 int cus = 256;
 std::map<const void *, std::string> names;
 std::map<std::string, uint64_t> launches;
@@ -84,7 +84,7 @@ void fake_reset() {
   launches.clear();
 }
 void fake_set_capacity(uint64_t bytes) { capacity = bytes; }
-void fake_fail_malloc(uint64_t nth) { fail_at = nth; }  // 1: the next one; 0: none
+void fake_fail_malloc(uint64_t nth) { fail_at = nth ? n_malloc + nth : 0; }  // 1: from the next one on; 0: none
 void fake_set_cus(int n) { cus = n; }
 uint64_t fake_live_bytes() { return live; }
 uint64_t fake_mallocs() { return n_malloc; }
@@ -128,7 +128,7 @@ hipError_t hipGetLastError() {
 hipError_t hipMalloc(void **p, size_t n) {
   std::lock_guard<std::mutex> lk(mu);
   ++n_malloc;
-  if ((fail_at && --fail_at == 0) || live + n > capacity) return ret(hipErrorOutOfMemory);
+  if ((fail_at && n_malloc >= fail_at) || live + n > capacity) return ret(hipErrorOutOfMemory);
   void *m = mmap(nullptr, n, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
   if (m == MAP_FAILED) return ret(hipErrorOutOfMemory);
   blocks[(uintptr_t)m] = n;

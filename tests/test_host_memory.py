@@ -49,3 +49,84 @@ def test_kept_blocks_make_room(what):
     """An allocation that the device refuses is tried again without the blocks
     that the context keeps, whoever makes it."""
     hostrun.call(_low_memory, what)
+
+
+def _graph():
+    e = np.unique(np.sort(np.random.default_rng(1).integers(0, 90, (300, 2)), axis=1), axis=0)
+    e = e[e[:, 0] != e[:, 1]].astype(np.uint32)
+    return 90, e, th.coloring_to_blocks(th.greedy_coloring(90, e))
+
+
+def _csr(dev):
+    n, e, blocks = _graph()
+    return th.IsingSamplingProgram(th.IsingEBM(n, e, np.zeros(n), np.zeros(len(e))), blocks, [], dev)
+
+
+def _potts(dev):
+    n, e, blocks = _graph()
+    return th.CategoricalProgram(n, 5, e, np.zeros((len(e), 5, 5)), np.zeros((n, 5)), blocks, dev)
+
+
+def _factors(dev):
+    n, e, blocks = _graph()
+    f = th.SpinEBMFactor([e[:, 0], e[:, 1]], np.zeros((len(e), 1, 1)))
+    return th.FactorSamplingProgram(np.zeros(n, np.uint8), 2, [f], blocks, [], dev)
+
+
+def _nothing(dev):
+    return dev
+
+
+def _energy(prog):
+    st = prog.new_state(3)
+    return lambda: th.energy(prog, st)
+
+
+# name: (what stands before, the call on it)
+CALLS = {
+    "lattice program": (_nothing, _lattice),
+    "irregular program": (_nothing, _csr),
+    "categorical program": (_nothing, _potts),
+    "factor program": (_nothing, _factors),
+    "dense program": (_nothing, _rbm),
+    "moments": (_csr, lambda p: th.MomentAccumulatorObserver(p, th.ising_moment_spec(np.arange(90), _graph()[1]))),
+    "observer": (_csr, lambda p: th.MomentAccumulatorObserver(p, [[[0], [1, 2, 3]]])),
+    "hinton_init": (lambda dev: (lambda p: (p, p.new_state(4)))(_rbm(dev)),
+                    lambda s: th.hinton_init(th.RngKey(1), s[0], state=s[1])),
+    "spin energies": (lambda dev: _energy(_csr(dev)), lambda f: f()),
+    "categorical energies": (lambda dev: _energy(_potts(dev)), lambda f: f()),
+    "factor energies": (lambda dev: _energy(_factors(dev)), lambda f: f()),
+    "dense energies": (lambda dev: _energy(_rbm(dev)), lambda f: f()),
+}
+
+
+def _each_allocation_fails(name):
+    before, do = CALLS[name]
+    fake = hostrun.fake
+    _lattice(th.Device(0))  # the device's one-time checks
+    fails = 0
+    for nth in range(1, 40):
+        dev = th.Device(0)
+        what = before(dev)
+        fake.fake_fail_malloc(nth)
+        try:
+            do(what)
+            done = True
+        except th.ThrmlError as e:
+            assert "device allocation of" in str(e)
+            done = False
+        assert fake.fake_pending_host() == 0, f"allocation {nth} refused: copies of freed memory are queued"
+        fake.fake_fail_malloc(0)
+        assert fake.hipGetLastError() == 0
+        if done:
+            return fails
+        do(what)  # and it works once there is memory
+        fails += 1
+    raise AssertionError("no end to the allocations")
+
+
+@pytest.mark.parametrize("name", CALLS)
+def test_no_copy_outlives_its_memory(name):
+    """Whichever allocation fails, the copies that a call has queued from or to
+    its own or the caller's memory have ended when it returns."""
+    assert hostrun.call(_each_allocation_fails, name) >= 1

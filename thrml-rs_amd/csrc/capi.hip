@@ -809,6 +809,8 @@ extern "C" int thrml_ising_program_create(thrml_ctx *ctx, const thrml_ising_desc
     p->kind = K_LATTICE;
     DevBuf d_dir, d_slots, d_b;
     const std::vector<uint32_t> slots2 = pack_slots(slot_pos, slot_w);
+    std::vector<uint8_t> keep;
+    StreamWait queued(ctx->stream);
     if ((rc = upload(p, p->row_off, row_off)) || (rc = upload(p, d_dir, dir)) ||
         (rc = upload(p, d_slots, slots2)) || (rc = upload(p, d_b, bias_w)) ||
         (rc = p->table.alloc(nf * 16 * sizeof(uint32_t), &ctx->pool))) {
@@ -822,10 +824,9 @@ extern "C" int thrml_ising_program_create(thrml_ctx *ctx, const thrml_ising_desc
     double mag = 0.0;
     for (float x : slot_w) mag += std::fabs((double)x);
     for (float x : bias_w) mag += std::fabs((double)x);
-    std::vector<uint8_t> keep;
     if (!rc && mag < 1e38)
       rc = resident_tables(p, row_off, p->row_off.as<uint32_t>(), d_slots.as<uint2>(), d_b.as<float>(), keep);
-    const hipError_t e = hipStreamSynchronize(ctx->stream);
+    const hipError_t e = queued.now();
     if (!rc && e != hipSuccess) rc = hip_fail(e, "lattice table");
     p->device_bytes -= p->row_off.bytes + d_dir.bytes + d_slots.bytes + d_b.bytes;
     p->row_off.release();
@@ -837,15 +838,16 @@ extern "C" int thrml_ising_program_create(thrml_ctx *ctx, const thrml_ising_desc
     p->kind = K_CSR;
     csr_windows(p, row_off);
     const std::vector<uint32_t> slots2 = pack_slots(slot_pos, slot_w);
+    std::vector<uint8_t> keep;
+    StreamWait queued(ctx->stream);
     if ((rc = upload(p, p->row_off, row_off)) || (rc = upload(p, p->slots, slots2)) ||
         (rc = upload(p, p->bias_w, bias_w))) {
       delete p;
       return rc;
     }
-    std::vector<uint8_t> keep;
     rc = resident_tables(p, row_off, p->row_off.as<uint32_t>(), p->slots.as<uint2>(),
                          p->bias_w.as<float>(), keep);
-    hipError_t e = hipStreamSynchronize(ctx->stream);
+    const hipError_t e = queued.now();
     if (!rc && e != hipSuccess) rc = hip_fail(e, "program upload");
     if (rc) {
       delete p;
@@ -1240,11 +1242,12 @@ extern "C" int thrml_discrete_program_create(thrml_ctx *ctx, const thrml_discret
   if (sp.empty()) sp.push_back(0u);
   if (tsp.empty()) tsp.push_back(0u);
   if (terms.empty()) terms.assign(8, 0u);
+  StreamWait queued(ctx->stream);
   if ((rc = upload(p, p->row_off, row_off)) || (rc = upload(p, p->d_slots, slots)) ||
       (rc = upload(p, p->d_sp, sp)) || (rc = upload(p, p->d_w, w)) ||
       (rc = upload(p, p->d_terms, terms)) || (rc = upload(p, p->d_tsp, tsp)))
     return bail(rc);
-  hipError_t e = hipStreamSynchronize(ctx->stream);
+  const hipError_t e = queued.now();
   if (e != hipSuccess) return bail(hip_fail(e, "program upload"));
   *out = p;
   return THRML_OK;
@@ -1808,9 +1811,10 @@ extern "C" int thrml_moments_run(thrml_prog *p, uint64_t key, thrml_schedule sch
   rc = launch_finalize_moments(p->ctx, c1, m->acc1, m->slot1, m->n1, c2, m->acc2, m->slot2, m->n2, cn, o1, o2);
   if (rc) return rc;
   if (!out_on_device) {
+    StreamWait queued(s);
     if (m->n1) THRML_HIP(hipMemcpyAsync(node_sums, o1, m->n1 * 8, hipMemcpyDeviceToHost, s));
     if (m->n2) THRML_HIP(hipMemcpyAsync(pair_sums, o2, m->n2 * 8, hipMemcpyDeviceToHost, s));
-    THRML_HIP(hipStreamSynchronize(s));
+    THRML_HIP(queued.now());
   }
   return THRML_OK;
 }
@@ -1858,11 +1862,12 @@ extern "C" int thrml_observer_create(thrml_prog *p, const uint64_t *row_offsets,
   o->max_row_log2 = max_log2;
   std::vector<uint64_t> off(row_offsets, row_offsets + n_rows + (n_rows ? 1 : 0));
   if (off.empty()) off.push_back(0);
+  StreamWait queued(p->ctx->stream);
   int rc = upload_to(p->ctx, o->row_off, off);
   if (!rc) rc = upload_to(p->ctx, o->pos, pos);
   if (!rc) rc = o->acc.alloc(std::max<uint64_t>(n_rows, 1) * sizeof(int64_t), &p->ctx->pool);
   if (!rc) {
-    hipError_t e = hipStreamSynchronize(p->ctx->stream);
+    const hipError_t e = queued.now();
     if (e != hipSuccess) rc = hip_fail(e, "observer upload");
   }
   if (rc) {
@@ -2011,6 +2016,7 @@ extern "C" int thrml_hinton_init(thrml_prog *p, uint64_t key, thrml_state *st) {
     for (int i = 0; i < 8; ++i) k8[8 * b + i] = e.k[i];
   }
   DevBuf dk, dp;
+  StreamWait queued(p->ctx->stream);
   int rc;
   if ((rc = dk.alloc(k8.size() * 4, &p->ctx->pool)) || (rc = dp.alloc(prob.size() * 4, &p->ctx->pool))) return rc;
   THRML_HIP(hipMemcpyAsync(dk.p, k8.data(), k8.size() * 4, hipMemcpyHostToDevice, p->ctx->stream));
@@ -2021,7 +2027,7 @@ extern "C" int thrml_hinton_init(thrml_prog *p, uint64_t key, thrml_state *st) {
   if (p->kind == K_DENSE)
     for (uint32_t b = 0; b < 2; ++b)
       if ((rc = launch_dense_sync_act(st, b))) return rc;
-  THRML_HIP(hipStreamSynchronize(p->ctx->stream));
+  THRML_HIP(queued.now());
   return THRML_OK;
 }
 

@@ -165,6 +165,26 @@ struct DevBuf {
   uint64_t era_ = 0;
 };
 
+// Declared after host memory that copies queued on a stream read or write: they
+// have ended when the scope is left, on whatever path.
+class StreamWait {
+ public:
+  explicit StreamWait(hipStream_t s) : stream_(s) {}
+  StreamWait(const StreamWait &) = delete;
+  StreamWait &operator=(const StreamWait &) = delete;
+  ~StreamWait() {
+    if (open_) (void)hipStreamSynchronize(stream_);
+  }
+  hipError_t now() {
+    open_ = false;
+    return hipStreamSynchronize(stream_);
+  }
+
+ private:
+  hipStream_t stream_;
+  bool open_ = true;
+};
+
 struct TimingSlot {
   std::vector<hipEvent_t> ev;  // pairs
   std::vector<uint64_t> n;     // half-sweeps of each pair's launch

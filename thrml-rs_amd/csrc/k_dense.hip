@@ -812,18 +812,19 @@ int dense_program_create(thrml_ctx *ctx, const DenseSpec &d, thrml_prog **out) {
   if (int rc = fast_math_gate(ctx, nullptr, nullptr)) return rc;
   // the fewest bf16 pieces that hold every weight exactly, found on the device
   DevBuf wraw, cnt;
+  const uint32_t cnt_init[2] = {1u, 0u};
+  uint32_t cnt_h[2] = {0u, 0u};
+  StreamWait queued(ctx->stream);
   if (int rc = upload_to(ctx, wraw, d.w)) return rc;
   if (int rc = cnt.alloc(2 * sizeof(uint32_t), &ctx->pool)) return rc;
-  const uint32_t cnt_init[2] = {1u, 0u};
   THRML_HIP(hipMemcpyAsync(cnt.p, cnt_init, sizeof cnt_init, hipMemcpyHostToDevice, ctx->stream));
   const uint64_t n_w = (uint64_t)V * H;
   if ((n_w + 255) / 256 > 0x7fffffffull) return fail(THRML_EUNSUPPORTED, "too many dense weights");
   hipLaunchKernelGGL(dense_pieces_count_kernel, dim3((uint32_t)std::min<uint64_t>((n_w + 255) / 256, 512)),
                      dim3(256), 0, ctx->stream, wraw.as<float>(), n_w, cnt.as<uint32_t>());
   THRML_HIP(hipGetLastError());
-  uint32_t cnt_h[2] = {0u, 0u};
   THRML_HIP(hipMemcpyAsync(cnt_h, cnt.p, sizeof cnt_h, hipMemcpyDeviceToHost, ctx->stream));
-  THRML_HIP(hipStreamSynchronize(ctx->stream));
+  THRML_HIP(queued.now());
   if (cnt_h[1])
     return fail(THRML_EUNSUPPORTED, "a dense weight is not finite or not a sum of three normal bf16 values");
   const uint32_t P = std::min(3u, std::max(1u, cnt_h[0]));

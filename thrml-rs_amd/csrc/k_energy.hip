@@ -181,7 +181,7 @@ static int energy_tables(thrml_prog *p) {
   std::lock_guard<std::mutex> lock(p->en_mu);
   if (p->en_ready) return THRML_OK;
   std::vector<uint32_t> pos;
-  std::vector<float> w;
+  std::vector<float> w, bias;
   pos.reserve(2 * p->eu.size());
   if (p->kind != K_POTTS) w.reserve(p->eu.size());
   for (size_t e = 0; e < p->eu.size(); ++e) {
@@ -192,15 +192,16 @@ static int energy_tables(thrml_prog *p) {
     if (p->kind != K_POTTS) w.push_back(p->w_raw[e]);
   }
   p->en_ne = pos.size() / 2;
+  StreamWait queued(p->ctx->stream);
   int rc = upload_to(p->ctx, p->en_pos, pos);
   if (!rc && p->kind != K_POTTS) rc = upload_to(p->ctx, p->en_w, w);
   if (!rc && p->kind != K_POTTS) {
-    std::vector<float> b(p->n_total);
-    for (uint64_t k = 0; k < p->n_total; ++k) b[k] = p->bias_raw[p->pos_node[k]];
-    rc = upload_to(p->ctx, p->en_bias, b);
+    bias.resize(p->n_total);
+    for (uint64_t k = 0; k < p->n_total; ++k) bias[k] = p->bias_raw[p->pos_node[k]];
+    rc = upload_to(p->ctx, p->en_bias, bias);
   }
   if (!rc) {
-    hipError_t e = hipStreamSynchronize(p->ctx->stream);
+    const hipError_t e = queued.now();
     if (e != hipSuccess) rc = hip_fail(e, "energy tables");
   }
   if (rc) return rc;

@@ -1,5 +1,8 @@
 """Device memory and waits of the library's host code, against a stand-in of the
 HIP runtime (hostrun.py): no GPU is used and no kernel runs."""
+import ctypes
+import threading
+
 import numpy as np
 import pytest
 
@@ -49,6 +52,60 @@ def test_kept_blocks_make_room(what):
     """An allocation that the device refuses is tried again without the blocks
     that the context keeps, whoever makes it."""
     hostrun.call(_low_memory, what)
+
+
+def _read_during_a_run():
+    """Whether a state can be read by a second thread while sample_states is
+    between two of its launches."""
+    dev = th.Device(0)
+    prog = _csr(dev)
+    st, other = prog.new_state(4), prog.new_state(4)
+    reads = []
+
+    @ctypes.CFUNCTYPE(None)
+    def launched():
+        hostrun.fake.fake_on_launch(None)
+        t = threading.Thread(target=lambda: reads.append(other.get_block(0)))
+        t.start()
+        t.join(timeout=10)
+        reads.append("run goes on")
+
+    hostrun.fake.fake_on_launch(launched)
+    th.sample_states(th.RngKey(1), prog, th.SamplingSchedule(1, 3, 1), st)
+    return [r if isinstance(r, str) else "read" for r in reads]
+
+
+def test_transfers_do_not_wait_for_a_run():
+    assert hostrun.call(_read_during_a_run) == ["read", "run goes on"]
+
+
+def _transfer_memory():
+    """Device memory after transfers of several sizes, whole states and blocks."""
+    dev = th.Device(0)
+    prog = _lattice(dev)
+    st = prog.new_state(1 << 13)
+    st.get_block(0)  # 16 MiB
+    fake = hostrun.fake
+    before, n = fake.fake_live_bytes(), fake.fake_mallocs()
+    st.get_global()
+    grown = fake.fake_live_bytes() - before
+    for _ in range(3):
+        st.get_block(0)
+        st.get_global()
+        small = prog.new_state(3)
+        small.set_global(small.get_global())
+    st.get_block(0, np.float32)
+    st.get_block(0)
+    return grown, fake.fake_mallocs() - n, fake.fake_live_bytes() - before
+
+
+def test_one_block_serves_transfers_of_every_size():
+    """The block grows to the largest transfer of up to 64 MiB and serves the
+    smaller ones."""
+    grown, mallocs, end = hostrun.call(_transfer_memory)
+    assert grown == 16 << 20          # 32 MiB in place of 16
+    assert end - (48 << 20) < 1 << 16  # 64 MiB in place of 16, and the small state
+    assert mallocs <= 4               # two larger blocks, the small state's words and flag
 
 
 def _graph():

@@ -1363,26 +1363,6 @@ struct ObservingScope {
   ObservingScope &operator=(const ObservingScope &) = delete;
 };
 
-// Device memory for one host transfer: the context's kept staging buffer, or
-// a buffer of its own when that would keep too much.
-struct Staging {
-  std::unique_lock<std::mutex> lk;
-  DevBuf own;
-  void *p = nullptr;
-  int get(thrml_ctx *ctx, size_t bytes) {
-    if (bytes > thrml_ctx::IO_KEEP) {
-      if (int rc = own.alloc_own(bytes, &ctx->pool)) return rc;
-      p = own.p;
-      return THRML_OK;
-    }
-    lk = std::unique_lock<std::mutex>(ctx->io_mu);
-    if (ctx->io.bytes < bytes)  // (its last use has ended: every user waits before unlocking)
-      if (int rc = ctx->io.alloc_own(std::max<size_t>(bytes, 1u << 16), &ctx->pool)) return rc;
-    p = ctx->io.p;
-    return THRML_OK;
-  }
-};
-
 // Blocks b0 .. b1 - 1 (consecutive positions) from / to rows of their values.
 static int state_io(thrml_state *st, uint32_t b0, uint32_t b1, void *buf, int dtype, int on_device,
                     bool write) {
@@ -1398,13 +1378,13 @@ static int state_io(thrml_state *st, uint32_t b0, uint32_t b1, void *buf, int dt
   const size_t bytes = (size_t)st->C * n * (dtype == THRML_DTYPE_U8 ? 1 : 4);
   hipStream_t s = p->ctx->stream;
   void *dev = buf;
-  Staging tmp;
+  DevBuf tmp;
   if (!on_device) {
-    if (int rc = tmp.get(p->ctx, bytes)) return rc;
+    if (int rc = tmp.alloc_transfer(bytes, &p->ctx->pool)) return rc;
     dev = tmp.p;
   }
-  // nothing of this call is in flight when it returns: the staging buffer and
-  // the caller's memory are free again
+  // nothing of this call is in flight when it returns: the caller's memory is
+  // free again
   const int rc = [&]() -> int {
     if (!write) {
       if (int r = byte_layout(p) ? launch_potts_unpack(st, p0, n, dev, dtype, n, 0)
@@ -1966,9 +1946,9 @@ extern "C" int thrml_sample_states_as(thrml_prog *p, uint64_t key, thrml_schedul
   const Plan plan = schedule_plan(p, st, key, sched);
   // observations are gathered on the device and copied out several at a time,
   // so that the sweeps are not stopped for each of them
-  const uint64_t batch = std::max<uint64_t>(1, std::min<uint64_t>(plan.obs_after.size(), thrml_ctx::IO_KEEP / per));
-  Staging tmp;
-  if (int rc = tmp.get(p->ctx, batch * per)) return rc;
+  const uint64_t batch = std::max<uint64_t>(1, std::min<uint64_t>(plan.obs_after.size(), DevPool::LARGEST / per));
+  DevBuf tmp;
+  if (int rc = tmp.alloc_transfer(batch * per, &p->ctx->pool)) return rc;
   uint8_t *dst = static_cast<uint8_t *>(out);
   uint64_t held = 0;
   auto flush = [&]() -> int {
@@ -1989,7 +1969,7 @@ extern "C" int thrml_sample_states_as(thrml_prog *p, uint64_t key, thrml_schedul
   ks.grow = &p->ctx->keys;
   int rc = run_plan(p, st, plan, nullptr, obs, ks);
   if (!rc) rc = flush();
-  const hipError_t e = hipStreamSynchronize(p->ctx->stream);  // before the staging buffer is let go
+  const hipError_t e = hipStreamSynchronize(p->ctx->stream);  // the caller's memory is free again
   if (!rc && e != hipSuccess) return hip_fail(e, "observation transfer");
   return rc;
 }

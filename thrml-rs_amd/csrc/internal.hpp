@@ -57,9 +57,11 @@ struct ResPart {
 // states and moments anew then allocates nothing (a hipMalloc and hipFree pair
 // of more than 2 MiB takes 100-200 us).  All work of a context is ordered on
 // its stream, so a block may be taken again while the last kernels that use it
-// still run.  Bounded by KEEP bytes; emptied with the context and when its
+// still run.  Bounded by KEEP bytes; emptied with the context, when its
 // stream changes (blocks taken before that are then freed, not kept: their
-// last use may lie on the old stream).
+// last use may lie on the old stream) and when an allocation fails.  Beside
+// them one block of at most LARGEST bytes for host transfers, which come in any
+// size; a transfer that finds it taken by another thread's gets its own.
 class DevPool {
  public:
   static constexpr size_t KEEP = 256u << 20, LARGEST = 64u << 20;
@@ -84,6 +86,27 @@ class DevPool {
     held_ += cap;
     return true;
   }
+  // the transfer block if it is free and holds n bytes (a smaller one makes way
+  // for the larger that the caller now allocates)
+  void *take_transfer(size_t n, size_t *cap, uint64_t *era) {
+    std::lock_guard<std::mutex> lk(mu_);
+    *era = era_;
+    void *p = transfer_;
+    transfer_ = nullptr;
+    if (p && transfer_cap_ < n) {
+      (void)hipFree(p);
+      p = nullptr;
+    }
+    *cap = transfer_cap_;
+    return p;
+  }
+  bool give_transfer(void *p, size_t cap, uint64_t era) {
+    std::lock_guard<std::mutex> lk(mu_);
+    if (era != era_ || cap > LARGEST || transfer_) return false;
+    transfer_ = p;
+    transfer_cap_ = cap;
+    return true;
+  }
   void new_stream() {
     clear();
     std::lock_guard<std::mutex> lk(mu_);
@@ -94,12 +117,15 @@ class DevPool {
     for (auto &b : free_) (void)hipFree(b.second);
     free_.clear();
     held_ = 0;
+    if (transfer_) (void)hipFree(transfer_);
+    transfer_ = nullptr;
   }
 
  private:
   std::mutex mu_;
   std::multimap<size_t, void *> free_;
-  size_t held_ = 0;
+  void *transfer_ = nullptr;
+  size_t held_ = 0, transfer_cap_ = 0;
   uint64_t era_ = 0;
 };
 
@@ -113,9 +139,11 @@ struct DevBuf {
   DevBuf &operator=(const DevBuf &) = delete;
   ~DevBuf() { release(); }
   void release() {
-    if (p && !(pool_ && pool_->give(p, cap_, era_))) (void)hipFree(p);
+    if (p && !(pool_ && (transfer_ ? pool_->give_transfer(p, cap_, era_) : pool_->give(p, cap_, era_))))
+      (void)hipFree(p);
     p = nullptr;
     pool_ = nullptr;
+    transfer_ = false;
     bytes = cap_ = 0;
   }
   // n bytes, from the pool and back to it
@@ -126,6 +154,17 @@ struct DevBuf {
     if (!p)
       if (int rc = allocate(n, pool)) return rc;
     pool_ = pool;
+    bytes = n;
+    return THRML_OK;
+  }
+  // n bytes for a host transfer
+  int alloc_transfer(size_t n, DevPool *pool) {
+    release();
+    p = pool->take_transfer(n, &cap_, &era_);
+    if (!p)
+      if (int rc = allocate(std::max<size_t>(n, 1u << 16), pool)) return rc;
+    pool_ = pool;
+    transfer_ = true;
     bytes = n;
     return THRML_OK;
   }
@@ -161,6 +200,7 @@ struct DevBuf {
   }
 
   DevPool *pool_ = nullptr;
+  bool transfer_ = false;
   size_t cap_ = 0;
   uint64_t era_ = 0;
 };
@@ -211,12 +251,6 @@ struct thrml_ctx {
   thrml::DevBuf keys;
   std::mutex run_mu;
   thrml::DevPool pool;  // what this context's objects have let go of
-  // Staging of host transfers (state import and export, moment sums), grown as
-  // needed up to IO_KEEP bytes (larger transfers allocate their own).  io_mu is
-  // held from the transfer's first use of it until its stream work has ended.
-  static constexpr size_t IO_KEEP = 64u << 20;
-  thrml::DevBuf io;
-  std::mutex io_mu;
   int flush_timing(int k);
   int time_begin(int k, hipEvent_t *start);
   int time_end(int k, hipEvent_t start, uint64_t half_sweeps = 1);

@@ -8,6 +8,7 @@ import pytest
 
 import hostrun
 import thrml_hip as th
+from thrml_hip import _lib
 
 def _lattice(dev, L=64):
     n, edges, up, lo = th.make_nearest_neighbor_lattice(L, True)
@@ -106,6 +107,46 @@ def test_one_block_serves_transfers_of_every_size():
     assert grown == 16 << 20          # 32 MiB in place of 16
     assert end == 48 << 20            # 64 MiB in place of 16
     assert mallocs == 2
+
+
+def _moment_memory(L):
+    """Bytes of a spec of all nodes and edges of a torus, allocated at its creation, by
+    a run into device memory and by a run into host memory, and the
+    allocations that a second spec and run make."""
+    dev = th.Device(0)
+    prog = _lattice(dev, L)
+    st = prog.new_state(2)
+    n, edges, _, _ = th.make_nearest_neighbor_lattice(L, True)
+    fake = hostrun.fake
+    sched = th.SamplingSchedule(1, 1, 1)
+    th.run_blocks(th.RngKey(1), prog, st, (), 1)
+
+    def spec():
+        return th.MomentAccumulatorObserver(prog, th.ising_moment_spec(np.arange(n), edges))
+
+    steps = [fake.fake_live_bytes()]
+    m = spec()
+    steps.append(fake.fake_live_bytes())
+    sums = np.zeros(n + len(edges), np.int64)
+    _lib.check(_lib.load().thrml_moments_run(prog._h, 1, sched._c(), st._h, m._h, sums.ctypes.data,
+                                             sums.ctypes.data, 1))
+    steps.append(fake.fake_live_bytes())
+    m.sample_with_observation(th.RngKey(1), sched, st)
+    steps.append(fake.fake_live_bytes())
+    m.close()
+    before = fake.fake_mallocs()
+    m = spec()
+    m.sample_with_observation(th.RngKey(1), sched, st)
+    return np.diff(steps).tolist(), fake.fake_mallocs() - before
+
+
+def test_moment_specs_hold_host_sums_for_host_outputs_only():
+    n, e = 1024 * 1024, 2 * 1024 * 1024
+    steps, again = hostrun.call(_moment_memory, 1024)
+    # 12 bytes per counter and 4 per table entry; 8 per sum on the host, unless a
+    # kept block holds them
+    assert steps[:2] == [16 * (n + e), 0] and steps[2] in (0, 8 * (n + e))
+    assert again == 0  # below the pool's largest block
 
 
 def _graph():

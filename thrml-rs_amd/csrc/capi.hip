@@ -1713,16 +1713,15 @@ extern "C" int thrml_moments_create(thrml_prog *p, const uint32_t *nodes, uint64
   m->native = p->kind == K_LATTICE && lattice_pair_slots(p, ppos, pslot);
   m->len1 = m->native ? p->n_total : n1;
   m->len2 = m->native ? (uint64_t)p->L * p->half * 4u : n2;
-  // 8-byte parts first: output staging, totals, then counters, then the table
+  // totals, then counters, then the table
   const std::vector<uint32_t> &tab2 = m->native ? pslot : ppos;
   const size_t tab = (npos.size() + tab2.size()) * 4;
-  const size_t wide = (n1 + n2 + m->len1 + m->len2) * 8, cnt = (m->len1 + m->len2) * 4;
+  const size_t wide = (m->len1 + m->len2) * 8, cnt = (m->len1 + m->len2) * 4;
   if (int rc = m->buf.alloc(wide + cnt + tab, &p->ctx->pool)) {
     delete m;
     return rc;
   }
-  m->out = m->buf.as<int64_t>();
-  m->acc1 = reinterpret_cast<uint64_t *>(m->out + n1 + n2);
+  m->acc1 = m->buf.as<uint64_t>();
   m->acc2 = m->acc1 + m->len1;
   m->cnt1 = reinterpret_cast<uint32_t *>(m->acc2 + m->len2);
   m->cnt2 = m->cnt1 + m->len1;
@@ -1786,7 +1785,13 @@ extern "C" int thrml_moments_run(thrml_prog *p, uint64_t key, thrml_schedule sch
   ks.grow = &p->ctx->keys;
   int rc = run_plan(p, st, schedule_plan(p, st, key, sched), m->native ? &lm : nullptr, obs, ks);
   if (rc) return rc;
-  int64_t *o1 = out_on_device ? node_sums : m->out, *o2 = out_on_device ? pair_sums : m->out + m->n1;
+  int64_t *o1 = node_sums, *o2 = pair_sums;
+  if (!out_on_device) {
+    if (!m->out.p)
+      if ((rc = m->out.alloc((m->n1 + m->n2) * 8, &p->ctx->pool))) return rc;
+    o1 = m->out.as<int64_t>();
+    o2 = o1 + m->n1;
+  }
   const int64_t cn = (int64_t)st->C * (int64_t)n_obs;
   rc = launch_finalize_moments(p->ctx, c1, m->acc1, m->slot1, m->n1, c2, m->acc2, m->slot2, m->n2, cn, o1, o2);
   if (rc) return rc;

@@ -402,13 +402,13 @@ struct thrml_moments {
   uint64_t len1 = 0, len2 = 0;  // counters
   // one allocation: native, the counter index per requested entry (slot1,
   // slot2), else the positions of nodes and of pair endpoints (npos, ppos);
-  // u32 counters of the current fold period, u64 totals, host-output staging
+  // u32 counters of the current fold period, u64 totals
   thrml::DevBuf buf;
   uint32_t *slot1 = nullptr, *slot2 = nullptr, *npos = nullptr, *ppos = nullptr;
   uint32_t *cnt1 = nullptr, *cnt2 = nullptr;
   uint64_t *acc1 = nullptr, *acc2 = nullptr;
-  int64_t *out = nullptr;
   size_t clear_bytes = 0;       // totals and counters, from acc1 on
+  thrml::DevBuf out;            // the sums of a run whose outputs lie on the host, from the first one on
 };
 
 // A general moment observer (MomentAccumulatorObserver with any spec): row r

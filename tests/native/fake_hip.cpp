@@ -125,6 +125,9 @@ hipError_t hipGetLastError() {
   last = hipSuccess;
   return e;
 }
+const char *hipGetErrorString(hipError_t e) {
+  return e == hipSuccess ? "no error" : e == hipErrorOutOfMemory ? "out of memory" : "error";
+}
 hipError_t hipMalloc(void **p, size_t n) {
   std::lock_guard<std::mutex> lk(mu);
   ++n_malloc;

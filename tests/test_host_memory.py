@@ -1,6 +1,7 @@
 """Device memory and waits of the library's host code, against a stand-in of the
 HIP runtime (hostrun.py): no GPU is used and no kernel runs."""
 import ctypes
+import os
 import threading
 
 import numpy as np
@@ -147,6 +148,18 @@ def test_moment_specs_hold_host_sums_for_host_outputs_only():
     # kept block holds them
     assert steps[:2] == [16 * (n + e), 0] and steps[2] in (0, 8 * (n + e))
     assert again == 0  # below the pool's largest block
+
+
+def _stream_changes():
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(hostrun.FAKE), "libpooltest.so"))
+    lib.pool_kept_across_stream_change.restype = ctypes.c_uint64
+    return lib.pool_kept_across_stream_change(ctypes.c_uint64(20000))
+
+
+def test_memory_of_the_old_stream_is_not_kept():
+    """A buffer whose last use lies on the old stream is never handed to an object
+    on the new one, also when it is let go of while the stream changes."""
+    assert hostrun.call(_stream_changes) == 0
 
 
 def _graph():

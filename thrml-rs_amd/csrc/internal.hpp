@@ -107,13 +107,19 @@ class DevPool {
     transfer_cap_ = cap;
     return true;
   }
+  // (at once: a block given back in between would be kept for the new stream)
   void new_stream() {
-    clear();
     std::lock_guard<std::mutex> lk(mu_);
+    empty();
     ++era_;
   }
   void clear() {
     std::lock_guard<std::mutex> lk(mu_);
+    empty();
+  }
+
+ private:
+  void empty() {
     for (auto &b : free_) (void)hipFree(b.second);
     free_.clear();
     held_ = 0;
@@ -121,7 +127,6 @@ class DevPool {
     transfer_ = nullptr;
   }
 
- private:
   std::mutex mu_;
   std::multimap<size_t, void *> free_;
   void *transfer_ = nullptr;

@@ -1,0 +1,30 @@
+"""Which kernels a call launches, and which sizes it refuses, against a stand-in of
+the HIP runtime (hostrun.py): no GPU is used and no kernel runs."""
+import numpy as np
+import pytest
+
+import hostrun
+import thrml_hip as th
+
+
+def _spin_factor_run(sites, chains):
+    """The spin kernel's launches of one sweep over one block, or the error."""
+    dev = th.Device(0)
+    prog = th.FactorSamplingProgram(np.zeros(sites, np.uint8), 2, [th.SpinEBMFactor([np.arange(sites)], np.zeros(sites))],
+                                    [np.arange(sites)], [], dev)
+    st = prog.new_state(chains)
+    hostrun.clear_launches()
+    try:
+        th.run_blocks(th.RngKey(1), prog, st, (), 1)
+    except th.ThrmlError as e:
+        return str(e)
+    return hostrun.launches().get("discrete_spin_kernel<unsigned_char>", 0)
+
+
+@pytest.mark.parametrize("sites,chains,runs", [(16148, 531900, True), (16145, 531900, True), (16149, 531900, False),
+                                               (1, 699000, True), (13, 660000, True)])
+def test_spin_factor_block_limit(sites, chains, runs):
+    """(sites / 4) x chains below 2^31, whatever the sites are modulo 16."""
+    assert ((sites + 3) // 4 * chains < 1 << 31) == runs
+    got = hostrun.call(_spin_factor_run, sites, chains)
+    assert got == 1 if runs else "must stay below 2^31" in got

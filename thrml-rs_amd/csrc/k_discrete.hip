@@ -510,8 +510,8 @@ int launch_discrete_half(thrml_prog *p, thrml_state *st, uint32_t b, const uint3
   // (parts start on a wave boundary, so that a wave holds one part)
   const uint64_t runs = (uint64_t)cdiv32(n_b, SG) * st->C;
   const uint64_t per = NP > 1 ? (runs + 63u) & ~63ull : runs;
-  // (a spin run takes four lanes: the launch itself stays below 2^32 threads)
-  if (per * (spin ? 4u : NP) >= (1ull << 31))
+  // (a spin run takes four lanes, one for every 4 of its sites)
+  if ((spin ? (uint64_t)cdiv32(n_b, 4) * st->C : per * NP) >= (1ull << 31))
     return fail(THRML_EINVAL, "block too large: (sites / runs) x chains must stay below 2^31");
   a.items_per_part = (uint32_t)per;
   a.n_items = (uint32_t)(per * NP);

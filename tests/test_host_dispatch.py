@@ -28,3 +28,21 @@ def test_spin_factor_block_limit(sites, chains, runs):
     assert ((sites + 3) // 4 * chains < 1 << 31) == runs
     got = hostrun.call(_spin_factor_run, sites, chains)
     assert got == 1 if runs else "must stay below 2^31" in got
+
+
+def _potts_run(q, sites, chains):
+    dev = th.Device(0)
+    prog = th.CategoricalProgram(sites, q, np.zeros((0, 2)), np.zeros((0, q, q)), np.zeros((sites, q)),
+                                 [np.arange(sites)], dev)
+    st = prog.new_state(chains)
+    hostrun.clear_launches()
+    th.run_blocks(th.RngKey(1), prog, st, (), 1)
+    return {k: n for k, n in hostrun.launches().items() if k.startswith("potts")}
+
+
+@pytest.mark.parametrize("sites,chains,lanes", [(3906, 549791, 1), (3906, 549759, 2)])
+def test_wide_categorical_block_limit(sites, chains, lanes):
+    """Up to 2^31 - 1 (site, chain) items run; two lanes each, where that is the
+    faster, while whole workgroups of them stay below 2^32 threads."""
+    assert sites * chains in ((1 << 31) - 2, (1 << 31) - 2 - 32 * 3906)
+    assert hostrun.call(_potts_run, 32, sites, chains) == {f"potts_wide_kernel<unsigned_char,{lanes}>": 1}

@@ -595,7 +595,7 @@ inline uint32_t wide_lanes(uint32_t q, uint64_t items, uint32_t slots) {
   uint32_t best = 1u;
   double best_t = 0.0;
   for (uint32_t P = 1; P <= (q > 256u ? 64u : 16u); P *= P == 16u ? 4u : 2u) {
-    if (items * P >= (1ull << 32)) break;  // lanes are indexed in 32 bits
+    if (items * P > (1ull << 32) - 256u) break;  // a launch, whole workgroups, stays below 2^32 threads
     double steps = 0.0;
     for (uint32_t o = 0; o < 16u; o += step) steps += (double)(((o + q + 15u) / 16u + P - 1u) / P);
     steps /= 16u / step;

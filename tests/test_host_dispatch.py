@@ -46,3 +46,46 @@ def test_wide_categorical_block_limit(sites, chains, lanes):
     faster, while whole workgroups of them stay below 2^32 threads."""
     assert sites * chains in ((1 << 31) - 2, (1 << 31) - 2 - 32 * 3906)
     assert hostrun.call(_potts_run, 32, sites, chains) == {f"potts_wide_kernel<unsigned_char,{lanes}>": 1}
+
+
+def _ising_kernels(prog, C, sched, cus=256):
+    """The sweep kernels that a run with moments launches."""
+    st = prog.new_state(C)
+    m = th.MomentAccumulatorObserver(prog, th.ising_moment_spec([0], np.zeros((0, 2))))
+    hostrun.clear_launches()
+    m.sample_with_observation(th.RngKey(1), th.SamplingSchedule(*sched), st)
+    return sorted(k for k in hostrun.launches() if "half" in k or k.startswith("resident") and "commit" not in k)
+
+
+def _one_block_of_many(clamped, C):
+    """512 free sites with 60 neighbours each among `clamped` clamped ones."""
+    rng = np.random.default_rng(0)
+    e = np.stack([np.repeat(np.arange(512), 60), 512 + rng.integers(0, clamped, 512 * 60)], axis=1)
+    e = np.unique(e, axis=0).astype(np.uint32)
+    n = 512 + clamped
+    prog = th.IsingSamplingProgram(th.IsingEBM(n, e, np.zeros(n), np.zeros(len(e))), [np.arange(512)],
+                                   [np.arange(512, n)], th.Device(0))
+    return _ising_kernels(prog, C, (2, 30, 2))
+
+
+@pytest.mark.parametrize("clamped,C,resident", [(20000, 256, True), (20000, 260, True), (54000, 256, True),
+                                                (54000, 260, False)])
+def test_resident_workgroups_that_lds_keeps_apart(clamped, C, resident):
+    """Chains beyond one per compute unit cost a second turn where two
+    workgroups' states and keystreams (n + 64 bytes per thread) do not fit one unit's LDS."""
+    k = hostrun.call(_one_block_of_many, clamped, C)
+    assert [x.startswith("resident") for x in k] == [resident], k
+
+
+def _lattice_on(cus, C):
+    hostrun.fake.fake_set_cus(cus)
+    n, edges, up, lo = th.make_nearest_neighbor_lattice(64, True)
+    prog = th.IsingSamplingProgram(th.IsingEBM(n, edges, np.zeros(n), np.zeros(len(edges)), 1.0), [up, lo], [],
+                                   th.Device(0))
+    return _ising_kernels(prog, C, (500, 1, 1))
+
+
+@pytest.mark.parametrize("cus,C,resident", [(256, 256, True), (32, 32, True), (32, 256, False)])
+def test_resident_turns_count_the_compute_units(cus, C, resident):
+    k = hostrun.call(_lattice_on, cus, C)
+    assert [x.startswith("resident") for x in k] == [resident], k

@@ -585,6 +585,9 @@ int resident_tables(thrml_prog *p, const std::vector<uint32_t> &row_off, const u
   return THRML_OK;
 }
 
+// LDS of a workgroup: the state, and a keystream block per thread.
+static size_t res_lds(const thrml_prog *p) { return ((p->n_total + 16u) & ~15ull) + (size_t)p->res_T * 64u; }
+
 // Whether n_seg segments (runs of sweeps between observations) of n_sweeps
 // sweeps in all go faster resident than block by block; fused: the lattice
 // kernel would count the observations itself.  Both sides are fits, in us, to
@@ -609,8 +612,10 @@ bool resident_pays(const thrml_prog *p, const thrml_state *st, uint64_t n_sweeps
                    bool fused) {
   if (!p->res_T) return false;
   const double C = st->C, G = st->G;
-  // workgroups of at most 512 threads share a CU
-  const double rounds = p->res_T > 512u ? std::ceil(C / 256.0) : std::max(1.0, C / 256.0);
+  // workgroups of at most 512 threads share a CU, if its LDS holds two of them
+  const double turns = C / p->ctx->cu_count;
+  const bool shared = p->res_T <= 512u && 2u * res_lds(p) <= (size_t)RES_LDS;
+  const double rounds = shared ? std::max(1.0, turns) : std::ceil(turns);
   const double res = 0.35 * p->n_free + rounds * p->res_work;
   double blk = 0.0;
   for (uint32_t b = 0; b < p->n_free; ++b) {
@@ -645,13 +650,12 @@ int launch_resident(thrml_prog *p, thrml_state *st, const uint32_t *d_keys, uint
   a.n_parts = p->res_parts;
   a.div_kb = make_fastdiv(p->res_kb);
   a.per_phase = p->res_parts == 1u ? p->res_T / p->res_kb : 1u;
-  const size_t lds = ((a.n_total + 16u) & ~15u) + (size_t)p->res_T * 64u;
   hipStream_t s = p->ctx->stream;
   hipEvent_t t0 = nullptr;
   if (p->ctx->time_begin(0, &t0)) return THRML_EHIP;
   void *args[] = {&a};
   THRML_HIP(hipLaunchKernel(p->res_ent ? reg_kernel(p->res_ent) : stream_kernel(p->res_pf), dim3(st->C),
-                            dim3(p->res_T), args, lds, s));
+                            dim3(p->res_T), args, res_lds(p), s));
   if (st->C > 1u) {
     const uint32_t n_tasks = a.n_words * st->G;
     hipLaunchKernelGGL(resident_commit_kernel, dim3((n_tasks + 3u) / 4u), dim3(256), 0, s, a.bits,

@@ -65,7 +65,7 @@ def _one_block_of_many(clamped, C):
     n = 512 + clamped
     prog = th.IsingSamplingProgram(th.IsingEBM(n, e, np.zeros(n), np.zeros(len(e))), [np.arange(512)],
                                    [np.arange(512, n)], th.Device(0))
-    return _ising_kernels(prog, C, (2, 30, 2))
+    return _ising_kernels(prog, C, (10, 30, 10))
 
 
 @pytest.mark.parametrize("clamped,C,resident", [(20000, 256, True), (20000, 260, True), (54000, 256, True),
@@ -74,7 +74,7 @@ def test_resident_workgroups_that_lds_keeps_apart(clamped, C, resident):
     """Chains beyond one per compute unit cost a second turn where two
     workgroups' states and keystreams (n + 64 bytes per thread) do not fit one unit's LDS."""
     k = hostrun.call(_one_block_of_many, clamped, C)
-    assert [x.startswith("resident") for x in k] == [resident], k
+    assert {x.startswith("resident") for x in k} == {resident}, k
 
 
 def _lattice_on(cus, C):
@@ -88,4 +88,38 @@ def _lattice_on(cus, C):
 @pytest.mark.parametrize("cus,C,resident", [(256, 256, True), (32, 32, True), (32, 256, False)])
 def test_resident_turns_count_the_compute_units(cus, C, resident):
     k = hostrun.call(_lattice_on, cus, C)
-    assert [x.startswith("resident") for x in k] == [resident], k
+    assert {x.startswith("resident") for x in k} == {resident}, k
+
+
+def _few_sites(free, clamped, C, sched):
+    rng = np.random.default_rng(0)
+    e = np.stack([np.repeat(np.arange(free), 6), free + rng.integers(0, clamped, free * 6)], axis=1)
+    e = np.unique(e, axis=0).astype(np.uint32)
+    n = free + clamped
+    prog = th.IsingSamplingProgram(th.IsingEBM(n, e, np.zeros(n), np.zeros(len(e))), [np.arange(free)],
+                                   [np.arange(free, n)], th.Device(0))
+    return _ising_kernels(prog, C, sched)
+
+
+def _random_graph(n, C, sched):
+    e = th.erdos_renyi(n, 6.0 / (n - 1), 3)
+    prog = th.IsingSamplingProgram(th.IsingEBM(n, e, np.zeros(n), np.zeros(len(e))),
+                                   th.coloring_to_blocks(th.greedy_coloring(n, e)), [], th.Device(0))
+    return _ising_kernels(prog, C, sched)
+
+
+@pytest.mark.parametrize("f,args,resident", [
+    # measured, us per segment:                     whole, block by block
+    (_few_sites, (64, 1000, 32, (5, 10, 5)), True),        # 17, 27
+    (_few_sites, (64, 60000, 32, (10, 10, 10)), False),    # 360, 51
+    (_few_sites, (64, 60000, 32, (200, 3, 200)), True),    # 442, 980
+    (_few_sites, (512, 60000, 256, (5, 10, 5)), False),    # 62, 29
+    (_few_sites, (2048, 1000, 32, (10, 10, 10)), True),    # 27, 52
+    (_random_graph, (60000, 200, (1, 10, 1)), False),      # 96, 85
+    (_random_graph, (20000, 200, (4, 10, 4)), True),       # 101, 211
+])
+def test_a_segment_costs_its_way_into_and_out_of_lds(f, args, resident):
+    """Every run between observations moves the whole state, clamped positions
+    too, with the lanes of its largest block."""
+    k = hostrun.call(f, *args)
+    assert {x.startswith("resident") for x in k} == {resident}, k

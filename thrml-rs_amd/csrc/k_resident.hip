@@ -592,43 +592,52 @@ static size_t res_lds(const thrml_prog *p) { return ((p->n_total + 16u) & ~15ull
 // sweeps in all go faster resident than block by block; fused: the lattice
 // kernel would count the observations itself.  Both sides are fits, in us, to
 // run times on MI355X (tori of side 10 .. 256, Erdos-Renyi graphs of 200 ..
-// 60000 nodes and mean degree 4 .. 12, double grids; 1 .. 1024 chains).
-// Resident: per sweep 0.35 per block and 0.0068 per (pair + 5) of the entries
-// (0.0145 or 0.025 per slice from registers), one chain per CU at a time, and
-// about 9 per segment for its two launches and the way into and out of LDS
-// (13 where a launch for the observation comes on top).  Block by block: a
-// launch takes 2.4 on a lattice, 3.4 (7 with 16-site runs) and more with the
-// degree otherwise, and grows with the sites times the chain groups.
-//   us per sweep           resident  block by block
-//   64^2, C = 1                 1.5   4.9
-//   64^2, C = 1024              6.8   6.6
-//   96^2, C = 256               4.5   6.5
-//   128^2, C = 64               9.5   5.4
-//   E-R 20K deg 7, C = 200       23    48
-//   E-R 50K deg 6, C = 32        48    32
-//   E-R 50K deg 6, C = 512       97    90
-//   grid 2 x 40^2, C = 1        4.1   8.0
+// 60000 nodes and mean degree 4 .. 12, double grids, 64 .. 2048 free sites among
+// 1000 .. 60000 clamped ones; 1 .. 1024 chains).
+// Resident, per sweep: 0.35 per block and 0.0068 per (pair + 5) of the entries
+// (0.0145 or 0.025 per slice from registers), for every turn of the chains over
+// the CUs.  Per segment: 6.5 for its two launches (4 for one chain's single
+// one) and 0.38 (0.19) for each step of the workgroup over all positions, on the
+// way into and out of LDS; where a launch for the observation comes on top, 3 and
+// 0.2 per 1000 words of the state.  Block by block: a launch takes 3.2 on a lattice
+// (between 2.4 and 4.1, by the host), 4.0 (7.6 with 16-site runs) and more with
+// the degree otherwise, and grows with the sites times the chain groups.
+//   us per sweep, + per segment beyond an observation   resident    block by block
+//   64^2, C = 1                                         1.6 + 7.8   4.9-8.3
+//   64^2, C = 512                                       3.3 + 21    7.6
+//   96^2, C = 256                                       4.3 + 18    6.5-9.3
+//   128^2, C = 64                                       9.5         5.4
+//   E-R 20K deg 6, C = 200                              21 + 15     52
+//   E-R 60K deg 6, C = 200                              56 + 35     80
+//   E-R 60K deg 6, C = 512                              113 + 66    101
+//   grid 2 x 40^2, C = 1                                4.1         8.0
+//   64 sites + 1000 clamped, C = 32                     0.43 + 13   5.0
+//   64 sites + 60000 clamped, C = 32                    0.43 + 353  4.9
+//   2048 sites + 60000 clamped, C = 256                 1.7 + 37    5.7
 bool resident_pays(const thrml_prog *p, const thrml_state *st, uint64_t n_sweeps, uint64_t n_seg,
                    bool fused) {
   if (!p->res_T) return false;
   const double C = st->C, G = st->G;
-  // workgroups of at most 512 threads share a CU, if its LDS holds two of them
-  const double turns = C / p->ctx->cu_count;
-  const bool shared = p->res_T <= 512u && 2u * res_lds(p) <= (size_t)RES_LDS;
-  const double rounds = shared ? std::max(1.0, turns) : std::ceil(turns);
+  // workgroups of at most 512 threads share a CU, as many as its LDS holds
+  const double per_cu = p->res_T > 512u ? 1.0 : (double)std::min<size_t>(2048u / p->res_T, (size_t)RES_LDS / res_lds(p));
+  const double turns = std::ceil(C / (p->ctx->cu_count * per_cu));
+  const double rounds = per_cu > 1.0 ? std::max(1.0, C / p->ctx->cu_count) : turns;
   const double res = 0.35 * p->n_free + rounds * p->res_work;
+  const double steps = std::ceil((double)p->n_total / p->res_T);
+  const double seg = (C > 1.0 ? 6.5 + 0.38 * turns * steps : 4.0 + 0.19 * steps) +
+                     (fused ? 3.0 + 0.2e-3 * (double)p->n_total * G : 0.0);
   double blk = 0.0;
   for (uint32_t b = 0; b < p->n_free; ++b) {
     const double n = (double)(p->blk_off[b + 1] - p->blk_off[b]);
     if (p->kind == K_LATTICE) {
-      blk += std::max(2.4, 1.0 + n * G * 0.05e-3);
+      blk += std::max(3.2, 1.0 + n * G * 0.05e-3);
     } else {
       const double deg = p->res_deg;
       const bool run16 = C > 32.0 && std::ceil(n / 16.0) * G >= 4096.0;  // as launch_csr_half
-      blk += 0.1 * deg + (run16 ? 7.0 + n * G * 0.11e-3 : 3.4 + n * (C <= 32.0 ? 0.06e-3 : (G - 0.5) * 0.22e-3));
+      blk += 0.1 * deg + (run16 ? 7.6 + n * G * 0.11e-3 : 4.0 + n * (C <= 32.0 ? 0.06e-3 : (G - 0.5) * 0.22e-3));
     }
   }
-  return res * (double)n_sweeps + (fused ? 13.0 : 9.0) * (double)n_seg < 0.95 * blk * (double)n_sweeps;
+  return res * (double)n_sweeps + seg * (double)n_seg < 0.95 * blk * (double)n_sweeps;
 }
 
 int launch_resident(thrml_prog *p, thrml_state *st, const uint32_t *d_keys, uint32_t n_sweeps) {

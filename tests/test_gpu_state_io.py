@@ -7,6 +7,7 @@ from memory that earlier ones let go of start clean."""
 import numpy as np
 import pytest
 
+import pyoracle as orc
 import thrml_hip as th
 from conftest import log_case
 
@@ -98,18 +99,21 @@ def test_mixed_state_checks_each_block(device):
 
 
 def test_observations_in_several_transfers(device):
-    """More observations than the staging buffer holds at once."""
+    """More observations than one transfer holds (64 MiB: 29 of 33 here), every one
+    of them against the oracle."""
     log_case("observations in several transfers")
-    prog = _ising(2048, device)
-    st = th.hinton_init(th.RngKey(3), prog, 1100)  # 2.25 MB per observation, 64 MiB kept
+    n, C = 2048, 1100  # 2.25 MB per observation
+    prog = _ising(n, device)
+    st = th.hinton_init(th.RngKey(3), prog, C)
+    init = st.get_global()
     out = th.sample_states(th.RngKey(4), prog, th.SamplingSchedule(0, 33, 1), st)
-    ref = th.hinton_init(th.RngKey(3), prog, 1100)
-    assert np.array_equal(out[0], ref.get_global())
-    assert np.array_equal(out[-1], st.get_global())
-    wk, sk = th.RngKey(4).split_two()
-    for i, k in enumerate(sk.split(32)):
-        th.run_blocks(k, prog, ref, (), 1)
-    assert out.shape[0] == 33 and all(out[i].any() for i in range(33))
+    assert out.shape == (33, C, n) and 29 * C * n < 64 << 20 < 30 * C * n
+    e = np.stack([np.arange(n - 1), np.arange(1, n)], axis=1)
+    o = orc.Ising(n, e, np.zeros(n), np.zeros(n - 1), 1.0, [np.arange(0, n, 2), np.arange(1, n, 2)])
+    want = o.sample_states(4, (0, 33, 1), init)
+    for i in range(33):
+        assert np.array_equal(out[i], want[i]), f"observation {i} differs"
+    assert np.array_equal(st.get_global(), want[-1])
 
 
 def test_memory_is_kept_within_one_stream(device):

@@ -146,8 +146,14 @@ def test_weight_pieces_found_on_the_device(device):
             th.RbmProgram(w, bv, bh, 1.0, device)
 
 
+# V, H, chains of the kernel for few tiles, and chains beyond it whatever V and H
+# (test_host_dispatch.py holds the launches to these)
+SMALL_TILES = [(1, 15, 1), (16, 33, 63), (31, 257, 64), (200, 64, 65), (300, 1100, 130)]
+LARGE_TILES_C = 97 * 256
+
+
 @pytest.mark.parametrize("f32", [False, True])
-@pytest.mark.parametrize("V,H,C", [(1, 15, 1), (16, 33, 63), (31, 257, 64), (200, 64, 65), (300, 1100, 130)])
+@pytest.mark.parametrize("V,H,C", SMALL_TILES)
 def test_small_tiles_equal_large_tiles(device, V, H, C, f32):
     """The kernel for products of few tiles against the one for many: the
     first C chains of a state large enough for the latter, from the same keys
@@ -160,7 +166,7 @@ def test_small_tiles_equal_large_tiles(device, V, H, C, f32):
     W = W if f32 else th.bf16_round(W)[0]
     bv, bh = rng.normal(0, 0.3, V), rng.normal(0, 0.3, H)
     prog = th.RbmProgram(W, bv, bh, 0.9, device)
-    big_c = 97 * 256  # more tiles than the small kernel takes, whatever V and H
+    big_c = LARGE_TILES_C
     small, big = prog.new_state(C), prog.new_state(big_c)
     x = rng.integers(0, 2, (big_c, V + H)).astype(np.uint8)
     small.set_global(x[:C])

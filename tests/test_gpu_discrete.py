@@ -118,11 +118,14 @@ def test_more_than_256_categories_mixed_model(device, q, C, m):
     _parity(prog, o, init, 19, 3)
 
 
-def test_wave_and_lane_factor_kernels_either_side_of_the_choice(device):
-    """q = 300 categorical blocks of 4096 sites on either side of the wave /
-    lane kernel choice (16 chains: 65,536 items per block on the wave kernel;
-    20 chains: 81,920 on the lane kernel), with spin nodes coupled to some of
-    them (two-byte spin tails), each against the oracle."""
+# chains -> lanes per item, on either side of two changes (test_host_dispatch.py
+# holds the launches to these)
+FACTOR_LANES = {2: 16, 3: 8, 10: 8, 12: 4}
+
+
+def wide_factor_model():
+    """(kinds, q, factors, free blocks): q = 300 categorical blocks of 4096 sites,
+    and spin nodes coupled to some of them (two-byte spin tails)."""
     q, n_spin, n_cat = 300, 64, 8192
     n = n_spin + n_cat
     rng = np.random.default_rng(3)
@@ -131,10 +134,17 @@ def test_wave_and_lane_factor_kernels_either_side_of_the_choice(device):
     factors = [([S], [], rng.normal(0, 0.5, (n_spin, 1, 1)).astype(np.float32)),
                ([], [X], rng.normal(0, 1.0, (n_cat, q, 1)).astype(np.float32)),
                ([S], [X[:n_spin]], rng.normal(0, 0.8, (n_spin, q, 1)).astype(np.float32))]
-    free = [S, X[0::2], X[1::2]]
-    prog, o = _programs(device, n, kinds, q, factors, free)
-    for C in (16, 20):
-        log_case(f"discrete q=300 wave/lane choice C={C}")
+    return kinds, q, factors, [S, X[0::2], X[1::2]]
+
+
+def test_factor_lane_counts_either_side_of_a_change(device):
+    """Chain counts on either side of two changes of the number of lanes per
+    (site, chain) item, each against the oracle."""
+    kinds, q, factors, free = wide_factor_model()
+    prog, o = _programs(device, kinds.size, kinds, q, factors, free)
+    rng = np.random.default_rng(4)
+    for C in FACTOR_LANES:
+        log_case(f"discrete q=300 lanes C={C}")
         init = _init(rng, kinds, q, C, free)
         st = prog.new_state(C)
         st.set_global(init)

@@ -371,12 +371,13 @@ def test_sample_states_u8_refuses_more_than_256_categories(device):
     st.close()
 
 
-@pytest.mark.parametrize("C,n_pairs", [(1, 7), (64, 70), (129, 70), (700, 70), (2100, 3),
-                                       (2, (1 << 20) + 5), (70, (1 << 20) - 3)])
+@pytest.mark.parametrize("C,n_pairs", [(1, 7), (64, 70), (129, 70), (700, 70), (2100, 3), (2100, 8058),
+                                       (2100, 16250), (2100, 70001), (70, (1 << 18) - 3)])
 def test_moment_sums_over_splits(device, C, n_pairs):
-    """Moment sums with one to 32 threads per item (1 to 33 chain groups) and,
-    from 2^20 items on, four items per thread: odd chain counts and remainders
-    of items, the nodes' end inside a turn of the pairs."""
+    """Moment sums with one to 32 threads per item: by the chain groups (1 to 33)
+    and, with many, by the items (up to 2^18 threads: 32, 16, 4 and 1 per item
+    in the last four cases); odd chain counts and remainders of items, the nodes' end
+    inside a workgroup."""
     ebm, blocks = wl.lattice_ising(20, 0.2, 0.3, 0.1)
     prog = th.IsingSamplingProgram(ebm, blocks, [], device)
     o = orc.Ising(ebm.n_nodes, ebm.edges, ebm.biases, ebm.weights, ebm.beta,

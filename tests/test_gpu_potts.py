@@ -173,8 +173,8 @@ def test_more_than_256_categories_parity(device, q, C, kind):
     any q): the wide kernels' sweeps equal the oracle's, with a superblock
     whose blocks hold edges between their own sites (staged writes) and
     with a clamped block; states read back as uint16.  3100 chains put
-    74,400 items in a block, which run on the lane kernel; the other cases
-    on the wave kernel."""
+    74,400 items in a block, which take fewer lanes each than the other
+    cases' items."""
     log_case(f"potts q={q} C={C} {kind}")
     n = 48
     rng, edges, W, bias = _ring(n, q, q + C)
@@ -236,7 +236,7 @@ def test_largest_category_counts(device, q, n, edged):
                                       (1027, 5, "ring"), (3000, 3, "inf")])
 def test_wave_kernel_parity(device, q, C, kind):
     """Blocks of few (site, chain) items for their categories run one wave
-    per item (potts_wave_kernel: the lanes split the site's keystream blocks
+    per item (the lanes split the site's keystream blocks
     and merge their top two scores): q a multiple of
     16, 4 and 2, and odd; a superblock with edges inside its blocks (staged
     writes), a clamped block, and a bias of +inf (the exact rescoring path
@@ -268,22 +268,29 @@ def test_wave_kernel_parity(device, q, C, kind):
     st.close()
 
 
-@pytest.mark.parametrize("q,Cs", [(300, (16, 20)), (1040, (4, 10))])
-def test_wave_and_lane_kernels_either_side_of_the_choice(device, q, Cs):
-    """Bias-only blocks of 4096 sites on either side of the wave / lane
-    kernel choice (q = 300: 65,536 items per block on the wave kernel,
-    81,920 on the lane kernel; q = 1040, 66 keystream blocks a site: 16,384
-    and 40,960), each against the oracle."""
+# q: chains -> lanes per item, on either side of two changes each
+# (test_host_dispatch.py holds the launches to these)
+BIAS_ONLY_LANES = {300: {6: 8, 8: 4, 40: 4, 48: 2}, 1040: {6: 16, 8: 8, 28: 8, 32: 2}}
+
+
+def bias_only_program(device, q):
     n = 8192
-    rng = np.random.default_rng(q)
-    bias = rng.normal(0, 1.0, (n, q)).astype(np.float32)
+    bias = np.random.default_rng(q).normal(0, 1.0, (n, q)).astype(np.float32)
     blocks = [np.arange(0, n, 2), np.arange(1, n, 2)]
-    no_e, no_w = np.zeros((0, 2), np.uint32), np.zeros((0, q, q), np.float32)
-    prog = th.CategoricalProgram(n, q, no_e, no_w, bias, blocks, device)
-    o = orc.Potts(n, q, no_e, no_w, bias, blocks)
-    for C in Cs:
+    args = (n, q, np.zeros((0, 2), np.uint32), np.zeros((0, q, q), np.float32), bias, blocks)
+    return th.CategoricalProgram(*args, device), args
+
+
+@pytest.mark.parametrize("q", BIAS_ONLY_LANES)
+def test_lane_counts_either_side_of_a_change(device, q):
+    """Bias-only blocks of 4096 sites with chain counts on either side of two
+    changes of the number of lanes per item, each against the oracle."""
+    prog, args = bias_only_program(device, q)
+    o = orc.Potts(*args)
+    rng = np.random.default_rng(q + 1)
+    for C in BIAS_ONLY_LANES[q]:
         log_case(f"potts q={q} bias-only C={C}")
-        init = rng.integers(0, q, (C, n)).astype(np.uint16)
+        init = rng.integers(0, q, (C, prog.n_total)).astype(np.uint16)
         st = prog.new_state(C)
         st.set_global(init)
         th.run_blocks(th.RngKey(C), prog, st, (), 2)

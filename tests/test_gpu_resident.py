@@ -55,35 +55,59 @@ def _bipartite_clamped(n, degree):
     return 3 * n, e, [th.Block(a), th.Block(c)], [th.Block(b)]
 
 
+def _regular(n, degree):
+    """Two bands of n sites with `degree` neighbours each in the other."""
+    i = np.arange(n)
+    e = np.concatenate([np.stack([i, n + (i + 37 * k) % n], axis=1) for k in range(degree)])
+    return 2 * n, e.astype(np.uint32), [th.Block(i), th.Block(n + i)], []
+
+
+# name, graph, chains, sweeps, kernel (test_host_dispatch.py holds the launches to it)
 CASES = [
-    ("one wave", _torus(10), 1, 40),
-    ("one wave, 65 chains", _torus(4), 65, 300),
-    ("register kernel, 2 entries", _torus(32), 64, 37),
-    ("register kernel, 4 entries", _torus(64), 3, 19),
-    ("register kernel, 6 entries", _torus(74), 2, 9),
-    ("register kernel, 10 entries", _torus(96), 2, 9),
-    ("streaming kernel, 4 slots, several parts", _torus(140), 200, 5),
-    ("no edges", _sparse(77, 0), 5, 21),
-    ("odd slot counts", _sparse(501, 3.0), 7, 33),
-    ("several entries per slice", _sparse(700, 14.0, hub=90), 9, 12),
-    ("wide slices", _sparse(1030, 22.0), 2, 9),
-    ("several parts, ragged", _sparse(17011, 5.0), 130, 4),
-    ("more blocks than waves", _ring(600, 30), 4, 17),
-    ("uneven blocks", _ring(1023, 3), 2, 70),
-    ("clamped block between", _bipartite_clamped(300, 3), 6, 25),
+    ("one wave", _torus(10), 1, 40, "reg_kernel<2>"),
+    ("one wave, 65 chains", _torus(4), 65, 300, "reg_kernel<2>"),
+    ("register kernel, 2 entries", _torus(32), 64, 37, "reg_kernel<2>"),
+    ("register kernel, 4 entries", _torus(64), 3, 19, "reg_kernel<4>"),
+    ("register kernel, 6 entries", _torus(74), 2, 9, "reg_kernel<10>"),
+    ("register kernel, 8 entries", _torus(80), 2, 60, "reg_kernel<10>"),
+    ("register kernel, 10 entries", _torus(96), 2, 60, "reg_kernel<10>"),
+    ("streaming kernel, 4 slots, several parts", _torus(140), 200, 5, "stream_kernel<2>"),
+    ("no edges", _sparse(77, 0), 5, 21, "reg_kernel<2>"),
+    ("odd slot counts", _sparse(501, 3.0), 7, 33, "stream_kernel<5>"),
+    ("several entries per slice", _sparse(700, 14.0, hub=90), 9, 12, "stream_kernel<8>"),
+    ("wide slices", _sparse(1030, 22.0), 2, 9, "stream_kernel<8>"),
+    ("eight slots", _regular(130, 8), 3, 14, "stream_kernel<4>"),
+    ("twelve slots", _regular(1100, 12), 2, 14, "stream_kernel<6>"),
+    ("fourteen slots", _regular(640, 14), 65, 14, "stream_kernel<7>"),
+    ("several parts, ragged", _sparse(17011, 5.0), 130, 4, "stream_kernel<3>"),
+    ("more blocks than waves", _ring(600, 30), 4, 17, "stream_kernel<2>"),
+    ("uneven blocks", _ring(1023, 3), 2, 70, "reg_kernel<4>"),
+    ("clamped block between", _bipartite_clamped(300, 3), 6, 25, "stream_kernel<3>"),
 ]
 
 
-@pytest.mark.parametrize("name,graph,chains,sweeps", CASES, ids=[c[0].replace(" ", "-") for c in CASES])
-def test_whole_run_matches_oracle(device, name, graph, chains, sweeps):
-    log_case(f"resident run: {name}")
+def case_program(device, graph):
     n, edges, free, clamped = graph
     rng = np.random.default_rng(5)
     ebm = th.IsingEBM(n, edges, rng.normal(0, 0.4, n), rng.normal(0.1, 0.5, len(edges)), 0.9)
-    prog = th.IsingSamplingProgram(ebm, free, clamped, device)
+    return ebm, th.IsingSamplingProgram(ebm, free, clamped, device)
+
+
+def observed_schedule(prog):
+    """Segments long enough for whole runs, which a lattice's own moment counters
+    compete with."""
+    return (3, 3, 20) if prog.kind == "lattice" else (3, 3, 4)
+
+
+@pytest.mark.parametrize("name,graph,chains,sweeps", [c[:4] for c in CASES],
+                         ids=[c[0].replace(" ", "-") for c in CASES])
+def test_whole_run_matches_oracle(device, name, graph, chains, sweeps):
+    log_case(f"resident run: {name}")
+    n, edges, free, clamped = graph
+    ebm, prog = case_program(device, graph)
     o = orc.Ising(n, ebm.edges, ebm.biases, ebm.weights, ebm.beta, [b.nodes for b in free],
                   [b.nodes for b in clamped])
-    init = rng.integers(0, 2, (chains, prog.n_total)).astype(np.uint8)
+    init = np.random.default_rng(6).integers(0, 2, (chains, prog.n_total)).astype(np.uint8)
     st = prog.new_state(chains)
     st.set_global(init)
     th.run_blocks(th.RngKey(77), prog, st, (), sweeps)
@@ -92,9 +116,10 @@ def test_whole_run_matches_oracle(device, name, graph, chains, sweeps):
     # again from where it stands, observed: segments of a few sweeps
     pairs = ebm.edges if len(edges) else np.zeros((0, 2), np.uint32)
     nodes = np.arange(n)
-    ns, es = th.estimate_moments(th.RngKey(78), nodes, pairs, prog, th.SamplingSchedule(3, 3, 4), st,
+    sched = observed_schedule(prog)
+    ns, es = th.estimate_moments(th.RngKey(78), nodes, pairs, prog, th.SamplingSchedule(*sched), st,
                                  return_sums=True)
-    wn, we, want, _ = o.estimate_moments(78, (3, 3, 4), want, nodes, pairs)
+    wn, we, want, _ = o.estimate_moments(78, sched, want, nodes, pairs)
     assert np.array_equal(ns, wn) and np.array_equal(es, we)
     assert np.array_equal(st.get_global(), want)
 

@@ -135,17 +135,19 @@ def test_q_range_checks(device):
                                  [np.array([0, 1])], [], device)
 
 
-@pytest.mark.parametrize("q,n,C,m", [(17, 40, 3, 90), (21, 900, 50, 4000), (33, 5, 1, 6),
-                                     (40, 12000, 64, 24000), (48, 2500, 128, 6000), (95, 300, 60, 900), (129, 64, 2, 100),
-                                     (255, 30, 1, 40), (256, 400, 64, 500), (257, 50, 3, 60),
-                                     (272, 3, 1, 2)])
-def test_lanes_per_item_parity(device, q, n, C, m):
-    """Every number of lanes that can split a site's categories (1 to 64, by
-    items, categories and slots per site), on both program kinds: sites whose
-    first keystream word has every offset, one to three and up to twenty
-    blocks per site, several slots per role and none, infinite biases that
-    send an item to the sequential scan, and near ties."""
-    log_case(f"lanes per item: q={q} n={n} C={C} edges={m}")
+# q, nodes, chains, edges, sweeps, lanes per item of the categorical program's blocks
+# and of the factor program's (test_host_dispatch.py holds the launches to these)
+LANES = [(17, 40, 3, 90, 2, {4}, {4}), (21, 900, 50, 4000, 2, {4}, {4}), (33, 5, 1, 6, 2, {4}, {4}),
+         (24, 6000, 120, 15000, 1, {2}, {2}), (40, 12000, 64, 24000, 2, {1, 4}, {1, 4}),
+         (48, 2500, 128, 6000, 2, {4}, {4}), (95, 300, 60, 900, 2, {8}, {8}), (129, 64, 2, 100, 2, {16}, {16}),
+         (255, 30, 1, 40, 2, {16}, {16}), (256, 400, 64, 500, 2, {16}, {16}), (257, 50, 3, 60, 2, {64}, {64}),
+         (272, 3, 1, 2, 2, {64}, {64}), (300, 400, 30, 60, 1, {8, 64}, {8, 64}),
+         (257, 700, 60, 40, 1, {4, 16}, {8, 16}), (257, 1300, 100, 60, 1, {2, 8}, {4, 8}),
+         (257, 3000, 110, 60, 1, {2}, {2}), (257, 14000, 110, 60, 1, {1, 2}, {1, 2})]
+
+
+def lanes_programs(device, q, n, C, m):
+    """The same model as a categorical and as a factor program, states and oracle."""
     edges, W, bias, blocks = _random_potts(n, m, q, 2, seed=q + n)
     bias[0, q - 1] = np.inf
     bias[1] = -np.inf
@@ -153,17 +155,27 @@ def test_lanes_per_item_parity(device, q, n, C, m):
     W[: max(1, m // 50)] = 0.0
     rng = np.random.default_rng(n)
     init = rng.integers(0, q, (C, n)).astype(np.uint16 if q > 256 else np.uint8)
-    o = orc.Potts(n, q, edges, W, bias, blocks)
-    want, _ = o.run_blocks(31, init, 2)
     prog = th.CategoricalProgram(n, q, edges, W, bias, blocks, device)
-    st = prog.new_state(C)
-    st.set_global(init)
-    th.run_blocks(th.RngKey(31), prog, st, (), 2)
-    assert np.array_equal(st.get_global(), want)
     fs = [th.CategoricalEBMFactor([np.arange(n)], bias.reshape(n, q, 1)),
           th.CategoricalEBMFactor([edges[:, 0], edges[:, 1]], W)]
     fp = th.FactorSamplingProgram(np.ones(n, np.uint8), q, fs, blocks, [], device)
-    sf = fp.new_state(C)
-    sf.set_global(init)
-    th.run_blocks(th.RngKey(31), fp, sf, (), 2)
-    assert np.array_equal(sf.get_global(), want)
+    return prog, fp, init, lambda: orc.Potts(n, q, edges, W, bias, blocks)
+
+
+@pytest.mark.parametrize("q,n,C,m,sweeps", [c[:5] for c in LANES])
+def test_lanes_per_item_parity(device, q, n, C, m, sweeps):
+    """Every number of lanes that can split a site's categories (by items,
+    categories and slots per site: 1 to 16 with one byte of state, 1 to 64 with
+    two), on both program kinds: sites whose
+    first keystream word has every offset, one to three and up to twenty
+    blocks per site, several slots per role and none, infinite biases that
+    send an item to the sequential scan, and near ties."""
+    log_case(f"lanes per item: q={q} n={n} C={C} edges={m}")
+    prog, fp, init, oracle = lanes_programs(device, q, n, C, m)
+    want, _ = oracle().run_blocks(31, init, sweeps)
+    for p in (prog, fp):
+        st = p.new_state(C)
+        st.set_global(init)
+        th.run_blocks(th.RngKey(31), p, st, (), sweeps)
+        assert np.array_equal(st.get_global(), want)
+        st.close()

@@ -4,7 +4,13 @@ import numpy as np
 import pytest
 
 import hostrun
+import test_gpu_dense as dense
+import test_gpu_discrete as discrete
+import test_gpu_potts as potts
+import test_gpu_resident as resident
+import test_gpu_wide_q as wide_q
 import thrml_hip as th
+from thrml_hip import workloads as wl
 
 
 def _spin_factor_run(sites, chains):
@@ -123,3 +129,114 @@ def test_a_segment_costs_its_way_into_and_out_of_lds(f, args, resident):
     too, with the lanes of its largest block."""
     k = hostrun.call(f, *args)
     assert {x.startswith("resident") for x in k} == {resident}, k
+
+
+def _wide_kernels(prog, C, sweeps=1):
+    """The wide categorical kernels of a run, as (kernel and element, lanes)."""
+    st = prog.new_state(C)
+    hostrun.clear_launches()
+    th.run_blocks(th.RngKey(1), prog, st, (), sweeps)
+    return {tuple(k.rstrip(">").rsplit(",", 1)) for k in hostrun.launches() if "wide_kernel" in k}
+
+
+def _lanes_of(i):
+    q, n, C, m = wide_q.LANES[i][:4]
+    prog, fp, _, _ = wide_q.lanes_programs(th.Device(0), q, n, C, m)
+    return _wide_kernels(prog, C), _wide_kernels(fp, C)
+
+
+@pytest.mark.parametrize("i", range(len(wide_q.LANES)))
+def test_lanes_of_the_parity_cases(i):
+    q, want = wide_q.LANES[i][0], wide_q.LANES[i][5:]
+    t = "unsigned_char" if q <= 256 else "unsigned_short"
+    for kernel, got, lanes in zip(("potts", "discrete"), hostrun.call(_lanes_of, i), want):
+        assert got == {(f"{kernel}_wide_kernel<{t}", str(p)) for p in lanes}
+
+
+def test_parity_cases_reach_every_lane_count():
+    for wide, every in ((False, {1, 2, 4, 8, 16}), (True, {1, 2, 4, 8, 16, 64})):
+        for kind in (5, 6):
+            assert set().union(*(c[kind] for c in wide_q.LANES if (c[0] > 256) == wide)) == every
+
+
+def _bias_only_lanes(q):
+    prog, _ = potts.bias_only_program(th.Device(0), q)
+    return {C: {int(lanes) for _, lanes in _wide_kernels(prog, C)} for C in potts.BIAS_ONLY_LANES[q]}
+
+
+@pytest.mark.parametrize("q", potts.BIAS_ONLY_LANES)
+def test_lanes_either_side_of_a_change(q):
+    assert hostrun.call(_bias_only_lanes, q) == {C: {p} for C, p in potts.BIAS_ONLY_LANES[q].items()}
+
+
+def _factor_lanes():
+    kinds, q, factors, free = discrete.wide_factor_model()
+    fs = [th.DiscreteEBMFactor(s, c, w) for s, c, w in factors]
+    prog = th.FactorSamplingProgram(kinds, q, fs, free, [], th.Device(0))
+    return {C: {int(lanes) for _, lanes in _wide_kernels(prog, C)} for C in discrete.FACTOR_LANES}
+
+
+def test_factor_lanes_either_side_of_a_change():
+    assert hostrun.call(_factor_lanes) == {C: {p} for C, p in discrete.FACTOR_LANES.items()}
+
+
+def _resident_case(i):
+    """The sweep kernels of a whole-run parity case: its run, its observed run."""
+    _, graph, C, sweeps, _ = resident.CASES[i]
+    ebm, prog = resident.case_program(th.Device(0), graph)
+    st = prog.new_state(C)
+    sched = resident.observed_schedule(prog)
+    seen = []
+    for run in (lambda: th.run_blocks(th.RngKey(1), prog, st, (), sweeps),
+                lambda: th.estimate_moments(th.RngKey(1), [0], ebm.edges, prog, th.SamplingSchedule(*sched), st)):
+        hostrun.clear_launches()
+        run()
+        seen.append({k: n for k, n in hostrun.launches().items() if "half" in k or "_kernel<" in k and "resident" in k})
+    return seen, sched[1]
+
+
+@pytest.mark.parametrize("i", range(len(resident.CASES)), ids=[c[0].replace(" ", "-") for c in resident.CASES])
+def test_kernels_of_the_whole_run_cases(i):
+    """One launch for the run, one per observation for the observed one."""
+    kernel = "resident_" + resident.CASES[i][4]
+    seen, n_obs = hostrun.call(_resident_case, i)
+    assert seen == [{kernel: 1}, {kernel: n_obs}]
+
+
+def test_whole_run_cases_reach_every_kernel():
+    assert {c[4] for c in resident.CASES} == {f"reg_kernel<{e}>" for e in (2, 4, 10)} | {
+        f"stream_kernel<{p}>" for p in range(2, 9)}
+
+
+def _dense_kernels(V, H, C):
+    prog = th.RbmProgram(np.zeros((V, H)), np.zeros(V), np.zeros(H), 1.0, th.Device(0))
+    st = prog.new_state(C)
+    seen = []
+    for blk in (0, 1):
+        hostrun.clear_launches()
+        prog.half_sweep(st, blk, np.zeros((C, 8), np.uint32))
+        seen += [k for k in hostrun.launches() if k.startswith("dense")]
+    return seen
+
+
+@pytest.mark.parametrize("V,H,C", dense.SMALL_TILES)
+def test_dense_tiles_of_the_parity_cases(V, H, C):
+    assert hostrun.call(_dense_kernels, V, H, C) == ["dense_small_kernel"] * 2
+    assert hostrun.call(_dense_kernels, V, H, dense.LARGE_TILES_C) == ["dense_half_kernel<false>"] * 2
+
+
+def _moment_kernels(C):
+    """Of two observations of a graph too large for whole runs, the first before any
+    sweep."""
+    ebm, blocks = wl.er_ising(70_001, 3.0, 0.2, 0.0, 0.3)
+    prog = th.IsingSamplingProgram(ebm, blocks, [], th.Device(0))
+    st = prog.new_state(C)
+    hostrun.clear_launches()
+    th.estimate_moments(th.RngKey(1), [0], ebm.edges, prog, th.SamplingSchedule(0, 2, 1), st)
+    return {k: n for k, n in hostrun.launches().items() if k.startswith("moments")}
+
+
+@pytest.mark.parametrize("C,kernels", [(32, {"moments_kernel<unsigned_int>": 1, "moments_kernel<unsigned_long>": 1}),
+                                       (33, {"moments_kernel<unsigned_long>": 2})])
+def test_moment_sums_read_the_low_halves(C, kernels):
+    assert hostrun.call(_moment_kernels, C) == kernels

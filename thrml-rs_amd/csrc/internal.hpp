@@ -584,11 +584,18 @@ constexpr uint32_t POTTS_WIDE_MAX_Q = 65536;  // Potts programs: two bytes above
 // of 0.8 and 1 instead of 1.1.  The first part is one wave's chain of dependent
 // loads, the second the whole chip's issue, to which idle lanes count as much
 // as busy ones.
-//   us per launch                        P = 1     2     4     8    16
-//   E-R 10007 deg 8, q = 21, 62K items      37    21    19    29    51
-//   E-R 1000 deg 8, q = 100, 7K items      111    49    23    15    15
-//   128^2, q = 32, 1M items                 79    70   121   234   459
-//   16^2, q = 256, 1K items                 62    33    16   9.5   6.0
+// The rule is taken for each block; a graph's colour blocks differ in size, so
+// that it can beat any one P.  us per launch, averaged over the program's blocks,
+// with the same P for all of them and by the rule:
+//                                          P = 1     2     4     8    16   rule
+//   E-R 10007 deg 8, q = 21, 50 chains        37    22    20    30    51     20
+//   E-R 10007 deg 8, q = 21, 25 chains        38    21    15    19    30     16
+//   E-R 10007 deg 8, q = 21, 100 chains       40    28    30    51    92     26
+//   E-R 20000 deg 6, q = 24, 30 chains        35    19    23    35    62     18
+//   E-R 10007 deg 8, q = 48, 50 chains        66    39    28    38    60     28
+//   E-R 1000 deg 8, q = 100, 8 chains        108    46    20    11    11     11
+//   128^2, q = 32, 128 chains                 77    67   121   233   456     67
+//   16^2, q = 256, 8 chains                   63    33    17    10   6.7    6.8
 inline uint32_t wide_lanes(uint32_t q, uint64_t items, uint32_t slots) {
   uint32_t step = 16u;  // the offsets a site's first word can have: multiples of gcd(q, 16)
   while (q % step) step /= 2u;

@@ -10,9 +10,10 @@
 // those of the per-block kernels (same sums in the same order, same words,
 // spin_decision), so the states are identical.
 //
-// Bound: instruction issue of one CU (16 waves, one chain): about 60 vector
-// instructions per 64 sites with the records in registers, 24 of them the
-// keystream.  Measured, per sweep: 64^2 torus, 256 chains 5.1 -> 1.7 us (7.35
+// Bound: instruction issue of one CU (16 waves, one chain): 42 vector
+// instructions per 64 sites with the records in registers (683 million for the
+// 2000 half-sweeps of 8192 slices of a 64^2 torus with 256 chains), 23 of them
+// the keystream.  Measured, per sweep: 64^2 torus, 256 chains 5.1 -> 1.7 us (7.35
 // -> 1.80 ms for 1000 sweeps and the read-back); Erdos-Renyi graph of 20011
 // nodes, mean degree 7, 200 chains 48 -> 23 us; two 40^2 layers with 13
 // neighbours each, one chain 8.0 -> 4.2 us.
@@ -48,7 +49,7 @@ struct ResArgs {
   const ResPiece *pieces;
   const ResPart *parts;
   const uint4 *ents;        // the waves' entries {byte offset of the data, meta, next entry, 0}
-  const uint4 *woff;        // [n_parts][waves] {first entry, entries, leading barriers, 0}
+  const uint4 *woff;        // [n_parts][waves] {first entry, entries, leading barriers, ring's first entry}
   const uint8_t *data;      // site records and slot pairs {position, weight, position, weight}
   uint32_t n_total, n_words, n_sweeps, n_blocks, C_pad;
   uint32_t n_parts, per_phase;  // sweeps per phase (1 with several parts)

@@ -55,6 +55,24 @@ def test_spin_state_round_trip(device, n, C):
     prog.close()
 
 
+@pytest.mark.parametrize("C", [1, 63, 65, 4100])
+def test_narrow_spin_blocks(device, C):
+    """Blocks around the widths that the export by rows of chains takes."""
+    sizes = [1, 2, 8, 9, 16, 17]
+    n = sum(sizes)
+    cuts = np.cumsum(sizes)[:-1]
+    log_case(f"narrow spin blocks C={C}")
+    prog = th.IsingSamplingProgram(th.IsingEBM(n, np.zeros((0, 2)), np.zeros(n), []), np.split(np.arange(n), cuts), [],
+                                   device)
+    x = np.random.default_rng(C).integers(0, 2, (C, n)).astype(np.uint8)
+    st = prog.new_state(C)
+    st.set_global(x)
+    for b, want in enumerate(np.split(x, cuts, axis=1)):
+        assert np.array_equal(st.get_block(b), want)
+        assert np.array_equal(st.get_block(b, np.float32), want.astype(np.float32))
+    st.close()
+
+
 @pytest.mark.parametrize("q,n,C", [(2, 7, 1), (3, 64, 64), (129, 65, 66), (256, 130, 3), (300, 67, 65)])
 def test_categorical_state_round_trip(device, q, n, C):
     log_case(f"categorical state io q={q} n={n} C={C}")

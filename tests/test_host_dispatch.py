@@ -240,3 +240,19 @@ def _moment_kernels(C):
                                        (33, {"moments_kernel<unsigned_long>": 2})])
 def test_moment_sums_read_the_low_halves(C, kernels):
     assert hostrun.call(_moment_kernels, C) == kernels
+
+
+def _export_kernels(n):
+    prog = th.IsingSamplingProgram(th.IsingEBM(n, np.zeros((0, 2)), np.zeros(n), []), [np.arange(n)], [], th.Device(0))
+    st = prog.new_state(100)
+    seen = []
+    for dt in (np.uint8, np.float32):
+        hostrun.clear_launches()
+        st.get_block(0, dt)
+        seen += hostrun.launches()
+    return seen
+
+
+@pytest.mark.parametrize("n,u8,f32", [(8, "_narrow", "_narrow"), (9, "_narrow", ""), (16, "_narrow", ""), (17, "", "")])
+def test_export_of_few_positions(n, u8, f32):
+    assert hostrun.call(_export_kernels, n) == [f"unpack{u8}_kernel<unsigned_char>", f"unpack{f32}_kernel<float>"]

@@ -150,6 +150,24 @@ __global__ __launch_bounds__(256) void unpack_kernel(V *__restrict__ dst, StateI
   }
 }
 
+// Export of few positions: a wave takes a chain group, lane = chain, so that all
+// lanes have a row (above, two positions leave one lane of 64).  Bound by its
+// stores, a row apart per lane, so that it loses from some width on.  us per
+// launch, above -> here:
+//   u8   2 positions, 1,024 chains 5.6 -> 3.6;  3, 600,000 38 -> 3.8
+//        16, 600,000 22 -> 14;  24, 600,000 22 -> 27
+//   f32  2, 600,000 15 -> 3.8;  8, 600,000 17 -> 14;  12, 600,000 16 -> 28
+constexpr uint32_t IO_NARROW_U8 = 16, IO_NARROW_F32 = 8;
+template <class V>
+__global__ __launch_bounds__(256) void unpack_narrow_kernel(V *__restrict__ dst, StateIo a, uint32_t G) {
+  const uint32_t g = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t c = g * 64u + (threadIdx.x & 63u);
+  if (g >= G || c >= a.C) return;
+  const uint64_t *w = a.words + (size_t)g * a.plane_stride;
+  V *row = dst + (size_t)c * a.stride + a.col0;
+  for (uint32_t i = 0; i < a.n; ++i) row[i] = (V)((w[i] >> (c & 63u)) & 1ull);
+}
+
 // Import check before any write: *bad becomes the smallest column that holds
 // something else than a state value (0..q-1 as u8, or the floats 0.0..q-1.0),
 // among columns col0 .. col0 + n - 1 of the rows of `stride` values.
@@ -238,12 +256,16 @@ int launch_unpack(thrml_state *st, uint64_t p0, uint32_t n, void *d_dst, int dty
   const StateIo a = state_io_args(st, p0, n, stride, col0, dtype);
   const uint64_t tasks = (uint64_t)a.n_chunks * cdiv(st->C, IO_CHAINS);
   if (tasks > 0x7fffffffull) return fail(THRML_EUNSUPPORTED, "block too large to export");
-  if (dtype == THRML_DTYPE_U8)
-    hipLaunchKernelGGL(unpack_kernel<uint8_t>, dim3(cdiv(tasks, 4)), dim3(256), 0, s,
-                       static_cast<uint8_t *>(d_dst), a, (uint32_t)tasks);
-  else
-    hipLaunchKernelGGL(unpack_kernel<float>, dim3(cdiv(tasks, 4)), dim3(256), 0, s,
-                       static_cast<float *>(d_dst), a, (uint32_t)tasks);
+  const dim3 grid(cdiv(tasks, 4)), narrow(cdiv(st->G, 4)), wg(256);
+  if (dtype == THRML_DTYPE_U8) {
+    uint8_t *dst = static_cast<uint8_t *>(d_dst);
+    if (n <= IO_NARROW_U8) hipLaunchKernelGGL(unpack_narrow_kernel<uint8_t>, narrow, wg, 0, s, dst, a, st->G);
+    else hipLaunchKernelGGL(unpack_kernel<uint8_t>, grid, wg, 0, s, dst, a, (uint32_t)tasks);
+  } else {
+    float *dst = static_cast<float *>(d_dst);
+    if (n <= IO_NARROW_F32) hipLaunchKernelGGL(unpack_narrow_kernel<float>, narrow, wg, 0, s, dst, a, st->G);
+    else hipLaunchKernelGGL(unpack_kernel<float>, grid, wg, 0, s, dst, a, (uint32_t)tasks);
+  }
   THRML_HIP(hipGetLastError());
   return THRML_OK;
 }

@@ -147,3 +147,50 @@ def test_noalloc_two_contexts_share_the_key_array(device):
             b.close()
     finally:
         dev_b.close()
+
+
+@pytest.mark.parametrize("model,C,sweeps", [("lattice", 65, 30), ("irregular", 3, 30), ("irregular", 1, 30),
+                                            ("categorical", 9, 4), ("dense", 70, 4)])
+def test_noalloc_in_a_captured_graph(model, C, sweeps):
+    """Captured on the context's stream and replayed, with other work of the
+    context in between: every replay does what the same call does eagerly."""
+    import torch
+
+    rng = np.random.default_rng(23)
+    dev = th.Device(0)
+    side = torch.cuda.Stream()
+    dev.set_stream(side.cuda_stream)
+    q = 2
+    if model == "lattice":
+        ebm, blocks = wl.lattice_ising(32, 0.1, 0.4, 0.05)
+        prog = th.IsingSamplingProgram(ebm, blocks, [], dev)
+    elif model == "irregular":
+        ebm, blocks = wl.er_ising(900, 5.0, 0.2, 0.0, 0.3)
+        prog = th.IsingSamplingProgram(ebm, blocks, [], dev)
+    elif model == "categorical":
+        q = 20
+        n, edges, W, bias, blocks = wl.potts_lattice(8, q, 0.5, 0.3, cfg=9)
+        prog = th.CategoricalProgram(n, q, edges, W, bias, blocks, dev)
+    else:
+        prog = th.RbmProgram(rng.normal(0, 0.1, (90, 60)), np.zeros(90), np.zeros(60), 1.0, dev)
+    log_case(f"noalloc captured: {model} C={C}")
+    init = rng.integers(0, q, (C, prog.n_total)).astype(np.uint8)
+    st, eager = prog.new_state(C), prog.new_state(C)
+    st.set_global(init)
+    eager.set_global(init)
+    _noalloc(prog, th.RngKey(41), eager, sweeps)  # (and the kernels are loaded)
+    want = [eager.get_global()]
+    for _ in range(3):
+        _noalloc(prog, th.RngKey(41), eager, sweeps)
+        want.append(eager.get_global())
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        _noalloc(prog, th.RngKey(41), st, sweeps)
+    assert np.array_equal(st.get_global(), init)  # captured, not run
+    for k in range(4):
+        with torch.cuda.stream(side):
+            g.replay()
+        assert np.array_equal(st.get_global(), want[k]), f"replay {k}"
+        _noalloc(prog, th.RngKey(5), eager, 3)
+    dev.close()
